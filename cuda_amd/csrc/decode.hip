@@ -10,34 +10,33 @@
 // dispatch_async_flash_decode (kernels_api.h:58-62). The reference walks each
 // (sequence, head) serially in one block; here contexts are split.
 //
-// Work decomposition (split-K, one wave per split)
-//   a wave owns (sequence n, kv head, query-head chunk of <= 16, split) and
-//   walks kPagesPerWave pages of 16 tokens, two pages per step, with the next
-//   step's K and V already in flight in a second register set (the step loop
-//   is unrolled by two so the sets swap roles without copies). Waves never
-//   synchronise; a workgroup is just four independent waves.
-//   The GQA group of query heads (Hq / Hkv <= 16 per chunk) shares every K/V
-//   byte loaded, so each cache byte is read from HBM once per kv head.
+// Work decomposition (split-K over pages of 16 tokens)
+//   a wave walks pages of one (sequence, kv head, query-head chunk of <= 16),
+//   two per step, with its K and V travelling HBM -> LDS in a wave-private
+//   ring; the GQA group of query heads (Hq / Hkv <= 16 per chunk) shares every
+//   K/V byte loaded, so each cache byte is read from HBM once per kv head.
+//   Larger paged launches balance the pages over one wave per SIMD
+//   (decode_sk_kernel); smaller ones and the contiguous cache split each
+//   sequence over workgroups of 1, 4 or 8 waves (decode_mw_kernel).
 // Per wave and step (16x16x32 MFMAs, query heads padded to 16):
 //   S^T[16 tok x 16 heads] = K^T Q^T per page; a page is [D][16] with tokens
 //   contiguous, so the K^T operand (8 consecutive d for one token) is read
-//   from a wave-private LDS copy with ds_read_b64_tr_b16 / _tr_b8;
+//   with ds_read_b64_tr_b16 / _tr_b8 (the contiguous cache's rows as they are);
 //   online softmax over tokens, rescaled only when the max grows by > 2^8;
-//   O[16 heads x D] += P V^T over the step's 32 tokens; the V^T operand
-//   (tokens contiguous for one d) is loaded from HBM in operand layout.
+//   O[16 heads x D] += P V^T over the step's 32 tokens; the V operand
+//   (tokens contiguous for one d) is the page layout (contiguous cache: a
+//   transpose read);
 //   FP8: codes are converted exactly to the MFMA element type; the k scale of
 //   a page multiplies that page's logits and the v scale is folded into P.
 // A sequence that fits one split writes its output directly; otherwise each
-// wave writes (o / l, log2-sum-exp) to the workspace and decode_merge_kernel
-// combines the splits. (This describes the contiguous-cache kernel; the
-// paged kernels below stream pages HBM -> LDS, and larger paged launches
-// balance the pages over one wave per SIMD instead of splitting per
-// sequence: decode_sk_kernel.)
+// split writes (o / l, log2-sum-exp) to the workspace and a merge kernel
+// combines them.
 #include <algorithm>
 #include <atomic>
 #include <climits>
 #include <functional>
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "launch.h"
@@ -45,7 +44,7 @@
 
 namespace ca {
 
-enum : int { kKindPaged16 = 0, kKindPagedFp8 = 1 };
+enum : int { kKindPaged16 = 0, kKindPagedFp8 = 1, kKindContig16 = 2 };
 
 template <typename Tr>
 struct Fp8Conv;
@@ -71,169 +70,299 @@ __device__ __forceinline__ typename Tr::vec8 fp8x8_to(uint32_t lo, uint32_t hi) 
   return __builtin_bit_cast(typename Tr::vec8, r);
 }
 
-// Streaming loads: every cache byte is used once per launch, so they bypass
-// the cache hierarchy's retention (non-temporal).
-template <typename T>
-__device__ __forceinline__ T ld_stream(const void* p) {
-  return __builtin_nontemporal_load((const T*)p);
+// ---------------------------------------------------------------------------
+// HBM -> LDS direct loads.
+//
+// Pages travel from HBM straight into a per-wave LDS ring with
+// global_load_lds_dwordx4 (each lane's 16 bytes land at ring slot + 16 *
+// lane), so bytes in flight cost no VGPRs: a wave keeps its ring's steps (two
+// pages each, K and V) in flight.
+// LDS is read with hand-issued ds_read instructions and the vector-memory
+// counter is waited on explicitly (s_waitcnt vmcnt(N) with N = the loads
+// issued after the step being consumed); the compiler's own conservative
+// wait-for-everything before LDS reads would serialise the ring.
+// Layouts in a ring slot: K pages as loaded ([D][16]; the 16-bit page's
+// 16-byte chunks are XOR-swizzled on bit 3 of the chunk index by row-octet
+// parity so the tr16 reads of lane groups 0/1 and 2/3 hit disjoint banks),
+// V pages [D][16] with the 16-bit page's chunks swizzled too (chunk q at
+// q ^ bit 4 of q): a 32-lane half of a V read takes the first or second 16
+// bytes of 16 rows, 32 bytes apart, which without the swizzle put rows r
+// and r + 8 on the same banks (a b64 read is conflict-free when each half
+// covers 256 distinct bytes modulo 256). FP8 V rows are 16 bytes, and a
+// b32 read of a lane's 4 tokens is 2-way conflicting (its halves need 32
+// distinct dwords modulo 128 bytes from 16 rows, two dwords each), so the
+// FP8 lanes read 8 bytes (tokens 8 (grp / 2) .. + 7: lane groups 0/1 and
+// 2/3 read the same addresses, 16 rows x 8 bytes per half) and keep the
+// dword of their own group. The contiguous cache's rows (a token's 2 D
+// bytes) hold chunk c at c ^ contig_swz(row): 16 rows' chunk c (the K read)
+// and 8 rows' chunks 2 nb, 2 nb + 1 (a half of the V transpose read) fall on
+// distinct positions of the 256 bytes of banks.
+// ---------------------------------------------------------------------------
+// Pages per split of the split grid: 128 FP8 pages, 64 16-bit ones (256 KB of
+// K and V at head dim 128 either way). Page loads use the "nt" cache policy:
+// every cache byte is read once per launch, so it is streamed rather than
+// retained.
+template <int KIND>
+struct DmaCfg {
+  // ring steps of the stream-K walk: 16 KB of K and V at head dim 128 for both
+  // cache kinds. Rings twice as deep: 16-bit 0 to -3 %, FP8 -2 to 0 %; three
+  // and four times 16-bit -1 to -5 %.
+  static constexpr int kRing = KIND == kKindPagedFp8 ? 2 : 1;
+  static constexpr int kPages = KIND == kKindPagedFp8 ? 128 : kPagesPerWave;
+  // pages per ring fill of the stream-K walk
+  static constexpr int kSkPages = 128;
+  // decode_workspace_bytes sizes the partials for kPagesPerWave-page splits
+  static_assert(kPages >= kPagesPerWave, "pages per split");
+};
+constexpr int kDmaPolicy = 2;  // global_load_lds cache policy bits: nt
+constexpr int kStepPages = 2;  // pages per step of a wave
+
+// f(integral constant 0 .. N - 1): loops whose index is an instruction's immediate
+template <int N, typename F, int I = 0>
+__device__ __forceinline__ void for_const(F& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    for_const<N, F, I + 1>(f);
+  }
 }
 
-// Contiguous-cache decode (flash_decode): one wave per split of kPagesPerWave
-// "pages" of 16 consecutive tokens of one (sequence, kv head, <= 16 q heads).
-// K^T operands come straight from the row-major cache (a lane's 16 bytes are
-// 8 consecutive head-dim elements of one token); V rows go through a
-// wave-private LDS copy [32][D + 16] and are read back transposed. Register
-// double-buffering: the next two pages load while the current two compute.
-template <int D>
-struct ContigGeom {
-  static constexpr int NKS = D / 32;  // S^T k-steps (32 d each)
-  static constexpr int NB = D / 16;   // PV output blocks (16 d each)
-  // V: 16 rows x D of one page as 16-byte chunks per lane
-  static constexpr int VROWREG = (16 * D * 2) / (64 * 16);
-  static constexpr int kLdsBytesPerWave = 32 * (D + 16) * 2;
-};
-
-// Registers of one step (two pages): K and V as loaded from HBM.
-template <int D>
-struct ContigRegs {
-  using G = ContigGeom<D>;
-  u32x4 k[2][G::NKS];
-  u32x4 vrow[2][G::VROWREG];
-};
-
+// The wave's GQA group of query rows (Gc <= 16 heads from `qrow`, D each) as
+// the B operand of S^T = K^T Q^T: lane (head l16, group grp) holds d = 32 ks
+// + 8 grp .. + 7; rows past Gc are zero.
 template <typename Tr, int D>
-__global__ __launch_bounds__(kDecodeWgWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void decode_split_kernel(
-    const uint16_t* __restrict__ Q, const uint16_t* __restrict__ Kc, const uint16_t* __restrict__ Vc,
-    uint16_t* __restrict__ O, float* __restrict__ ws_o, float* __restrict__ ws_lse, int Hq,
-    int Hkv, int S_contig, int max_splits, int n_hc, long long total_waves, float scale_log2) {
+__device__ __forceinline__ void dma_load_q(const uint16_t* __restrict__ qrow, int Gc,
+                                           typename Tr::vec8 (&qv)[D / 32]) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, grp = lane >> 4;
+#pragma unroll
+  for (int ks = 0; ks < D / 32; ++ks) {
+    if (l16 < Gc) {
+      qv[ks] = *(const typename Tr::vec8*)(qrow + (size_t)l16 * D + 32 * ks + 8 * grp);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qv[ks][e] = 0;
+    }
+  }
+}
+
+// One wave's walk over pages [p_begin, p_end) (at most PAGES)
+// of one (sequence, kv head hk) whose block-table row is `bt_row` (kContig16:
+// of a contiguous head whose rows start at Kc / Vc). The online-softmax state
+// (o, m_run, l_run) is carried in and out, so a context can be walked in
+// several calls; the ring is filled at the start and drained at the end of
+// each call. A step takes two pages: its instructions form one dependent
+// chain (LDS reads, K^T Q, max, exponentials, P V), about 0.5 us whether it
+// carries 16 tokens or 32, which is what a wave alone on its SIMD waits for.
+template <typename Tr, int D, int KIND, int RING, int PAGES>
+__device__ __forceinline__ void dma_walk(const typename Tr::vec8 (&qv)[D / 32], f32x4 (&o)[D / 16],
+                                         float& m_run, float& l_run, unsigned char* ring,
+                                         const void* __restrict__ Kc, const void* __restrict__ Vc,
+                                         const float* __restrict__ k_scale,
+                                         const float* __restrict__ v_scale, int per_block,
+                                         const int32_t* __restrict__ bt_row, int Hkv, int hk,
+                                         int num_blocks, int p_begin, int p_end, int Lctx,
+                                         float scale_log2, const unsigned char* dummy) {
   using vec8 = typename Tr::vec8;
-  using vec4 = typename Tr::vec4;
-  using vec2 = typename Tr::vec2;
-  using G = ContigGeom<D>;
-  constexpr int NKS = G::NKS, NB = G::NB;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kDecodeWgWaves * G::kLdsBytesPerWave];
+  constexpr int NKS = D / 32, NB = D / 16;
+  constexpr bool FP8 = KIND == kKindPagedFp8, CONTIG = KIND == kKindContig16;
+  constexpr int ELEM = FP8 ? 1 : 2;
+  constexpr int CHUNK = D * 16 * ELEM;        // bytes of one (page, head) chunk
+  constexpr int NDMA = CHUNK / 1024;          // 16 B x 64 lanes per load
+  constexpr int STAGE = kStepPages * 2 * CHUNK;   // K and V of the step's pages
+  constexpr int DPS = kStepPages * 2 * NDMA;      // loads per step
+  constexpr int PB = PAGES / 64;              // page-id registers per lane
+  static_assert(kStepPages == 2, "a step is two pages");
+  static_assert(PAGES % 64 == 0 && PB <= 2, "pages per walk");
+  static_assert((RING - 1) * DPS <= 63, "vmcnt range");
 
-  // the wave index is uniform: readfirstlane keeps every per-wave quantity
-  // derived from it (work item, page range, masks) in scalar registers
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const long long wid = (long long)blockIdx.x * kDecodeWgWaves + wave;
-  if (wid >= total_waves) return;
-
-  // ---- work item ----
-  long long w = wid;
-  const int split = (int)(w % max_splits);
-  w /= max_splits;
-  const int hc = (int)(w % n_hc);
-  w /= n_hc;
-  const int hk = (int)(w % Hkv);
-  const int n = (int)(w / Hkv);
-  const int Gq = Hq / Hkv;
-  const int hq0 = hk * Gq + hc * 16;
-  const int Gc = min(16, Gq - hc * 16);
-
-  const int Lctx = S_contig;
-  const int n_pages = (Lctx + kDecodePage - 1) / kDecodePage;
-  const int n_splits = max(1, (n_pages + kPagesPerWave - 1) / kPagesPerWave);
-  if (split >= n_splits) return;
-
+  const int lane = threadIdx.x & 63;
   const int l16 = lane & 15, grp = lane >> 4;
-  const int p_begin = split * kPagesPerWave;
-  const int p_end = min(p_begin + kPagesPerWave, n_pages);
-  const int n_steps = (p_end - p_begin + 1) / 2;  // 0 only for an empty context
+  const int n_pg = p_end - p_begin, n_steps = (n_pg + 1) / 2;
 
-  // ---- Q^T operand: lane (head g = l16, k-group grp) ----
-  vec8 qv[NKS];
-  {
-    const uint16_t* qrow = Q + ((size_t)n * Hq + hq0 + l16) * D;
+  // page ids and per-page scales: lane j of register b holds page
+  // p_begin + 64 b + j; read back for page index i (uniform) with lane_val
+  int pid_lane[PB];
+  float ksc_lane[PB], vsc_lane[PB];
+  if constexpr (!CONTIG) {
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      if (l16 < Gc) {
-        qv[ks] = *(const vec8*)(qrow + 32 * ks + 8 * grp);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) qv[ks][e] = 0;
+    for (int pb = 0; pb < PB; ++pb) {
+      const int page = p_begin + 64 * pb + lane;
+      pid_lane[pb] = 0;
+      ksc_lane[pb] = vsc_lane[pb] = 1.f;
+      if (page < p_end) {
+        pid_lane[pb] = bt_row[page];
+        pid_lane[pb] = min(max(pid_lane[pb], 0), num_blocks - 1);
+      }
+      if (FP8) {
+        if (per_block) {
+          if (page < p_end) {
+            ksc_lane[pb] = k_scale[(size_t)pid_lane[pb] * Hkv + hk];
+            vsc_lane[pb] = v_scale[(size_t)pid_lane[pb] * Hkv + hk];
+          }
+        } else {
+          ksc_lane[pb] = k_scale[hk];
+          vsc_lane[pb] = v_scale[hk];
+        }
       }
     }
   }
-  unsigned char* wlds = lds + wave * G::kLdsBytesPerWave;
-  const size_t base = ((size_t)n * Hkv + hk) * (size_t)S_contig * D;
-  const uint16_t* Kp = Kc + base;
-  const uint16_t* Vp = Vc + base;
+  auto lane_val = [&](const auto (&r)[PB], int i) CA_INLINE {
+    const auto v = (PB > 1 && i >= 64) ? r[PB - 1] : r[0];
+    return __builtin_bit_cast(std::remove_const_t<std::remove_reference_t<decltype(r[0])>>,
+                              __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i & 63));
+  };
 
-  // ---- HBM -> registers for one step ----
-  auto load_step = [&](ContigRegs<D>& R, int step) {
+  // source byte offset of this lane's 16 bytes for load i of a K chunk
+  auto k_src = [&](int i) -> int {
+    const int p = 64 * i + lane;  // physical 16-byte slot in LDS
+    if (FP8) return 16 * p;
+    return 16 * (p ^ (((p >> 4) & 1) << 3));
+  };
+  // source offset of this lane's 16 bytes in each 1 KB of a V chunk
+  const int v_src = 16 * (FP8 ? lane : lane ^ ((lane >> 4) & 1));
+  // contiguous rows: LDS row r (a token, 2 D bytes) holds its 16-byte chunk c
+  // at c ^ contig_swz(r); load i covers rows kRpl i + lane / kCpr
+  constexpr int kCpr = D / 8, kRpl = 64 / kCpr;
+  auto contig_swz = [](int r) CA_INLINE {
+    return D == 128 ? ((r & 7) << 1) | ((r >> 3) & 1) : (((r >> 1) & 3) << 1) | ((r >> 3) & 1);
+  };
+  auto issue_step = [&](int step, int slot) {
 #pragma unroll
-    for (int pp = 0; pp < 2; ++pp) {
-      const int page = p_begin + 2 * step + pp;
-      const bool valid = page < p_end;
-      const int tok = page * 16 + l16;
+    for (int pp = 0; pp < kStepPages; ++pp) {
+      const int pg = kStepPages * step + pp;
+      unsigned char* base = ring + slot * STAGE + pp * 2 * CHUNK;
+      const bool valid = pg < n_pg;
+      if constexpr (CONTIG) {
+        // rows past the context (its last page) read the last token instead
+        const int tok0 = 16 * (p_begin + pg), last = Lctx - 1 - tok0;
+        const size_t chunk = (size_t)tok0 * (2 * D);
+        const unsigned char* kp = (const unsigned char*)Kc + chunk;
+        const unsigned char* vp = (const unsigned char*)Vc + chunk;
 #pragma unroll
-      for (int ks = 0; ks < NKS; ++ks)
-        R.k[pp][ks] = (valid && tok < S_contig)
-                          ? ld_stream<u32x4>(Kp + (size_t)tok * D + 32 * ks + 8 * grp)
-                          : u32x4{0, 0, 0, 0};
-      constexpr int CH = D / 8;
+        for (int i = 0; i < NDMA; ++i) {
+          const int r = kRpl * i + lane / kCpr;
+          const int off = min(r, last) * (2 * D) + 16 * ((lane % kCpr) ^ contig_swz(r));
+          dma16<kDmaPolicy>(valid ? kp + off : dummy, (CA_LDS void*)(base + 1024 * i));
+          dma16<kDmaPolicy>(valid ? vp + off : dummy, (CA_LDS void*)(base + CHUNK + 1024 * i));
+        }
+      } else {
+        const int pid = lane_val(pid_lane, valid ? pg : 0);
+        const size_t chunk = ((size_t)pid * Hkv + hk) * (size_t)CHUNK;
+        const unsigned char* kp = (const unsigned char*)Kc + chunk;
+        const unsigned char* vp = (const unsigned char*)Vc + chunk;
 #pragma unroll
-      for (int i = 0; i < G::VROWREG; ++i) {
-        const int c = lane + 64 * i;
-        const int vt = page * 16 + c / CH;
-        R.vrow[pp][i] = (valid && vt < S_contig)
-                            ? ld_stream<u32x4>(Vp + (size_t)vt * D + (c % CH) * 8)
-                            : u32x4{0, 0, 0, 0};
+        for (int i = 0; i < NDMA; ++i) {
+          dma16<kDmaPolicy>(valid ? kp + k_src(i) : dummy, (CA_LDS void*)(base + 1024 * i));
+          dma16<kDmaPolicy>(valid ? vp + 1024 * i + v_src : dummy,
+                            (CA_LDS void*)(base + CHUNK + 1024 * i));
+        }
       }
     }
   };
 
-  f32x4 o[NB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = kNegInf, l_run = 0.f;
+  // per-lane LDS read offsets inside a page's K / V chunk
+  uint32_t k_lo, k_hi;
+  if (FP8) {
+    k_lo = 16 * (8 * grp + (l16 >> 1)) + 8 * (l16 & 1);
+    k_hi = 0;
+  } else {
+    const int c = l16 & 3, j = l16 >> 2, par = grp & 1;
+    k_lo = 16 * (16 * grp + 8 * par + 2 * j + (c >> 1)) + 8 * (c & 1);
+    k_hi = 16 * (16 * grp + 8 * (1 - par) + 2 * j + (c >> 1)) + 8 * (c & 1);
+  }
+  // V: lane (d = l16, token group grp) needs tokens 4 grp .. 4 grp + 3 of row d
+  // (FP8: the 8 bytes of tokens 8 (grp / 2) .. + 7, then its own dword)
+  const uint32_t v_off = FP8 ? (uint32_t)(16 * l16 + 8 * (grp >> 1))
+                             : (uint32_t)(16 * ((2 * l16 + (grp >> 1)) ^ ((l16 >> 3) & 1)) + 8 * (grp & 1));
+  // contiguous: K row l16, chunk 4 ks + grp (XOR of a lane part and 4 ks); V by
+  // transpose reads, source lane (l16 / 4, l16 % 4) = row 4 grp + l16 / 4, 8
+  // bytes l16 % 4 of the 32 of d-block nb (chunks 2 nb, 2 nb + 1)
+  const uint32_t c_krow = l16 * (2 * D), c_k = 16 * (grp ^ contig_swz(l16));
+  const int c_vr = 4 * grp + (l16 >> 2);
+  const uint32_t c_vrow = c_vr * (2 * D) + 8 * (l16 & 1);
+  const uint32_t c_v = 16 * (((l16 & 3) >> 1) ^ contig_swz(c_vr));
+  const uint32_t ring0 = lds_off(ring);
 
-  // ---- one step of attention on registers R ----
-  auto compute_step = [&](const ContigRegs<D>& R, int step) {
-    // stage the V rows into the wave's LDS
-    {
-      uint16_t* vl = (uint16_t*)wlds;
-      constexpr int CH = D / 8;
+  // RING steps in flight from the start; a slot is refilled as soon as its
+  // LDS reads have returned, so RING steps stay in flight during the math
 #pragma unroll
-      for (int pp = 0; pp < 2; ++pp)
+  for (int st = 0; st < RING; ++st) issue_step(st, st);
+  int slot = 0;
+  for (int step = 0; step < n_steps; ++step) {
+    wait_vmcnt<(RING - 1) * DPS>();  // this step's loads are the oldest outstanding
+
+    // ---- LDS -> operands ----
+    u32x4 kop[kStepPages][NKS];   // K^T operand (FP8: two dwords of codes)
+    u32x2 vop[kStepPages][NB];    // V operand half (FP8: 8 codes, one dword kept)
 #pragma unroll
-        for (int i = 0; i < G::VROWREG; ++i) {
-          const int c = lane + 64 * i;
-          *(u32x4*)(vl + (16 * pp + c / CH) * (D + 16) + (c % CH) * 8) = R.vrow[pp][i];
+    for (int pp = 0; pp < kStepPages; ++pp) {
+      const uint32_t kb = ring0 + slot * STAGE + pp * 2 * CHUNK;
+      auto k_read = [&](auto i) CA_INLINE {
+        constexpr int ks = decltype(i)::value;
+        if constexpr (FP8) {
+          const u32x2 t = lds_read_tr8<512 * ks>(kb + k_lo);
+          kop[pp][ks][0] = t[0];
+          kop[pp][ks][1] = t[1];
+        } else if constexpr (CONTIG) {
+          kop[pp][ks] = lds_read_b128<0>(kb + c_krow + (c_k ^ (64 * ks)));
+        } else {
+          const u32x2 lo = lds_read_tr16<1024 * ks>(kb + k_lo), hi = lds_read_tr16<1024 * ks>(kb + k_hi);
+          kop[pp][ks] = u32x4{lo[0], lo[1], hi[0], hi[1]};
         }
+      };
+      auto v_read = [&](auto i) CA_INLINE {
+        constexpr int nb = decltype(i)::value;
+        if constexpr (FP8) vop[pp][nb] = lds_read_b64<256 * nb>(kb + CHUNK + v_off);
+        else if constexpr (CONTIG) vop[pp][nb] = lds_read_tr16<0>(kb + CHUNK + c_vrow + (c_v ^ (32 * nb)));
+        else vop[pp][nb] = lds_read_b64<512 * nb>(kb + CHUNK + v_off);
+      };
+      for_const<NKS>(k_read);
+      for_const<NB>(v_read);
     }
-    __builtin_amdgcn_wave_barrier();
+    wait_lgkm0();
+#pragma unroll
+    for (int pp = 0; pp < kStepPages; ++pp) {
+#pragma unroll
+      for (int i = 0; i < NKS; ++i) after_wait(kop[pp][i]);
+#pragma unroll
+      for (int i = 0; i < NB; ++i) after_wait(vop[pp][i]);
+    }
+    issue_step(step + RING, slot);  // the slot's data is in registers now
 
-    // S^T per page
-    f32x4 s[2];
+    // ---- S^T of the pages ----
+    f32x4 s[kStepPages];
 #pragma unroll
-    for (int pp = 0; pp < 2; ++pp) {
-      s[pp] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int pp = 0; pp < kStepPages; ++pp) s[pp] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < NKS; ++ks)
-        s[pp] = Tr::mfma16(__builtin_bit_cast(vec8, R.k[pp][ks]), qv[ks], s[pp]);
-    }
+    for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+      for (int pp = 0; pp < kStepPages; ++pp) {
+        const vec8 a = FP8 ? fp8x8_to<Tr>(kop[pp][ks][0], kop[pp][ks][1])
+                           : __builtin_bit_cast(vec8, kop[pp][ks]);
+        s[pp] = Tr::mfma16(a, qv[ks], s[pp]);
+      }
 
-    // online softmax over the step's 32 tokens
-    const int pageA = p_begin + 2 * step;
-    float x[8];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      x[r] = s[0][r] * scale_log2;
-      x[4 + r] = s[1][r] * scale_log2;
-    }
-    // tokens past the context (or the wave's last page) are masked; their V
-    // slots are zeroed too
-    const bool partial = (pageA + 2) * 16 > Lctx || pageA + 1 >= p_end;
+    // ---- online softmax over the step's 32 tokens ----
+    const int page0 = p_begin + kStepPages * step;
+    // tokens past the context (or past the walk's last page) are masked;
+    // their V slots are zeroed too, so stale cache bytes (NaN patterns
+    // included) in a partially filled page cannot reach the PV product
+    const int tok_end = min(Lctx, 16 * p_end);
+    const bool partial = (page0 + kStepPages) * 16 > tok_end;
+    float x[8], vs[kStepPages];
     bool slot_ok[8];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int tA = pageA * 16 + 4 * grp + r;
-      slot_ok[r] = tA < Lctx;
-      slot_ok[4 + r] = (tA + 16 < Lctx) && (pageA + 1 < p_end);
+    for (int pp = 0; pp < kStepPages; ++pp) {
+      float c = scale_log2;
+      vs[pp] = 1.f;
+      if (FP8) {
+        c *= lane_val(ksc_lane, kStepPages * step + pp);
+        vs[pp] = lane_val(vsc_lane, kStepPages * step + pp);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        x[4 * pp + r] = s[pp][r] * c;
+        slot_ok[4 * pp + r] = (page0 + pp) * 16 + 4 * grp + r < tok_end;
+      }
     }
     if (partial) {
 #pragma unroll
@@ -257,373 +386,36 @@ void decode_split_kernel(
     float p[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) p[i] = fast_exp2(x[i] - msub);
-    l_run += (p[0] + p[1]) + (p[2] + p[3]) + (p[4] + p[5]) + (p[6] + p[7]);
-    vec8 pa;
+    l_run += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+    // P operand (v scale folded in): k values 0-3 of a lane are its 4 tokens
+    // of the first page, 4-7 of the second
+    u32x4 pw;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const vec2 ua = Tr::pack2(p[2 * j], p[2 * j + 1]);
-      const vec2 ub = Tr::pack2(p[4 + 2 * j], p[4 + 2 * j + 1]);
-      pa[2 * j] = ua[0];
-      pa[2 * j + 1] = ua[1];
-      pa[4 + 2 * j] = ub[0];
-      pa[4 + 2 * j + 1] = ub[1];
-    }
-
-    // O += P V^T
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      // tr16: source lane (j = l16/4, c = l16%4) -> row (16pp + 4grp + j), col 16nb + 4c
-      const uint16_t* vl = (const uint16_t*)wlds;
-      const int row = 4 * grp + (l16 >> 2);
-      const int col = 16 * nb + 4 * (l16 & 3);
-      const vec4 lo = Tr::tr_read((const CA_LDS void*)(vl + row * (D + 16) + col));
-      const vec4 hi = Tr::tr_read((const CA_LDS void*)(vl + (16 + row) * (D + 16) + col));
-      vec8 bv = cat4<vec8, vec4>(lo, hi);
-      if (partial) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (!slot_ok[i]) bv[i] = 0;
-      }
-      o[nb] = Tr::mfma16(pa, bv, o[nb]);
-    }
-    __builtin_amdgcn_wave_barrier();
-  };
-
-  // ---- the walk: register sets A and B alternate ----
-  ContigRegs<D> A, B;
-  if (n_steps > 0) load_step(A, 0);
-  for (int step = 0; step < n_steps; step += 2) {
-    if (step + 1 < n_steps) load_step(B, step + 1);
-    compute_step(A, step);
-    if (step + 1 >= n_steps) break;
-    if (step + 2 < n_steps) load_step(A, step + 2);
-    compute_step(B, step + 1);
-  }
-
-  // ---- totals over the 4 lanes of a head; m is already uniform ----
-  l_run = pair16_sum(l_run);
-  l_run = pair32_sum(l_run);
-  const bool single = (n_splits == 1);
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int g = 4 * grp + r;
-    const float lg = __shfl(l_run, g, 64);
-    const float mg = __shfl(m_run, g, 64);
-    if (g >= Gc) continue;
-    const float inv = (lg > 0.f) ? 1.f / lg : 0.f;
-    const int hq = hq0 + g;
-    if (single) {
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        const vec2 pk = Tr::pack2(o[nb][r] * inv, 0.f);
-        O[((size_t)n * Hq + hq) * D + 16 * nb + l16] = (uint16_t)(__builtin_bit_cast(uint32_t, pk) & 0xffffu);
-      }
-    } else {
-      const size_t slot = ((size_t)n * Hq + hq) * max_splits + split;
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) ws_o[slot * D + 16 * nb + l16] = o[nb][r] * inv;
-      if (l16 == 0) ws_lse[slot] = (lg > 0.f) ? mg + __log2f(lg) : kNegInf;
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Paged decode with HBM -> LDS direct loads.
-//
-// Same math and work split as decode_split_kernel, but the pages travel from
-// HBM straight into a per-wave LDS ring with global_load_lds_dwordx4 (each
-// lane's 16 bytes land at ring slot + 16 * lane), so bytes in flight cost no
-// VGPRs: a wave keeps kRing - 1 steps (two pages each, K and V) in flight.
-// LDS is read with hand-issued ds_read instructions and the vector-memory
-// counter is waited on explicitly (s_waitcnt vmcnt(N) with N = the loads
-// issued after the step being consumed); the compiler's own conservative
-// wait-for-everything before LDS reads would serialise the ring.
-// Layouts in a ring slot: K pages as loaded ([D][16]; the 16-bit page's
-// 16-byte chunks are XOR-swizzled on bit 3 of the chunk index by row-octet
-// parity so the tr16 reads of lane groups 0/1 and 2/3 hit disjoint banks),
-// V pages [D][16] with the 16-bit page's chunks swizzled too (chunk q at
-// q ^ bit 4 of q): a 32-lane half of a V read takes the first or second 16
-// bytes of 16 rows, 32 bytes apart, which without the swizzle put rows r
-// and r + 8 on the same banks (a b64 read is conflict-free when each half
-// covers 256 distinct bytes modulo 256). FP8 V rows are 16 bytes, and a
-// b32 read of a lane's 4 tokens is 2-way conflicting (its halves need 32
-// distinct dwords modulo 128 bytes from 16 rows, two dwords each), so the
-// FP8 lanes read 8 bytes (tokens 8 (grp / 2) .. + 7: lane groups 0/1 and
-// 2/3 read the same addresses, 16 rows x 8 bytes per half) and keep the
-// dword of their own group.
-// ---------------------------------------------------------------------------
-// Ring depth (steps of one page, K and V, in flight per wave) and pages per
-// split of the direct-load decode: 256 KB of K and V per split for both
-// cache kinds (128 fp8 pages, two page-id registers per lane; 64 16-bit
-// pages, one). A split's start (context length, block-table row, scales,
-// filling the ring) is paid once per split: 128 fp8 pages measured +3.5 % on
-// C4 over 64, while 128 16-bit pages leave C3 too few waves (-3 %). One page
-// per step keeps a ring slot small (K + V of one page), so more waves fit a
-// CU's LDS and more bytes are in flight per CU; the PV product then runs on
-// 16x16x16 MFMAs, whose 4 k-values per lane are exactly the 4 tokens a lane
-// holds. Page loads use the "nt" cache policy: every cache byte is read
-// once per launch, so it is streamed rather than retained.
-template <int KIND>
-struct DmaCfg {
-  // (rings of 3 / 2 fp8 steps or 2 16-bit steps, which let more waves share
-  // a CU, measured within +-1 % on C4 / C3)
-  // (the stream-K walk uses the same depths: deeper rings measured within
-  // -0.5 % at head dim 128 and -3 .. +4 % at 64)
-  static constexpr int kRing = KIND == kKindPagedFp8 ? 4 : 3;
-  static constexpr int kPages = KIND == kKindPagedFp8 ? 128 : kPagesPerWave;
-  // pages per ring fill of the stream-K walk
-  static constexpr int kSkPages = 128;
-  // decode_workspace_bytes sizes the partials for kPagesPerWave-page splits
-  static_assert(kPages >= kPagesPerWave, "pages per split");
-};
-constexpr int kDmaPolicy = 2;  // global_load_lds cache policy bits: nt
-
-// The wave's GQA group of query rows (Gc <= 16 heads from `qrow`, D each) as
-// the B operand of S^T = K^T Q^T: lane (head l16, group grp) holds d = 32 ks
-// + 8 grp .. + 7; rows past Gc are zero.
-template <typename Tr, int D>
-__device__ __forceinline__ void dma_load_q(const uint16_t* __restrict__ qrow, int Gc,
-                                           typename Tr::vec8 (&qv)[D / 32]) {
-  const int lane = threadIdx.x, l16 = lane & 15, grp = lane >> 4;
-#pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) {
-    if (l16 < Gc) {
-      qv[ks] = *(const typename Tr::vec8*)(qrow + (size_t)l16 * D + 32 * ks + 8 * grp);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) qv[ks][e] = 0;
-    }
-  }
-}
-
-// One wave's walk over pages [p_begin, p_end) (at most PAGES)
-// of one (sequence, kv head hk) whose block-table row is `bt_row`. The
-// online-softmax state (o, m_run, l_run) is carried in and out, so a
-// context can be walked in several calls; the ring is filled at the start
-// and drained at the end of each call.
-template <typename Tr, int D, int KIND, int RING = DmaCfg<KIND>::kRing,
-          int PAGES = DmaCfg<KIND>::kPages>
-__device__ __forceinline__ void dma_walk(const typename Tr::vec8 (&qv)[D / 32], f32x4 (&o)[D / 16],
-                                         float& m_run, float& l_run, unsigned char* ring,
-                                         const void* __restrict__ Kc, const void* __restrict__ Vc,
-                                         const float* __restrict__ k_scale,
-                                         const float* __restrict__ v_scale, int per_block,
-                                         const int32_t* __restrict__ bt_row, int Hkv, int hk,
-                                         int num_blocks, int p_begin, int p_end, int Lctx,
-                                         float scale_log2, const unsigned char* dummy) {
-  using vec8 = typename Tr::vec8;
-  using vec4 = typename Tr::vec4;
-  constexpr int NKS = D / 32, NB = D / 16;
-  constexpr bool FP8 = KIND == kKindPagedFp8;
-  constexpr int ELEM = FP8 ? 1 : 2;
-  constexpr int CHUNK = D * 16 * ELEM;        // bytes of one (page, head) chunk
-  constexpr int NDMA = CHUNK / 1024;          // 16 B x 64 lanes per load
-  constexpr int STAGE = 2 * CHUNK;            // K and V of the step's page
-  constexpr int DPS = 2 * NDMA;               // loads per step
-  constexpr int KRD = FP8 ? NKS : 2 * NKS;    // LDS reads for one page's K^T operands
-  constexpr int PB = PAGES / 64;              // page-id registers per lane
-  static_assert(PAGES % 64 == 0 && PB <= 2, "pages per split");
-  static_assert((RING - 1) * DPS <= 63, "vmcnt range");
-
-  const int lane = threadIdx.x;
-  const int l16 = lane & 15, grp = lane >> 4;
-  const int n_steps = p_end - p_begin;
-
-  // page ids and per-page scales: lane j of register b holds page
-  // p_begin + 64 b + j; read back for page index i (uniform) with lane_val
-  int pid_lane[PB];
-  float ksc_lane[PB], vsc_lane[PB];
-#pragma unroll
-  for (int pb = 0; pb < PB; ++pb) {
-    const int page = p_begin + 64 * pb + lane;
-    pid_lane[pb] = 0;
-    ksc_lane[pb] = vsc_lane[pb] = 1.f;
-    if (page < p_end) {
-      pid_lane[pb] = bt_row[page];
-      pid_lane[pb] = min(max(pid_lane[pb], 0), num_blocks - 1);
-    }
-    if (FP8) {
-      if (per_block) {
-        if (page < p_end) {
-          ksc_lane[pb] = k_scale[(size_t)pid_lane[pb] * Hkv + hk];
-          vsc_lane[pb] = v_scale[(size_t)pid_lane[pb] * Hkv + hk];
-        }
-      } else {
-        ksc_lane[pb] = k_scale[hk];
-        vsc_lane[pb] = v_scale[hk];
-      }
-    }
-  }
-  auto lane_val = [&](const auto (&r)[PB], int i) CA_INLINE {
-    const auto v = (PB > 1 && i >= 64) ? r[PB - 1] : r[0];
-    return __builtin_bit_cast(std::remove_const_t<std::remove_reference_t<decltype(r[0])>>,
-                              __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i & 63));
-  };
-
-  // source byte offset of this lane's 16 bytes for load i of a K chunk
-  auto k_src = [&](int i) -> int {
-    const int p = 64 * i + lane;  // physical 16-byte slot in LDS
-    if (FP8) return 16 * p;
-    return 16 * (p ^ (((p >> 4) & 1) << 3));
-  };
-  // source offset of this lane's 16 bytes in each 1 KB of a V chunk
-  const int v_src = 16 * (FP8 ? lane : lane ^ ((lane >> 4) & 1));
-  auto issue_step = [&](int step, int slot) {
-    unsigned char* base = ring + slot * STAGE;
-    const bool valid = step < n_steps;
-    const int pid = lane_val(pid_lane, valid ? step : 0);
-    const size_t chunk = ((size_t)pid * Hkv + hk) * (size_t)CHUNK;
-    const unsigned char* kp = (const unsigned char*)Kc + chunk;
-    const unsigned char* vp = (const unsigned char*)Vc + chunk;
-#pragma unroll
-    for (int i = 0; i < NDMA; ++i) {
-      dma16<kDmaPolicy>(valid ? kp + k_src(i) : dummy, (CA_LDS void*)(base + 1024 * i));
-      dma16<kDmaPolicy>(valid ? vp + 1024 * i + v_src : dummy,
-                        (CA_LDS void*)(base + CHUNK + 1024 * i));
-    }
-  };
-
-  // per-lane LDS read offsets inside a page's K / V chunk
-  uint32_t k_lo, k_hi;
-  if (FP8) {
-    k_lo = 16 * (8 * grp + (l16 >> 1)) + 8 * (l16 & 1);
-    k_hi = 0;
-  } else {
-    const int c = l16 & 3, j = l16 >> 2, par = grp & 1;
-    k_lo = 16 * (16 * grp + 8 * par + 2 * j + (c >> 1)) + 8 * (c & 1);
-    k_hi = 16 * (16 * grp + 8 * (1 - par) + 2 * j + (c >> 1)) + 8 * (c & 1);
-  }
-  // V: lane (d = l16, token group grp) needs tokens 4 grp .. 4 grp + 3 of row d
-  // (FP8: the 8 bytes of tokens 8 (grp / 2) .. + 7, then its own dword)
-  const uint32_t v_off = FP8 ? (uint32_t)(16 * l16 + 8 * (grp >> 1))
-                             : (uint32_t)(16 * ((2 * l16 + (grp >> 1)) ^ ((l16 >> 3) & 1)) + 8 * (grp & 1));
-  const uint32_t ring0 = lds_off(ring);
-
-  // RING steps in flight from the start; a slot is refilled as soon as its
-  // LDS reads have returned, so RING steps stay in flight during the math
-#pragma unroll
-  for (int st = 0; st < RING; ++st) issue_step(st, st);
-  int slot = 0;
-  for (int step = 0; step < n_steps; ++step) {
-    wait_vmcnt<(RING - 1) * DPS>();  // this step's loads are the oldest outstanding
-    const uint32_t kb = ring0 + slot * STAGE;
-    const uint32_t vb = kb + CHUNK + v_off;
-
-    // ---- LDS -> operands ----
-    u32x2 kraw[KRD];
-    u32x2 v8r[FP8 ? NB : 1];
-    u32x2 v16r[FP8 ? 1 : NB];
-    if (FP8) {
-      const uint32_t a = kb + k_lo;
-      kraw[0] = lds_read_tr8<0>(a);
-      if (NKS > 1) kraw[1 % KRD] = lds_read_tr8<512>(a);
-      if (NKS > 2) kraw[2 % KRD] = lds_read_tr8<1024>(a);
-      if (NKS > 3) kraw[3 % KRD] = lds_read_tr8<1536>(a);
-#define CA_V8(NBI) if (NBI < NB) v8r[NBI % NB] = lds_read_b64<256 * NBI>(vb);
-      CA_V8(0) CA_V8(1) CA_V8(2) CA_V8(3) CA_V8(4) CA_V8(5) CA_V8(6) CA_V8(7)
-#undef CA_V8
-    } else {
-      const uint32_t alo = kb + k_lo, ahi = kb + k_hi;
-      kraw[0] = lds_read_tr16<0>(alo);
-      kraw[1] = lds_read_tr16<0>(ahi);
-      if (NKS > 1) { kraw[2 % KRD] = lds_read_tr16<1024>(alo); kraw[3 % KRD] = lds_read_tr16<1024>(ahi); }
-      if (NKS > 2) { kraw[4 % KRD] = lds_read_tr16<2048>(alo); kraw[5 % KRD] = lds_read_tr16<2048>(ahi); }
-      if (NKS > 3) { kraw[6 % KRD] = lds_read_tr16<3072>(alo); kraw[7 % KRD] = lds_read_tr16<3072>(ahi); }
-#define CA_V16(NBI) if (NBI < NB) v16r[NBI % NB] = lds_read_b64<512 * NBI>(vb);
-      CA_V16(0) CA_V16(1) CA_V16(2) CA_V16(3) CA_V16(4) CA_V16(5) CA_V16(6) CA_V16(7)
-#undef CA_V16
-    }
-    wait_lgkm0();
-#pragma unroll
-    for (int i = 0; i < KRD; ++i) after_wait(kraw[i]);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      if (FP8) after_wait(v8r[i % (FP8 ? NB : 1)]);
-      else after_wait(v16r[i % (FP8 ? 1 : NB)]);
-    }
-    issue_step(step + RING, slot);  // the slot's data is in registers now
-
-    // ---- S^T of the page ----
-    f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      vec8 a;
-      if (FP8) {
-        a = fp8x8_to<Tr>(kraw[ks % KRD][0], kraw[ks % KRD][1]);
-      } else {
-        const u32x4 t = {kraw[(2 * ks) % KRD][0], kraw[(2 * ks) % KRD][1],
-                         kraw[(2 * ks + 1) % KRD][0], kraw[(2 * ks + 1) % KRD][1]};
-        a = __builtin_bit_cast(vec8, t);
-      }
-      s = Tr::mfma16(a, qv[ks], s);
-    }
-
-    // ---- online softmax over the page's 16 tokens ----
-    const int page0 = p_begin + step;
-    float c = scale_log2, vs = 1.f;
-    if (FP8) {
-      c *= lane_val(ksc_lane, step);
-      vs = lane_val(vsc_lane, step);
-    }
-    float x[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) x[r] = s[r] * c;
-    // tokens past the context are masked; their V slots are zeroed too, so
-    // stale cache bytes (NaN patterns included) in a partially filled page
-    // cannot reach the PV product
-    const bool partial = (page0 + 1) * 16 > Lctx;
-    bool slot_ok[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) slot_ok[r] = page0 * 16 + 4 * grp + r < Lctx;
-    if (partial) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (!slot_ok[i]) x[i] = kNegInf;
-    }
-    float tmax = max3(x[0], x[1], __builtin_fmaxf(x[2], x[3]));
-    tmax = pair16_max(tmax);
-    tmax = pair32_max(tmax);
-    const bool need = tmax > m_run + 8.0f;
-    if (wave_any(need)) {
-      const float m_new = __builtin_fmaxf(m_run, tmax);
-      const float alpha = (m_new == kNegInf) ? 1.f : fast_exp2(m_run - m_new);
-#pragma unroll
-      for (int i = 0; i < NB; ++i) o[i] *= alpha;
-      l_run *= alpha;
-      m_run = m_new;
-    }
-    const float msub = (m_run == kNegInf) ? 0.f : m_run;
-    float p[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) p[i] = fast_exp2(x[i] - msub);
-    float psum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) psum += p[i];
-    l_run += psum;
-    // P operand (v scale folded in): the lane's 4 tokens (16x16x16)
-    u32x2 pw;
-    pw[0] = __builtin_bit_cast(uint32_t, Tr::pack2(p[0] * vs, p[1] * vs));
-    pw[1] = __builtin_bit_cast(uint32_t, Tr::pack2(p[2] * vs, p[3] * vs));
+    for (int j = 0; j < 4; ++j)
+      pw[j] = __builtin_bit_cast(uint32_t, Tr::pack2(p[2 * j] * vs[j / 2], p[2 * j + 1] * vs[j / 2]));
 
     // ---- O += P V^T ----
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      u32x2 bw;
-      if (FP8) {
-        const uint32_t v = (grp & 1) ? v8r[nb % (FP8 ? NB : 1)][1] : v8r[nb % (FP8 ? NB : 1)][0];
-        bw[0] = __builtin_bit_cast(uint32_t, Fp8Conv<Tr>::template cvt<false>(v));
-        bw[1] = __builtin_bit_cast(uint32_t, Fp8Conv<Tr>::template cvt<true>(v));
-      } else {
-        bw[0] = v16r[nb % (FP8 ? 1 : NB)][0];
-        bw[1] = v16r[nb % (FP8 ? 1 : NB)][1];
+      u32x4 bw;
+#pragma unroll
+      for (int pp = 0; pp < kStepPages; ++pp) {
+        if (FP8) {
+          const uint32_t v = (grp & 1) ? vop[pp][nb][1] : vop[pp][nb][0];
+          bw[2 * pp] = __builtin_bit_cast(uint32_t, Fp8Conv<Tr>::template cvt<false>(v));
+          bw[2 * pp + 1] = __builtin_bit_cast(uint32_t, Fp8Conv<Tr>::template cvt<true>(v));
+        } else {
+          bw[2 * pp] = vop[pp][nb][0];
+          bw[2 * pp + 1] = vop[pp][nb][1];
+        }
       }
       if (partial) {
         // zero masked token slots: 16-bit halves of the operand dwords
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 8; ++i)
           if (!slot_ok[i]) bw[i >> 1] &= (i & 1) ? 0x0000ffffu : 0xffff0000u;
       }
-      o[nb] = Tr::mfma16k16(__builtin_bit_cast(vec4, pw), __builtin_bit_cast(vec4, bw), o[nb]);
+      o[nb] = Tr::mfma16(__builtin_bit_cast(vec8, pw), __builtin_bit_cast(vec8, bw), o[nb]);
     }
     slot = (slot == RING - 1) ? 0 : slot + 1;
   }
@@ -640,7 +432,7 @@ __device__ __forceinline__ void dma_finish(const f32x4 (&o)[D / 16], float m_run
                                            float* __restrict__ plse, size_t plse_stride) {
   using vec2 = typename Tr::vec2;
   constexpr int NB = D / 16;
-  const int lane = threadIdx.x, l16 = lane & 15, grp = lane >> 4;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, grp = lane >> 4;
   l_run = pair16_sum(l_run);
   l_run = pair32_sum(l_run);
 #pragma unroll
@@ -664,24 +456,47 @@ __device__ __forceinline__ void dma_finish(const f32x4 (&o)[D / 16], float m_run
   }
 }
 
-// Split grid: one wave per split of DmaCfg<KIND>::kPages pages of one
-// (sequence, kv head, query-head chunk of <= 16).
-template <typename Tr, int D, int KIND>
-__global__ __launch_bounds__(64) void decode_dma_kernel(
+// Split grid: one workgroup of NW waves per split of `pages_per_split` pages
+// of one (sequence, kv head, query-head chunk of <= 16). The waves take equal
+// contiguous shares of the split's pages, each with its own ring and online
+// softmax, and their results meet in LDS. Bound by latency: a wave's step is
+// one dependent chain (about 0.5 us), so a split walked by a single wave took
+// 34 us for 1000 tokens of a 16-bit cache where 8 waves take 9-13, and 73 us
+// for 2000 tokens of an FP8 one where they take 16; a contiguous cache of 4001
+// tokens, 8 heads, 63 us -> 16.
+template <int KIND, int D, int NW>
+struct MwCfg {
+  static constexpr int kStep = kStepPages * 2 * D * 16 * (KIND == kKindPagedFp8 ? 1 : 2);  // K + V of a step
+  // One step in flight per wave where several workgroups share a CU; two for
+  // the 8-wave workgroups, which have a CU to themselves, if LDS holds them
+  // (64 splits of 4096 contiguous tokens, head dim 64: 21.2 -> 19.6 us; two
+  // steps for 4-wave workgroups of a 4 KB step: 34.5 -> 37.9 us).
+  static constexpr int kRing = NW == 8 && 2 * kStep * NW <= 128 * 1024 ? 2 : 1;
+  static constexpr int kPages = 128;      // pages per call of dma_walk (two page-id registers)
+};
+
+template <typename Tr, int D, int KIND, int NW>
+__global__ __launch_bounds__(64 * NW) void decode_mw_kernel(
     const uint16_t* __restrict__ Q, const void* __restrict__ Kc, const void* __restrict__ Vc,
     const float* __restrict__ k_scale, const float* __restrict__ v_scale, int per_block,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ context_lens,
     uint16_t* __restrict__ O, float* __restrict__ ws_o, float* __restrict__ ws_lse, int Hq,
-    int Hkv, int max_blocks, int num_blocks, int max_splits, int n_hc, float scale_log2) {
+    int Hkv, int max_blocks, int S_contig, int num_blocks, int max_splits, int pages_per_split,
+    int n_hc, float scale_log2) {
+  using Cfg = MwCfg<KIND, D, NW>;
+  constexpr bool CONTIG = KIND == kKindContig16;
   constexpr int NKS = D / 32, NB = D / 16;
-  constexpr int STAGE = 2 * D * 16 * (KIND == kKindPagedFp8 ? 1 : 2);
-  constexpr int kDmaPages = DmaCfg<KIND>::kPages;
-  __shared__ __attribute__((aligned(1024))) unsigned char ring[DmaCfg<KIND>::kRing * STAGE];
+  constexpr int kRingB = Cfg::kRing * Cfg::kStep;
+  static_assert(kRingB >= 16 * D * 4, "a wave's ring holds its 16 x D floats for the merge");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[NW * kRingB];
+  __shared__ float red_m[NW][16], red_l[NW][16];
 
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, l16 = lane & 15, grp = lane >> 4;
   int w = blockIdx.x;
-  // split index outermost, counted from each sequence's end: the waves of
-  // splits before a sequence's start (none exist) come first and retire at
-  // once, and every sequence's last (partial) split is in the final group
+  // split index outermost, counted from each sequence's end: the workgroups
+  // of splits before a sequence's start (none exist) come first and retire
+  // at once, and every sequence's last (partial) split is in the final group
   const int per_split = (int)(gridDim.x / max_splits);
   const int from_end = max_splits - 1 - w / per_split;
   w %= per_split;
@@ -692,29 +507,79 @@ __global__ __launch_bounds__(64) void decode_dma_kernel(
   const int Gq = Hq / Hkv;
   const int hq0 = hk * Gq + hc * 16;
   const int Gc = min(16, Gq - hc * 16);
-  const int Lctx = min(max(0, context_lens[n]), max_blocks * kDecodePage);
+  const int Lctx = CONTIG ? S_contig : min(max(0, context_lens[n]), max_blocks * kDecodePage);
   const int n_pages = (Lctx + kDecodePage - 1) / kDecodePage;
-  const int n_splits = max(1, (n_pages + kDmaPages - 1) / kDmaPages);
+  const int n_splits = max(1, (n_pages + pages_per_split - 1) / pages_per_split);
   const int split = n_splits - 1 - from_end;
   if (split < 0) return;
-  const int p_begin = split * kDmaPages;
-  const int p_end = min(p_begin + kDmaPages, n_pages);
+  const int s_begin = split * pages_per_split;
+  const int s_len = min(pages_per_split, n_pages - s_begin);
+  const int p_begin = s_begin + wave * s_len / NW, p_end = s_begin + (wave + 1) * s_len / NW;
 
-  typename Tr::vec8 qv[NKS];
-  dma_load_q<Tr, D>(Q + ((size_t)n * Hq + hq0) * D, Gc, qv);
   f32x4 o[NB];
 #pragma unroll
   for (int i = 0; i < NB; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m_run = kNegInf, l_run = 0.f;
-  dma_walk<Tr, D, KIND>(qv, o, m_run, l_run, ring, Kc, Vc, k_scale, v_scale, per_block,
-                        block_tables + (size_t)n * max_blocks, Hkv, hk, num_blocks, p_begin, p_end,
-                        Lctx, scale_log2, (const unsigned char*)Q);
-  if (n_splits == 1) {
-    dma_finish<Tr, D>(o, m_run, l_run, Gc, O + ((size_t)n * Hq + hq0) * D, nullptr, 0, nullptr, 0);
-  } else {
-    const size_t sl = ((size_t)n * Hq + hq0) * max_splits + split;
-    dma_finish<Tr, D>(o, m_run, l_run, Gc, nullptr, ws_o + sl * D, (size_t)max_splits * D,
-                      ws_lse + sl, (size_t)max_splits);
+  if (p_begin < p_end) {
+    typename Tr::vec8 qv[NKS];
+    dma_load_q<Tr, D>(Q + ((size_t)n * Hq + hq0) * D, Gc, qv);
+    const size_t head = CONTIG ? ((size_t)n * Hkv + hk) * (size_t)S_contig * (2 * D) : 0;
+    for (int p = p_begin; p < p_end; p += Cfg::kPages)
+      dma_walk<Tr, D, KIND, Cfg::kRing, Cfg::kPages>(
+          qv, o, m_run, l_run, lds + wave * kRingB, (const unsigned char*)Kc + head,
+          (const unsigned char*)Vc + head, k_scale, v_scale, per_block,
+          CONTIG ? nullptr : block_tables + (size_t)n * max_blocks, Hkv, hk, num_blocks, p,
+          min(p + Cfg::kPages, p_end), Lctx, scale_log2, (const unsigned char*)Q);
+  }
+
+  if constexpr (NW == 1) {
+    if (n_splits == 1) {
+      dma_finish<Tr, D>(o, m_run, l_run, Gc, O + ((size_t)n * Hq + hq0) * D, nullptr, 0, nullptr, 0);
+    } else {
+      const size_t sl = ((size_t)n * Hq + hq0) * max_splits + split;
+      dma_finish<Tr, D>(o, m_run, l_run, Gc, nullptr, ws_o + sl * D, (size_t)max_splits * D,
+                        ws_lse + sl, (size_t)max_splits);
+    }
+    return;
+  }
+  // ---- the waves' results meet in LDS: wave i's rows in its own ring ----
+  l_run = pair16_sum(l_run);
+  l_run = pair32_sum(l_run);
+  if (lane < 16) {
+    red_m[wave][l16] = m_run;
+    red_l[wave][l16] = l_run;
+  }
+  float* rows = (float*)(lds + wave * kRingB);
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (4 * grp + r < Gc) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) rows[(4 * grp + r) * D + 16 * nb + l16] = o[nb][r];
+    }
+  __syncthreads();
+  for (int i = threadIdx.x; i < Gc * D; i += 64 * NW) {
+    const int g = i / D, d = i % D;
+    float M = red_m[0][g];
+#pragma unroll
+    for (int j = 1; j < NW; ++j) M = __builtin_fmaxf(M, red_m[j][g]);
+    float l = 0.f, acc = 0.f;
+    if (M != kNegInf) {
+#pragma unroll
+      for (int j = 0; j < NW; ++j) {
+        const float a = fast_exp2(red_m[j][g] - M);
+        l += a * red_l[j][g];
+        acc += a * ((const float*)(lds + j * kRingB))[g * D + d];
+      }
+    }
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const size_t hq = (size_t)n * Hq + hq0 + g;
+    if (n_splits == 1) {
+      Tr::store(O, hq * D + d, acc * inv);
+    } else {
+      const size_t sl = hq * max_splits + split;
+      ws_o[sl * D + d] = acc * inv;
+      if (d == 0) ws_lse[sl] = l > 0.f ? M + __log2f(l) : kNegInf;
+    }
   }
 }
 
@@ -752,7 +617,7 @@ __global__ __launch_bounds__(64) void decode_sk_kernel(
     int32_t* __restrict__ ws_prefix, int N, int Hq, int Hkv, int max_blocks, int num_blocks,
     int n_hc, float scale_log2) {
   constexpr int NKS = D / 32, NB = D / 16;
-  constexpr int STAGE = 2 * D * 16 * (KIND == kKindPagedFp8 ? 1 : 2);
+  constexpr int STAGE = kStepPages * 2 * D * 16 * (KIND == kKindPagedFp8 ? 1 : 2);
   constexpr int kDmaPages = DmaCfg<KIND>::kSkPages;
   constexpr int NCH = kSkMaxSeqs / 64;
   __shared__ __attribute__((aligned(1024))) unsigned char ring[DmaCfg<KIND>::kRing * STAGE];
@@ -971,6 +836,22 @@ __global__ __launch_bounds__(64) void decode_sk_merge_kernel(
                     ws_o, ws_lse, O, orow);
 }
 
+// Splits per (sequence, kv head, chunk) of a contiguous decode of `segs` of
+// them, `pages` pages each: enough for two workgroups per CU (160 heads of
+// 3000 tokens, head dim 128: 43 us against 51 with one split, 43 with twice as
+// many), as far as the workspace goes; none when the heads alone are about one
+// workgroup per CU, which saves the merge (256 heads of 4096 tokens, head dim
+// 64: 47 us against 52 with two splits).
+static int contig_splits(long long segs, int pages) {
+  const int cus = device_cus();
+  if (segs <= cus && segs >= cus - cus / 8) return 1;
+  const int most = std::max(1, pages / kPagesPerWave + (pages % kPagesPerWave != 0));
+  int s = 1;
+  while (s < most && segs * s < 2 * cus) ++s;
+  const int per = std::max(1, (pages + s - 1) / s);
+  return std::max(1, (pages + per - 1) / per);
+}
+
 // Bytes of split partials for max_splits splits per (sequence, query head):
 // [N][Hq][max_splits] x D floats of o / l, then [N][Hq][max_splits] floats
 // of log2-sum-exp; none when every context fits one split.
@@ -987,9 +868,9 @@ size_t decode_workspace_bytes(int N, int Hq, int D, int max_tokens) {
 
 // Waves per CU of a stream-K launch. Every wave streams the same bytes, so a
 // CU must hold a multiple of four for its SIMDs to finish together; one per
-// SIMD measured best, except where a page step is only 2 KB (FP8 at head dim
-// 64): there one wave cannot cover its own per-step latency, and two per
-// SIMD run 5632-6006 GB/s against 4375-4611 (reference-grid shapes).
+// SIMD measured best, except where a page is only 2 KB (FP8 at head dim 64):
+// there one wave cannot cover its own per-step latency (256 sequences of up to
+// 16000 tokens: 408 us with two per SIMD, 420 with one).
 template <int KIND, int D>
 constexpr int sk_waves_per_cu() {
   return 2 * D * 16 * (KIND == kKindPagedFp8 ? 1 : 2) < 4096 ? 8 : 4;
@@ -1049,6 +930,22 @@ static PagedPlan paged_plan(int N, int Hq, int Hkv, int max_blocks) {
   return p;
 }
 
+// Waves per workgroup of a split grid of `grid` workgroups, at most `pages`
+// pages each. A share of a few pages does not pay for the merge in LDS (128
+// sequences of up to 200 tokens: one wave 15.4 us, four 19.4); up to one
+// workgroup per CU, eight waves shorten the chain further (one sequence of
+// 1000 tokens, 8 kv heads: 9.0 us against 10.7 with four).
+static int mw_waves(long long grid, int pages) {
+  if (pages <= 16) return 1;
+  return grid <= device_cus() && pages >= 32 ? 8 : 4;
+}
+template <typename Tr, int D, int KIND>
+static auto mw_kernel(int nw) {
+  return nw == 8   ? &decode_mw_kernel<Tr, D, KIND, 8>
+         : nw == 4 ? &decode_mw_kernel<Tr, D, KIND, 4>
+                   : &decode_mw_kernel<Tr, D, KIND, 1>;
+}
+
 template <typename Tr, int D, int KIND>
 static hipError_t launch_paged_decode_t(const void* q, const void* kc, const void* vc,
                                         const float* k_scale, const float* v_scale, int per_block,
@@ -1082,10 +979,11 @@ static hipError_t launch_paged_decode_t(const void* q, const void* kc, const voi
   const long long total_waves = (long long)N * Hkv * n_hc * max_splits;
   if (total_waves == 0) return hipSuccess;
   if (total_waves > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((decode_dma_kernel<Tr, D, KIND>), dim3((unsigned)total_waves), dim3(64), 0,
-                     stream, (const uint16_t*)q, kc, vc, k_scale, v_scale, per_block, bt, lens,
-                     (uint16_t*)out, ws_o, ws_lse, Hq, Hkv, max_blocks, num_blocks, max_splits,
-                     n_hc, scale * kLog2e);
+  const int nw = mw_waves(total_waves, std::min(max_blocks, DmaCfg<KIND>::kPages));
+  const auto kernel = mw_kernel<Tr, D, KIND>(nw);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)total_waves), dim3(64 * nw), 0, stream, (const uint16_t*)q, kc, vc, k_scale, v_scale, per_block, bt, lens,
+                     (uint16_t*)out, ws_o, ws_lse, Hq, Hkv, max_blocks, 0, num_blocks, max_splits,
+                     DmaCfg<KIND>::kPages, n_hc, scale * kLog2e);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || max_splits <= 1) return e;
   hipLaunchKernelGGL((decode_merge_kernel<Tr, D>), dim3((unsigned)(N * Hq)), dim3(64), 0, stream,
@@ -1097,26 +995,28 @@ template <typename Tr, int D>
 static hipError_t launch_contig_decode_t(const void* q, const void* k, const void* v, void* out,
                                          int N, int Hq, int Hkv, int S, float scale, void* ws,
                                          size_t ws_bytes, hipStream_t stream) {
-  const int pages = (S + kDecodePage - 1) / kDecodePage;
-  const int max_splits = max(1, (pages + kPagesPerWave - 1) / kPagesPerWave);
+  constexpr int KIND = kKindContig16;
+  const int pages = S / kDecodePage + (S % kDecodePage != 0);
   const int Gq = Hq / Hkv;
   const int n_hc = (Gq + 15) / 16;
   const size_t need = decode_workspace_bytes(N, Hq, D, S);
   if (ws_bytes < need) return hipErrorInvalidValue;
+  const int max_splits = contig_splits((long long)N * Hkv * n_hc, pages);
+  const int pages_per_split = std::max(1, (pages + max_splits - 1) / max_splits);
   float* ws_o = (float*)ws;
   float* ws_lse = need ? ws_o + (size_t)N * Hq * max_splits * D : nullptr;
-  const long long total_waves = (long long)N * Hkv * n_hc * max_splits;
-  if (total_waves == 0) return hipSuccess;
-  const long long grid = (total_waves + kDecodeWgWaves - 1) / kDecodeWgWaves;
+  const long long grid = (long long)N * Hkv * n_hc * max_splits;
+  if (grid == 0) return hipSuccess;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((decode_split_kernel<Tr, D>), dim3((unsigned)grid), dim3(kDecodeWgWaves * 64),
-                     0, stream, (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,
-                     (uint16_t*)out, ws_o, ws_lse, Hq, Hkv, S, max_splits, n_hc, total_waves,
-                     scale * kLog2e);
+  const int nw = mw_waves(grid, pages_per_split);
+  const auto kernel = mw_kernel<Tr, D, KIND>(nw);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * nw), 0, stream, (const uint16_t*)q, k, v, nullptr, nullptr, 0, nullptr, nullptr,
+                     (uint16_t*)out, ws_o, ws_lse, Hq, Hkv, 0, S, 1, max_splits, pages_per_split,
+                     n_hc, scale * kLog2e);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || max_splits <= 1) return e;
   hipLaunchKernelGGL((decode_merge_kernel<Tr, D>), dim3((unsigned)(N * Hq)), dim3(64), 0, stream,
-                     nullptr, S, ws_o, ws_lse, out, Hq, max_splits, kPagesPerWave);
+                     nullptr, S, ws_o, ws_lse, out, Hq, max_splits, pages_per_split);
   return hipGetLastError();
 }
 

@@ -99,14 +99,11 @@ inline long long prefill_grid(int B, int Hq, int n_qt, bool causal, int wg_per_c
   return *paired ? pairs : single;
 }
 
-// Split-K geometry of the decode kernels: pages of 16 tokens. The
-// workspace and the contiguous-cache kernel split at kPagesPerWave pages
-// (one page id per lane of a wave); the paged kernels split at a multiple of
-// it (decode.hip, DmaCfg), so the workspace sized for kPagesPerWave-page
-// splits covers them.
+// Split-K geometry of the decode kernels: pages of 16 tokens. The workspace
+// is sized for splits of kPagesPerWave pages, the finest that any kernel
+// takes (decode.hip: DmaCfg, contig_splits; the float32 kernel splits there).
 constexpr int kDecodePage = 16;
 constexpr int kPagesPerWave = 64;
-constexpr int kDecodeWgWaves = 4;  // independent waves per workgroup (contiguous kernel)
 
 // Workspace for split-K partial results: [N][Hq][max_splits] x (D + 1) floats.
 size_t decode_workspace_bytes(int N, int Hq, int D, int max_tokens);

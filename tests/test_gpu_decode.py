@@ -255,6 +255,55 @@ def test_flash_decode_gqa_split(dev, hq, hkv, kv_len):
     assert_close(to_np(out), ref, **TOL_16BIT, name="flash_decode gqa")
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("width,n", [(1, 3), (16, 6), (17, 6), (31, 6), (32, 6), (64, 6), (65, 6),
+                                     (129, 6), (40, 130)])
+def test_split_grid_waves(dev, head_dim, fp8, width, n):
+    """The split grid's workgroups of 1, 4 and 8 waves (by table width and
+    grid): contexts at the edges of pages, of two-page steps, of the waves'
+    shares and of splits; 130 sequences x 2 kv heads are more workgroups than
+    CUs. Bytes past each length are NaN patterns."""
+    edge = [0, 1, 16, 17, 33, 16 * width - 17, 16 * width - 1, 16 * width]
+    lens = [min(max(edge[-1 - i % len(edge)], 0), 16 * width) for i in range(n)]
+    dtype = torch.float16 if head_dim == 64 else torch.bfloat16
+    case = build_paged(lens, 10, 2, head_dim, dtype, dev, fp8=fp8, seed=width)
+    assert case["block_tables"].shape[1] == width
+    assert not balanced_walk_taken(n, 10, 2, head_dim, width, fp8)
+    ref = paged_oracle(case)
+    for i, length in enumerate(lens):
+        if length % 16:
+            blk = int(case["block_tables"][i, length // 16])
+            for name in ("key_cache", "value_cache"):
+                case[name][blk, :, :, length % 16:] = 0x7F if fp8 else float("nan")
+    out = _run_paged(case)
+    torch.cuda.synchronize()
+    assert_close(to_np(out), ref, **(TOL_FP8 if fp8 else TOL_16BIT), name=f"width {width}")
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("b,hq,hkv,kv_len", [(1, 32, 8, 15), (2, 3, 1, 257), (3, 40, 2, 511),
+                                             (1, 16, 16, 513), (1, 4, 2, 4097), (30, 16, 8, 1041),
+                                             (129, 2, 2, 300), (2, 20, 4, 16369)])
+def test_flash_decode_waves_and_splits(dev, head_dim, b, hq, hkv, kv_len):
+    """Contiguous cache: one wave, 4 and 8 waves per split, none and several
+    splits, last pages of 1 to 15 tokens, groups above 16 heads; NaN follows
+    the caches in memory and must not reach the result."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(kv_len)
+    dtype = torch.float16 if head_dim == 64 else torch.bfloat16
+    q = torch.randn(b, hq, 1, head_dim, device=dev, generator=g).to(dtype)
+    size = b * hkv * kv_len * head_dim
+    k, v = (torch.full((size + 64 * head_dim,), float("nan"), device=dev, dtype=dtype) for _ in range(2))
+    for t in (k, v):
+        t[:size] = torch.randn(size, device=dev, generator=g).to(dtype)
+    k, v = (t[:size].view(b, hkv, kv_len, head_dim) for t in (k, v))
+    out = cuda_llm.flash_decode(q, k, v)
+    torch.cuda.synchronize()
+    assert_close(to_np(out), oracle.attention(to_np(q), to_np(k), to_np(v)), **TOL_16BIT,
+                 name=f"decode {kv_len}")
+
+
 def test_baseline_c3_shape(dev):
     """C3: N=64, Hq=32/Hkv=8, D=128, L ~ U[512, 8192], 40k-page pool,
     permuted; every sequence against the oracle."""
