@@ -291,7 +291,10 @@ __device__ __forceinline__ void dma_walk(const typename Tr::vec8 (&qv)[D / 32], 
     wait_vmcnt<(RING - 1) * DPS>();  // this step's loads are the oldest outstanding
 
     // ---- LDS -> operands ----
-    u32x4 kop[kStepPages][NKS];   // K^T operand (FP8: two dwords of codes)
+    // (kept as read until the wait: combining them earlier could copy registers
+    // that a load in flight has yet to write)
+    u32x2 klo[kStepPages][NKS], khi[kStepPages][NKS];  // K^T operand halves (FP8: codes, in klo)
+    u32x4 kop[kStepPages][NKS];                        // kContig16: the whole operand
     u32x2 vop[kStepPages][NB];    // V operand half (FP8: 8 codes, one dword kept)
 #pragma unroll
     for (int pp = 0; pp < kStepPages; ++pp) {
@@ -299,14 +302,12 @@ __device__ __forceinline__ void dma_walk(const typename Tr::vec8 (&qv)[D / 32], 
       auto k_read = [&](auto i) CA_INLINE {
         constexpr int ks = decltype(i)::value;
         if constexpr (FP8) {
-          const u32x2 t = lds_read_tr8<512 * ks>(kb + k_lo);
-          kop[pp][ks][0] = t[0];
-          kop[pp][ks][1] = t[1];
+          klo[pp][ks] = lds_read_tr8<512 * ks>(kb + k_lo);
         } else if constexpr (CONTIG) {
           kop[pp][ks] = lds_read_b128<0>(kb + c_krow + (c_k ^ (64 * ks)));
         } else {
-          const u32x2 lo = lds_read_tr16<1024 * ks>(kb + k_lo), hi = lds_read_tr16<1024 * ks>(kb + k_hi);
-          kop[pp][ks] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+          klo[pp][ks] = lds_read_tr16<1024 * ks>(kb + k_lo);
+          khi[pp][ks] = lds_read_tr16<1024 * ks>(kb + k_hi);
         }
       };
       auto v_read = [&](auto i) CA_INLINE {
@@ -322,7 +323,17 @@ __device__ __forceinline__ void dma_walk(const typename Tr::vec8 (&qv)[D / 32], 
 #pragma unroll
     for (int pp = 0; pp < kStepPages; ++pp) {
 #pragma unroll
-      for (int i = 0; i < NKS; ++i) after_wait(kop[pp][i]);
+      for (int i = 0; i < NKS; ++i) {
+        if constexpr (CONTIG) {
+          after_wait(kop[pp][i]);
+        } else {
+          after_wait(klo[pp][i]);
+          if constexpr (!FP8) {
+            after_wait(khi[pp][i]);
+            kop[pp][i] = u32x4{klo[pp][i][0], klo[pp][i][1], khi[pp][i][0], khi[pp][i][1]};
+          }
+        }
+      }
 #pragma unroll
       for (int i = 0; i < NB; ++i) after_wait(vop[pp][i]);
     }
@@ -336,7 +347,7 @@ __device__ __forceinline__ void dma_walk(const typename Tr::vec8 (&qv)[D / 32], 
     for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
       for (int pp = 0; pp < kStepPages; ++pp) {
-        const vec8 a = FP8 ? fp8x8_to<Tr>(kop[pp][ks][0], kop[pp][ks][1])
+        const vec8 a = FP8 ? fp8x8_to<Tr>(klo[pp][ks][0], klo[pp][ks][1])
                            : __builtin_bit_cast(vec8, kop[pp][ks]);
         s[pp] = Tr::mfma16(a, qv[ks], s[pp]);
       }
