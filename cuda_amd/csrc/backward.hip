@@ -13,12 +13,14 @@
 // Three launches and no atomics, so the result does not depend on timing:
 //   bwd_rowdot_kernel   the pair (LSE log2 e, D = rowsum(dO * O)) per query
 //                       row into a [B, Hq, S] x 2 fp32 workspace;
-//   bwd_dkv_dma_kernel  key-outer: 8 waves x 32 keys of one (b, kv head);
+//   bwd_dkv_dma_kernel  key-outer: 8 waves x 32 keys of one (b, kv head) (or
+//                       2 or 4 waves on the same 32 keys, bwd_split);
 //                       query tiles of 32 (Q, dO, pairs) stream through an
 //                       LDS ring, for every q head of the kv head; per tile
 //                       S = Q K^T, dP = dO V^T, dS, dV^T += dO^T P,
 //                       dK^T += Q^T dS;
-//   bwd_dq_dma_kernel   query-outer: 8 waves x 32 queries of one (b, h); key
+//   bwd_dq_dma_kernel   query-outer: 8 waves x 32 queries of one (b, h) (or 2
+//                       waves on the same 32); key
 //                       tiles of 64 (K, V) stream through an LDS ring; per
 //                       32 keys S^T = K Q^T, dP^T = V dO^T, dS^T,
 //                       dQ^T += K^T dS^T.
@@ -30,6 +32,8 @@
 // the next product's k-steps, so P and dS go from accumulators to operands
 // without leaving registers. The transposed operands (K^T, Q^T, dO^T) come
 // from row-major LDS tiles through ds_read_b64_tr_b16.
+#include <algorithm>
+
 #include "common.h"
 #include "launch.h"
 #include "lds_dma.h"
@@ -141,8 +145,13 @@ __device__ __forceinline__ void store_rowsT_lds(uint16_t* head, int row0, int n,
 // ---------------------------------------------------------------------------
 namespace bwdma {
 constexpr int kNW = 8;         // waves per workgroup
-constexpr int kStages = 4;     // ring tiles
+constexpr int kStages = 4;     // ring tiles of the dQ walk
 constexpr int kDist = kStages - 1;
+// ring stages of the dK/dV walk: what 160 KB of LDS hold beside the V rows
+template <int D, int KG>
+constexpr int dkv_stages() {
+  return D == 64 || KG == 8 ? 4 : KG == 4 ? 3 : 2;
+}
 struct TrOfs {
   uint32_t a, b;
 };
@@ -191,9 +200,44 @@ struct Geom {
 };
 }  // namespace bwdma
 
-// dQ of query tile qt (256 rows) of head bh: the keys [0, kv_end) in tiles of
-// 64, each computed as two halves of 32 keys.
-template <typename Tr, int D, bool CAUSAL>
+// Sums the accumulators of the QS waves that share rows (wave = part * NG +
+// row group) into part 0, through LDS at `lds` (NG * QS / 2 blocks of the
+// accumulators as they lie in registers); every wave calls it, with the ring
+// no longer in use.
+template <int NACC, int NG, int QS>
+__device__ __forceinline__ void reduce_parts(f32x16 (&acc)[NACC], unsigned char* lds, int part,
+                                             int group, int lane) {
+#pragma unroll
+  for (int half = QS / 2; half >= 1; half /= 2) {
+    __syncthreads();  // the ring, or the blocks of the step before, are no longer read
+    f32x4* blk = (f32x4*)lds + (size_t)((part % half) * NG + group) * (NACC * 4 * 64) + lane;
+    if (part >= half && part < 2 * half) {
+#pragma unroll
+      for (int i = 0; i < NACC; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          blk[64 * (4 * i + j)] = f32x4{acc[i][4 * j], acc[i][4 * j + 1], acc[i][4 * j + 2], acc[i][4 * j + 3]};
+    }
+    __syncthreads();
+    if (part < half) {
+#pragma unroll
+      for (int i = 0; i < NACC; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const f32x4 x = blk[64 * (4 * i + j)];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][4 * j + e] += x[e];
+        }
+    }
+  }
+  __syncthreads();
+}
+
+// dQ of query tile qt (32 QG rows) of head bh: the keys [0, kv_end) in tiles of
+// 64, each computed as two halves of 32 keys. QG = 8: a wave per 32 rows; QG =
+// 4: two waves share 32 rows, each taking one half of every tile, and add up
+// at the end.
+template <typename Tr, int D, bool CAUSAL, int QG>
 __device__ CA_INLINE void bwd_dq_dma_tile(const uint16_t* __restrict__ Q,
                                          const uint16_t* __restrict__ K,
                                          const uint16_t* __restrict__ V,
@@ -205,8 +249,10 @@ __device__ CA_INLINE void bwd_dq_dma_tile(const uint16_t* __restrict__ Q,
   using vec8 = typename Tr::vec8;
   using vec2 = typename Tr::vec2;
   constexpr int kRowB = Gm::kRowB, kNKS = Gm::kNKS, kNOB = Gm::kNOB;
-  constexpr int BM = 32 * kNW;
+  constexpr int BM = 32 * QG;
   constexpr int BN = 64;
+  constexpr int KS = kNW / QG;                 // waves per 32 rows
+  static_assert(KS == 1 || KS == 2, "a half of a key tile per wave");
   constexpr int kTileB = BN * kRowB;           // 16 KB (D = 128), 8 KB (D = 64)
   constexpr int kStageB = 2 * kTileB;          // K tile, then V tile
   constexpr int kDma = kTileB / 1024 / kNW;    // 1-KB loads per wave per K (and V) tile
@@ -223,8 +269,9 @@ __device__ CA_INLINE void bwd_dq_dma_tile(const uint16_t* __restrict__ Q,
   const uint16_t* Vp = V + (size_t)(b * Hkv + hk) * S * D;
   const int lane = __builtin_amdgcn_workitem_id_x() & 63;
   const int wave = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_workitem_id_x() >> 6);
+  const int qg = KS == 1 ? wave : wave % QG, part = KS == 1 ? 0 : wave / QG;
   const int l32 = lane & 31, hl = lane >> 5;
-  const int qw0 = q0 + 32 * wave;
+  const int qw0 = q0 + 32 * qg;
   const int myq = qw0 + l32;
   const bool qvalid = myq < S;
   const float c2 = scale * kLog2e;
@@ -360,17 +407,19 @@ __device__ CA_INLINE void bwd_dq_dma_tile(const uint16_t* __restrict__ Q,
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
       const int j = 2 * t + hh;
-      if (j < w_halves) {
+      if (j < w_halves && (KS == 1 || hh == part)) {
         half(sb + hh * 32 * kRowB, 32 * j, CAUSAL ? (j == w_halves - 1) : (32 * j + 32 > S));
       }
     }
   }
   wait_vmcnt<0>();  // no load may still target this workgroup's LDS when it exits
-  store_rowsT_lds<Tr, kNOB, 128>(dQ + qoff * D, qw0, S, acc, scale,
-                                 lds_off(qstg) + (uint32_t)(wave * 32 * 128), lane);
+  if constexpr (KS > 1) reduce_parts<kNOB, QG, KS>(acc, lds, part, qg, lane);
+  if (part == 0)
+    store_rowsT_lds<Tr, kNOB, 128>(dQ + qoff * D, qw0, S, acc, scale,
+                                   lds_off(qstg) + (uint32_t)(qg * 32 * 128), lane);
 }
 
-template <typename Tr, int D, bool CAUSAL>
+template <typename Tr, int D, bool CAUSAL, int QG>
 __global__ __launch_bounds__(64 * bwdma::kNW) void bwd_dq_dma_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ dO,
@@ -382,16 +431,18 @@ __global__ __launch_bounds__(64 * bwdma::kNW) void bwd_dq_dma_kernel(
 #pragma clang loop unroll(disable)
   for (int pass = 0; pass < n_pass; ++pass) {
     if (pass) __builtin_amdgcn_s_barrier();  // every wave is done reading the ring
-    bwd_dq_dma_tile<Tr, D, CAUSAL>(Q, K, V, dO, LD, dQ, S, Hq, Hkv, scale, pass ? wk.bh1 : wk.bh0,
+    bwd_dq_dma_tile<Tr, D, CAUSAL, QG>(Q, K, V, dO, LD, dQ, S, Hq, Hkv, scale, pass ? wk.bh1 : wk.bh0,
                                pass ? wk.qt1 : wk.qt0);
   }
 }
 
-// dK, dV of key tile kt (256 keys) of kv head bhk: every q head of the kv head,
+// dK, dV of key tile kt (32 KG keys) of kv head bhk: every q head of the kv head,
 // queries in tiles of 32 (from the tile holding the first key when causal).
-// K^T stays in registers; each wave keeps its own 32 V rows in LDS (the V^T B
-// operand of dP); Q, dO and the (LSE log2 e, D) pairs stream through the ring.
-template <typename Tr, int D, bool CAUSAL>
+// K^T stays in registers; the V rows sit in LDS (the V^T B operand of dP); Q,
+// dO and the (LSE log2 e, D) pairs stream through the ring. KG = 8: a wave
+// per 32 keys. KG = 4 or 2: QS = 8 / KG waves share 32 keys, each taking every
+// QS-th query tile, and add up at the end.
+template <typename Tr, int D, bool CAUSAL, int KG>
 __device__ CA_INLINE void bwd_dkv_dma_tile(const uint16_t* __restrict__ Q,
                                           const uint16_t* __restrict__ K,
                                           const uint16_t* __restrict__ V,
@@ -404,17 +455,24 @@ __device__ CA_INLINE void bwd_dkv_dma_tile(const uint16_t* __restrict__ Q,
   using vec8 = typename Tr::vec8;
   using vec2 = typename Tr::vec2;
   constexpr int kRowB = Gm::kRowB, kNKS = Gm::kNKS, kNOB = Gm::kNOB;
-  constexpr int BK = 32 * kNW;                  // keys per workgroup
-  constexpr int BQ = 32;                        // queries per ring tile
+  constexpr int QS = kNW / KG;                  // waves per 32 keys
+  constexpr int BK = 32 * KG;                   // keys per workgroup
+  constexpr int BQ = 32;                        // queries per tile
   constexpr int kTileB = BQ * kRowB;            // 8 KB (D = 128), 4 KB (D = 64)
-  constexpr int kStageB = 2 * kTileB + 1024;    // Q tile, dO tile, pairs
-  constexpr int kVB = 32 * kRowB;               // V rows of one wave
-  // D = 128: every wave loads 1 KB of the Q tile and 1 KB of the dO tile;
-  // D = 64: waves 0..3 load the Q tile, waves 4..7 the dO tile
-  constexpr bool kSplit = kTileB < 1024 * kNW;
-  static_assert(kTileB == 1024 * kNW || 2 * kTileB == 1024 * kNW, "whole 1-KB loads per wave");
-  constexpr int kLoads = kSplit ? 1 : 2;        // ring loads per wave per tile (+1: pairs, wave 0)
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[kNW * kVB + kStages * kStageB];
+  constexpr int kSubB = 2 * kTileB + 1024;      // Q tile, dO tile, pairs
+  constexpr int kStageB = QS * kSubB;           // a ring stage: one tile per part
+  constexpr int kVB = 32 * kRowB;               // V rows of one key group
+  // stages that LDS (160 KB) holds beside the V rows: 4, 3 or 2 (D = 128), 4 (D = 64)
+  constexpr int kStages = dkv_stages<D, KG>();
+  constexpr int kDist = kStages - 1;
+  // 1-KB loads of a stage, dealt to the waves in turn (load 8 j + wave):
+  // per tile kT of Q, then kT of dO
+  constexpr int kT = kTileB / 1024;
+  constexpr int kLoads = QS * 2 * kT / kNW;     // per wave per stage (+ QS pair loads, wave 0)
+  static_assert(kLoads * kNW == QS * 2 * kT, "whole loads per wave");
+  constexpr int kRedB = QS > 1 ? kNW / 2 * 2 * kNOB * 4096 : 0;  // reduce_parts
+  constexpr int kLdsB = KG * kVB + kStages * kStageB;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[kLdsB > kRedB ? kLdsB : kRedB];
 
   const int b = bhk / Hkv, hk = bhk % Hkv;
   const int G = Hq / Hkv;
@@ -426,14 +484,16 @@ __device__ CA_INLINE void bwd_dkv_dma_tile(const uint16_t* __restrict__ Q,
   // 256 VGPRs spills them (measured: 13-14 spilled registers at D = 128).
   const int lane = lane_here();
   const int wave = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_workitem_id_x() >> 6);
+  const int kg = QS == 1 ? wave : wave % KG, part = QS == 1 ? 0 : wave / KG;
   const int l32 = lane & 31, hl = lane >> 5;
-  const int kw0 = K0 + 32 * wave;
+  const int kw0 = K0 + 32 * kg;
   const int mykey = kw0 + l32;
   const bool kvalid = mykey < S;
   const float c2 = scale * kLog2e;
 
-  // this wave's V rows -> LDS (rows past S read as zero)
-  unsigned char* vw = lds + wave * kVB;
+  // the key group's V rows -> LDS (rows past S read as zero); its other parts
+  // write the same bytes, so a wave's own loads cover its reads
+  unsigned char* vw = lds + kg * kVB;
   {
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(V + kvoff * D, (uint32_t)S * kRowB);
 #pragma unroll
@@ -454,39 +514,55 @@ __device__ CA_INLINE void bwd_dkv_dma_tile(const uint16_t* __restrict__ Q,
 
   const int t_begin = CAUSAL ? K0 / BQ : 0;
   const int nt = max(0, (S + BQ - 1) / BQ - t_begin);  // query tiles per q head
-  const int n_it = G * nt;
-  // ring load of tile it: 1-KB loads of Q and dO (tile rows from kRpk wsub),
-  // the 64 floats of pairs by wave 0
-  const int wsub = kSplit ? (wave & (kNW / 2 - 1)) : wave;
-  const uint32_t dma_off = Gm::dma_ofs(Gm::kRpk * wsub, lane);
-  auto issue = [&](int it) CA_INLINE {
-    unsigned char* st = lds + kNW * kVB + (it % kStages) * kStageB;
-    // past the walk (slots the loop never reads): offsets past the slice, zeros
-    const bool past = it >= n_it;
-    const int itc = past ? 0 : it;
-    const int h = hk * G + itc / max(nt, 1);
-    const int q0 = past ? S : (t_begin + itc % max(nt, 1)) * BQ;
-    const size_t ho = (size_t)(b * Hq + h) * S;
-    const uint32_t qoff = (uint32_t)q0 * kRowB, sz = (uint32_t)S * kRowB;
-    if (!kSplit || wave < kNW / 2)
-      dma16_buf(make_rsrc_at(Q + ho * D, qoff, sz), (CA_LDS void*)(st + 1024 * wsub), dma_off);
-    if (!kSplit || wave >= kNW / 2)
-      dma16_buf(make_rsrc_at(dO + ho * D, qoff, sz), (CA_LDS void*)(st + kTileB + 1024 * wsub),
-                dma_off);
-    if (wave == 0)
-      dma4_buf(make_rsrc_at(LD + 2 * ho, (uint32_t)q0 * 8, (uint32_t)S * 8),
-               (CA_LDS void*)(st + 2 * kTileB), 4 * lane);
+  const int n_u = G * nt;                         // tiles of all q heads
+  const int n_it = (n_u + QS - 1) / QS;
+  // tile u of the walk: head hk G + u / nt, queries from BQ (t_begin + u % nt)
+  const int wsub = kT == kNW ? wave : wave % kT;
+  auto issue = [&](int it, int slot) CA_INLINE {
+    unsigned char* st = lds + KG * kVB + slot * kStageB;
+    // from the lane index as it stands here: one register less across the loop
+    const int ln = QS > 1 ? lane_here() : lane;
+    const uint32_t dma_off = Gm::dma_ofs(Gm::kRpk * wsub, ln);
+    auto tile_of = [&](int u, size_t& ho, int& q0) CA_INLINE {
+      // past the walk (slots the loop never reads): offsets past the slice, zeros
+      const bool past = u >= n_u;
+      const int uc = past ? 0 : u;
+      q0 = past ? S : (t_begin + uc % max(nt, 1)) * BQ;
+      ho = (size_t)(b * Hq + hk * G + uc / max(nt, 1)) * S;
+    };
+    const uint32_t sz = (uint32_t)S * kRowB;
+#pragma unroll
+    for (int sub = 0; sub < QS; ++sub) {
+      size_t ho;
+      int q0;
+      tile_of(it * QS + sub, ho, q0);
+      unsigned char* dst = st + sub * kSubB + 1024 * wsub;
+      if (kT == kNW) {
+        dma16_buf(make_rsrc_at(Q + ho * D, (uint32_t)q0 * kRowB, sz), (CA_LDS void*)dst, dma_off);
+        dma16_buf(make_rsrc_at(dO + ho * D, (uint32_t)q0 * kRowB, sz), (CA_LDS void*)(dst + kTileB),
+                  dma_off);
+      } else if (wave < kT) {
+        dma16_buf(make_rsrc_at(Q + ho * D, (uint32_t)q0 * kRowB, sz), (CA_LDS void*)dst, dma_off);
+      } else {
+        dma16_buf(make_rsrc_at(dO + ho * D, (uint32_t)q0 * kRowB, sz), (CA_LDS void*)(dst + kTileB),
+                  dma_off);
+      }
+      if (wave == 0)
+        dma4_buf(make_rsrc_at(LD + 2 * ho, (uint32_t)q0 * 8, (uint32_t)S * 8),
+                 (CA_LDS void*)(st + sub * kSubB + 2 * kTileB), 4 * ln);
+    }
   };
   const uint32_t lds0 = lds_off(lds);
   const uint32_t rofs = Gm::row_ofs(rho32(l32), hl);  // Q / dO rows (A operands)
-  const uint32_t vofs = lds0 + wave * kVB + Gm::row_ofs(l32, hl);  // V rows (B operand)
+  const uint32_t vofs = lds0 + kg * kVB + Gm::row_ofs(l32, hl);  // V rows (B operand)
   const TrOfs tofs = Gm::tr_ofs(lane);
 
-  f32x16 dk[kNOB], dv[kNOB];  // dK^T, dV^T: rows d = 32 ob + .., column = this lane's key
+  // dK^T (acc[ob]) and dV^T (acc[kNOB + ob]): rows d = 32 ob + .., column = this lane's key
+  f32x16 acc[2 * kNOB];
 #pragma unroll
-  for (int i = 0; i < kNOB; ++i)
+  for (int i = 0; i < 2 * kNOB; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) { dk[i][r] = 0.f; dv[i][r] = 0.f; }
+    for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
 
   // One query tile at LDS byte `sb`; only the softmax step differs between
   // masked and unmasked tiles (a branch around the whole tile doubles the
@@ -574,34 +650,44 @@ __device__ CA_INLINE void bwd_dkv_dma_tile(const uint16_t* __restrict__ Q,
       after_wait(a1);
       after_wait(b0);
       after_wait(b1);
-      dv[ob] = Tr::mfma32(a0, pp[0], dv[ob]);
-      dk[ob] = Tr::mfma32(b0, pd[0], dk[ob]);
-      dv[ob] = Tr::mfma32(a1, pp[1], dv[ob]);
-      dk[ob] = Tr::mfma32(b1, pd[1], dk[ob]);
+      acc[kNOB + ob] = Tr::mfma32(a0, pp[0], acc[kNOB + ob]);
+      acc[ob] = Tr::mfma32(b0, pd[0], acc[ob]);
+      acc[kNOB + ob] = Tr::mfma32(a1, pp[1], acc[kNOB + ob]);
+      acc[ob] = Tr::mfma32(b1, pd[1], acc[ob]);
     }
   };
 
 #pragma unroll
-  for (int i = 0; i < kDist; ++i) issue(i);
+  for (int i = 0; i < kDist; ++i) issue(i, i);
+  constexpr bool kPow2 = (kStages & (kStages - 1)) == 0;
+  int slot = 0;  // it % kStages
   for (int it = 0; it < n_it; ++it) {
-    // this wave's loads of tile it (and its V rows, issued first) landed
-    if (wave == 0) wait_vmcnt<(kLoads + 1) * (kDist - 1)>();
+    if (kPow2) slot = it % kStages;
+    // this wave's loads of stage it (and its V rows, issued first) landed
+    if (wave == 0) wait_vmcnt<(kLoads + QS) * (kDist - 1)>();
     else wait_vmcnt<kLoads * (kDist - 1)>();
     __builtin_amdgcn_s_barrier();  // ... and every wave's; slot of it-1 is free
-    issue(it + kDist);
-    const int q0 = (t_begin + it % nt) * BQ;
-    if (kw0 < S && (!CAUSAL || q0 >= kw0)) {  // causal: queries before every key of the wave
-      const uint32_t sb = lds0 + kNW * kVB + (uint32_t)((it % kStages) * kStageB);
+    issue(it + kDist, kPow2 ? (it + kDist) % kStages : slot == 0 ? kStages - 1 : slot - 1);
+    const int u = it * QS + part;
+    const int q0 = (t_begin + u % nt) * BQ;
+    if ((QS == 1 || u < n_u) && kw0 < S && (!CAUSAL || q0 >= kw0)) {  // causal: queries before every key of the wave
+      const uint32_t sb = lds0 + KG * kVB + (uint32_t)(slot * kStageB + part * kSubB);
       tile(sb, q0, (CAUSAL && q0 == kw0) || q0 + BQ > S);
     }
+    if (!kPow2) slot = slot == kStages - 1 ? 0 : slot + 1;
   }
   wait_vmcnt<0>();  // no load may still target this workgroup's LDS when it exits
-  // the wave's V rows are no longer read: their LDS block stages dK, then dV
-  store_rowsT_lds<Tr, kNOB, kRowB>(dK + kvoff * D, kw0, S, dk, scale, lds_off(vw), lane_here());
-  store_rowsT_lds<Tr, kNOB, kRowB>(dV + kvoff * D, kw0, S, dv, 1.f, lds_off(vw), lane_here());
+  if constexpr (QS > 1) reduce_parts<2 * kNOB, KG, QS>(acc, lds, part, kg, lane_here());
+  // the key group's V rows are no longer read: their LDS block stages dK, then dV
+  if (part == 0) {
+    store_rowsT_lds<Tr, kNOB, kRowB>(dK + kvoff * D, kw0, S, *(const f32x16(*)[kNOB])(acc), scale,
+                                     lds_off(vw), lane_here());
+    store_rowsT_lds<Tr, kNOB, kRowB>(dV + kvoff * D, kw0, S, *(const f32x16(*)[kNOB])(acc + kNOB), 1.f,
+                                     lds_off(vw), lane_here());
+  }
 }
 
-template <typename Tr, int D, bool CAUSAL>
+template <typename Tr, int D, bool CAUSAL, int KG>
 __global__ __launch_bounds__(64 * bwdma::kNW) void bwd_dkv_dma_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ dO,
@@ -615,9 +701,48 @@ __global__ __launch_bounds__(64 * bwdma::kNW) void bwd_dkv_dma_kernel(
 #pragma clang loop unroll(disable)
   for (int pass = 0; pass < n_pass; ++pass) {
     if (pass) __builtin_amdgcn_s_barrier();  // every wave is done reading the ring and V
-    bwd_dkv_dma_tile<Tr, D, CAUSAL>(Q, K, V, dO, LD, dK, dV, S, Hq, Hkv, scale,
+    bwd_dkv_dma_tile<Tr, D, CAUSAL, KG>(Q, K, V, dO, LD, dK, dV, S, Hq, Hkv, scale,
                                 pass ? wk.bh1 : wk.bh0, n_kt - 1 - (pass ? wk.qt1 : wk.qt0));
   }
+}
+
+// Row groups (of 32) per workgroup of a backward launch over `heads` heads per
+// batch, with its tiles and grid: 8, or 4 or 2 where that shortens the busiest
+// CU's work by a fifth or more. The work is the walk lengths in tiles times the
+// work of a tile (groups^2), with what a split costs in percent (cost4, cost2;
+// 0: not built): the same waves fetch Q and dO (K and V) for fewer rows and
+// add up at the end, measured at a full grid (4 x 32 heads of 4096) as +9 % for
+// 4 groups and +42 % for 2 of dK/dV at head dim 128, +22 % and +68 % at 64; dQ
+// +10 % for 4.
+// Below a full grid the walks rule: 2 x 8 kv heads of 4096 keys, four q heads
+// each, are 256 unpaired walks of very different lengths with 8 groups and 256
+// equal pairs with 4 (dK/dV 827 -> 605 us); 8 kv heads of 1000, forward and dQ
+// aside, are 32 workgroups with 8 groups and 128 with 2 (backward 243 -> 114 us).
+struct BwdSplit {
+  int groups, n_tiles, paired;
+  long long grid;
+};
+BwdSplit bwd_split(int B, int heads, int S, bool causal, int cost4, int cost2) {
+  const long long cus = std::max(device_cus(), 1);
+  BwdSplit best{};
+  long long best_cost = 0;
+  for (int groups = 8; groups >= (cost2 ? 2 : 4); groups /= 2) {
+    BwdSplit s{};
+    s.groups = groups;
+    s.n_tiles = (S + 32 * groups - 1) / (32 * groups);
+    s.grid = prefill_grid(B, heads, s.n_tiles, causal, 1, &s.paired);
+    // walk lengths in tiles of the busiest CU, times the work of a tile
+    const long long tiles = (long long)B * heads * s.n_tiles;
+    const long long walks = causal ? (s.paired ? (s.grid + cus - 1) / cus * (s.n_tiles + 1)
+                                               : std::max<long long>(s.n_tiles, tiles * (s.n_tiles + 1) / 2 / cus))
+                                   : (tiles + cus - 1) / cus * s.n_tiles;
+    const long long cost = walks * groups * groups * (groups == 8 ? 100 : groups == 4 ? cost4 : cost2);
+    if (groups == 8 || cost * 10 < best_cost * 8) {
+      best = s;
+      best_cost = cost;
+    }
+  }
+  return best;
 }
 
 template <typename Tr, int D, bool CAUSAL>
@@ -628,27 +753,27 @@ hipError_t launch_bwd_t(const void* q, const void* k, const void* v, const void*
   const long long threads = rows * (D / 8);
   const long long g0 = (threads + 255) / 256;
   if (g0 > 0x7fffffffLL) return hipErrorInvalidValue;
-  // 256 keys (dK, dV) / 256 queries (dQ) per workgroup, one workgroup per CU
-  constexpr int BT = 32 * bwdma::kNW;
-  const int n_t = (S + BT - 1) / BT;
-  int pk = 0, pq = 0;
-  const long long gk = prefill_grid(B, Hkv, n_t, CAUSAL, 1, &pk);
-  const long long gq = prefill_grid(B, Hq, n_t, CAUSAL, 1, &pq);
-  if (gk > 0x7fffffffLL || gq > 0x7fffffffLL) return hipErrorInvalidValue;
+  const BwdSplit sk = bwd_split(B, Hkv, S, CAUSAL, D == 64 ? 122 : 109, D == 64 ? 168 : 142);
+  const BwdSplit sq = bwd_split(B, Hq, S, CAUSAL, 110, 0);
+  if (sk.grid > 0x7fffffffLL || sq.grid > 0x7fffffffLL) return hipErrorInvalidValue;
   hipLaunchKernelGGL((bwd_rowdot_kernel<Tr, D>), dim3((unsigned)g0), dim3(256), 0, stream,
                      (const uint16_t*)o, (const uint16_t*)dout, lse, ws, rows);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((bwd_dkv_dma_kernel<Tr, D, CAUSAL>), dim3((unsigned)gk), dim3(64 * bwdma::kNW),
-                     0, stream, (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,
-                     (const uint16_t*)dout, ws, (uint16_t*)dk, (uint16_t*)dv, S, Hq, Hkv, scale,
-                     n_t, B * Hkv, (int)gk, pk);
+  const dim3 block(64 * bwdma::kNW);
+  const auto dkv = sk.groups == 8   ? &bwd_dkv_dma_kernel<Tr, D, CAUSAL, 8>
+                   : sk.groups == 4 ? &bwd_dkv_dma_kernel<Tr, D, CAUSAL, 4>
+                                    : &bwd_dkv_dma_kernel<Tr, D, CAUSAL, 2>;
+  hipLaunchKernelGGL(dkv, dim3((unsigned)sk.grid), block, 0, stream, (const uint16_t*)q,
+                     (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)dout, ws, (uint16_t*)dk,
+                     (uint16_t*)dv, S, Hq, Hkv, scale, sk.n_tiles, B * Hkv, (int)sk.grid, sk.paired);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((bwd_dq_dma_kernel<Tr, D, CAUSAL>), dim3((unsigned)gq), dim3(64 * bwdma::kNW),
-                     0, stream, (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,
-                     (const uint16_t*)dout, ws, (uint16_t*)dq, S, Hq, Hkv, scale, n_t, B * Hq,
-                     (int)gq, pq);
+  const auto dqk = sq.groups == 8 ? &bwd_dq_dma_kernel<Tr, D, CAUSAL, 8>
+                                  : &bwd_dq_dma_kernel<Tr, D, CAUSAL, 4>;
+  hipLaunchKernelGGL(dqk, dim3((unsigned)sq.grid), block, 0, stream, (const uint16_t*)q,
+                     (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)dout, ws, (uint16_t*)dq,
+                     S, Hq, Hkv, scale, sq.n_tiles, B * Hq, (int)sq.grid, sq.paired);
   return hipGetLastError();
 }
 

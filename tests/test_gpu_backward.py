@@ -268,6 +268,31 @@ def test_backward_large_paired_tiles(dev, b, h, s, is_causal, d):
             _check_grad(a[bi:bi + 1, hi:hi + 1], r, f"{name} b{bi} h{hi}")
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("b,hq,hkv,s,is_causal", [(2, 32, 32, 1000, True), (1, 40, 20, 1500, False),
+                                                  (1, 6, 2, 33, True), (1, 6, 2, 65, False)])
+def test_backward_shared_rows(dev, b, hq, hkv, s, is_causal, d):
+    """Workgroups whose waves share rows: two waves per 32 keys or queries
+    (the first two shapes, pairs of tiles and single ones, ragged ends), four
+    per 32 keys (the last two: as many query tiles as waves, one more, fewer)."""
+    g = torch.Generator(device=dev).manual_seed(s)
+    q, k, v = qkv(b, hq, s, d, torch.bfloat16, dev, hkv=hkv, gen=g)
+    dout = torch.randn(b, hq, s, d, device=dev, generator=g).to(torch.bfloat16)
+    out, lse = cuda_llm.flash_attention_forward_lse(q, k, v, is_causal=is_causal)
+    dq, dk, dv = cuda_llm.flash_attention_backward(dout, q, k, v, out, lse, is_causal=is_causal)
+    torch.cuda.synchronize()
+    ratio = hq // hkv
+    for bi, h in ((0, 0), (b - 1, hkv - 1)):
+        qs = slice(h * ratio, (h + 1) * ratio)
+        sub = [to_np(t[bi:bi + 1, x]).astype(np.float64)
+               for t, x in ((dout, qs), (q, qs), (k, slice(h, h + 1)), (v, slice(h, h + 1)),
+                            (out, qs), (lse, qs))]
+        ref = oracle.attention_backward(*sub, is_causal=is_causal, dtype=np.float64)
+        for name, a, r in zip(("dq", "dk", "dv"), (dq[bi:bi + 1, qs], dk[bi:bi + 1, h:h + 1],
+                                                   dv[bi:bi + 1, h:h + 1]), ref):
+            _check_grad(a, r, f"{name} of head {h}")
+
+
 def test_backward_reference_benchmark_shape(dev):
     """The reference benchmark's backward shape (benchmark_pytorch.py:659-661:
     fp16, B = 2, H = 32, S = 4096, head dim 64, non-causal): every head is
