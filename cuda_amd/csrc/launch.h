@@ -17,22 +17,14 @@ constexpr int kDtypeF32 = 0;
 constexpr int kDtypeF16 = 1;
 constexpr int kDtypeBF16 = 2;
 
-// RoPE tables (fp32 [S, D], rotate-half) applied to Q as the 16-bit prefill
-// kernels load it; null: no rotation.
-struct RopeQ {
-  const float* cos = nullptr;
-  const float* sin = nullptr;
-};
-
 // Prefill; lse (may be null) receives the natural-log row logsumexp [B, Hq, S].
-// rq (16-bit dtypes only) rotates q on load.
+// q may be o itself (16-bit: every row is read as Q before it is written).
 hipError_t launch_prefill(int dtype, const void* q, const void* k, const void* v, void* o,
                           float* lse, int B, int Hq, int Hkv, int S, int D, float scale,
-                          bool causal, hipStream_t stream, RopeQ rq = RopeQ{});
+                          bool causal, hipStream_t stream);
 // 64-row-per-wave prefill (prefill_w64.hip): bf16 or fp16 (f16), head dim
-// 128, softmax scale >= 0, no RoPE; launch_prefill dispatches to it when
-// supported.
-bool prefill_w64_supported(int D, int S, float scale, bool rope);
+// 128, softmax scale >= 0; launch_prefill dispatches to it when supported.
+bool prefill_w64_supported(int D, int S, float scale);
 hipError_t launch_prefill_w64(bool f16, const void* q, const void* k, const void* v, void* o, float* lse, int B,
                               int Hq, int Hkv, int S, float scale, bool causal, hipStream_t stream);
 void magic_div(uint32_t d, uint32_t* m, uint32_t* sh);

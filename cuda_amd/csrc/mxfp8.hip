@@ -170,7 +170,7 @@ hipError_t launch_mxfp8(int out_dtype, int scale_kind, const uint8_t* q, const v
   const long long rows = (long long)B * H * S;
   if (rows == 0) return hipSuccess;
   // the attention kernel's limits (checked before the prepare launch)
-  if (!prefill_w64_supported(128, S, scale < 0.f ? -scale : scale, false) || rows >= (1LL << 30))
+  if (!prefill_w64_supported(128, S, scale < 0.f ? -scale : scale) || rows >= (1LL << 30))
     return hipErrorInvalidValue;
   if (ws_bytes < mx_workspace_bytes(scale_kind, B, H, S, D)) return hipErrorInvalidValue;
   unsigned char* w = (unsigned char*)ws;

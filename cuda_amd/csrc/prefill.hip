@@ -40,41 +40,6 @@
 
 namespace ca {
 
-// Rotate-half RoPE of the Q operand of query row `pos` in registers (the
-// rotation of rope.hip, fused_rope_flash_attention_kernel.cuh:60-70): qv[ks]
-// holds dims 16 ks + 8 hl + e, so dim c < D/2 and its partner c + D/2 sit in
-// k-steps ks and ks + D/32 of the same lane.
-template <typename Tr, int D>
-__device__ __forceinline__ void rope_q(typename Tr::vec8 (&qv)[D / 16], RopeQ rq, int pos, int hl) {
-  using vec2 = typename Tr::vec2;
-  constexpr int H = D / 2, HKS = D / 32;
-  const float* cr = rq.cos + (size_t)pos * D;
-  const float* sr = rq.sin + (size_t)pos * D;
-#pragma unroll
-  for (int ks = 0; ks < HKS; ++ks) {
-    const int c = 16 * ks + 8 * hl;
-    float ca[8], sa[8], cb[8], sb[8];
-#pragma unroll
-    for (int h4 = 0; h4 < 8; h4 += 4) {
-      *(float4*)(ca + h4) = *(const float4*)(cr + c + h4);
-      *(float4*)(sa + h4) = *(const float4*)(sr + c + h4);
-      *(float4*)(cb + h4) = *(const float4*)(cr + c + H + h4);
-      *(float4*)(sb + h4) = *(const float4*)(sr + c + H + h4);
-    }
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-      const float a0 = (float)qv[ks][e], a1 = (float)qv[ks][e + 1];
-      const float b0 = (float)qv[ks + HKS][e], b1 = (float)qv[ks + HKS][e + 1];
-      const vec2 lo = Tr::pack2(a0 * ca[e] - b0 * sa[e], a1 * ca[e + 1] - b1 * sa[e + 1]);
-      const vec2 hi = Tr::pack2(b0 * cb[e] + a0 * sb[e], b1 * cb[e + 1] + a1 * sb[e + 1]);
-      qv[ks][e] = lo[0];
-      qv[ks][e + 1] = lo[1];
-      qv[ks + HKS][e] = hi[0];
-      qv[ks + HKS][e + 1] = hi[1];
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Head dim 64 and 128 kernel.
 //
@@ -155,10 +120,10 @@ struct PfItem {
 // the next item.
 //
 template <typename Tr, int D, bool CAUSAL, bool POS>
-__device__ CA_INLINE bool prefill_dma_qtile(const void* __restrict__ Qv, const void* __restrict__ Kv,
-                                            const uint16_t* __restrict__ V, void* __restrict__ Ov,
+__device__ CA_INLINE bool prefill_dma_qtile(const void* Qv, const void* __restrict__ Kv,
+                                            const uint16_t* __restrict__ V, void* Ov,
                                             float* __restrict__ Lse, int S, int Hq, int Hkv, float scale_log2,
-                                            int bh, int qt, int q_shift, RopeQ rq, PfItem nx, bool pre,
+                                            int bh, int qt, int q_shift, PfItem nx, bool pre,
                                             int& g0, typename Tr::vec8 (&qv)[D / 16]) {
   using Gv = PfGeom<D>;                   // K and V tile geometry
   using Gk = Gv;
@@ -220,7 +185,7 @@ __device__ CA_INLINE bool prefill_dma_qtile(const void* __restrict__ Qv, const v
 #pragma unroll
     for (int ks = 0; ks < Gv::kNKS; ++ks) qv[ks] = *(const vec8*)(Qr + 16 * ks + 8 * hl);
   };
-  // ... then zeroed outside [0, S) and rotated (RoPE).
+  // ... then zeroed outside [0, S).
   auto fix_q = [&]() CA_INLINE {
     if (!q_in) {
 #pragma unroll
@@ -228,7 +193,6 @@ __device__ CA_INLINE bool prefill_dma_qtile(const void* __restrict__ Qv, const v
 #pragma unroll
         for (int e = 0; e < 8; ++e) qv[ks][e] = 0;
     }
-    if (rq.cos && q_in) rope_q<Tr, D>(qv, rq, myq, hl);
   };
 
   const int kv_end = CAUSAL ? min(S, q0 + kBM) : S;
@@ -790,7 +754,7 @@ struct PfArgs {
 template <typename Tr, int D, bool CAUSAL, bool POS>
 __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_dma_kernel(
     PfArgs a, int S, int Hq, int Hkv, float scale_log2, int n_qt, int n_bh, int n_work, int paired,
-    int q_shift, RopeQ rq) {
+    int q_shift) {
   // Work items v = blockIdx.x, + gridDim.x, ... (a persistent launch when the
   // grid is smaller than n_work; gridDim.x is then a multiple of 8, so every
   // item keeps the XCD that xcd_remap gives it). A paired item is two query
@@ -822,7 +786,7 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_dma_kernel(
     const PfItem nx{__builtin_amdgcn_readfirstlane(nx0.bh), __builtin_amdgcn_readfirstlane(nx0.qt)};
     g0 = __builtin_amdgcn_readfirstlane(g0);
     pre = prefill_dma_qtile<Tr, D, CAUSAL, POS>(a.q, a.k, a.v, a.o, a.lse, S, Hq, Hkv, scale_log2, bh, qt,
-                                                 q_shift, rq, nx, pre, g0, qv);
+                                                 q_shift, nx, pre, g0, qv);
     if (nx.qt < 0) break;
     // a drained ring is refilled by the next tile: every wave must be done reading it
     if (!pre) __builtin_amdgcn_s_barrier();
@@ -835,7 +799,7 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_dma_kernel(
 // Grid, ragged-S shift and launch of the prefill kernel.
 template <typename Tr, int D, bool CAUSAL>
 static hipError_t launch_prefill_kernel(const PfArgs& a, int B, int Hq, int Hkv, int S, float scale,
-                                        hipStream_t stream, RopeQ rq) {
+                                        hipStream_t stream) {
   using Gm = PfGeom<D>;
   const int n_qt = (S + kPfRows - 1) / kPfRows;
   // the padding rows of a ragged S go before row 0, in whole key tiles (so a
@@ -858,11 +822,11 @@ static hipError_t launch_prefill_kernel(const PfArgs& a, int B, int Hq, int Hkv,
   if (sl2 >= 0.f) {
     hipLaunchKernelGGL((prefill_dma_kernel<Tr, D, CAUSAL, true>), dim3((unsigned)grid),
                        block, 0, stream, a, S, Hq, Hkv, sl2, n_qt, B * Hq, (int)n_work, paired,
-                       q_shift, rq);
+                       q_shift);
   } else {
     hipLaunchKernelGGL((prefill_dma_kernel<Tr, D, CAUSAL, false>), dim3((unsigned)grid),
                        block, 0, stream, a, S, Hq, Hkv, sl2, n_qt, B * Hq, (int)n_work, paired,
-                       q_shift, rq);
+                       q_shift);
   }
   return hipGetLastError();
 }
@@ -870,22 +834,22 @@ static hipError_t launch_prefill_kernel(const PfArgs& a, int B, int Hq, int Hkv,
 template <typename Tr, int D, bool CAUSAL>
 static hipError_t launch_prefill_dma(const void* q, const void* k, const void* v, void* o, float* lse,
                                      int B, int Hq, int Hkv, int S, float scale,
-                                     hipStream_t stream, RopeQ rq) {
+                                     hipStream_t stream) {
   const PfArgs a{q, k, (const uint16_t*)v, o, lse};
-  return launch_prefill_kernel<Tr, D, CAUSAL>(a, B, Hq, Hkv, S, scale, stream, rq);
+  return launch_prefill_kernel<Tr, D, CAUSAL>(a, B, Hq, Hkv, S, scale, stream);
 }
 
 
 hipError_t launch_prefill(int dtype, const void* q, const void* k, const void* v, void* o, float* lse,
                           int B, int Hq, int Hkv, int S, int D, float scale, bool causal,
-                          hipStream_t stream, RopeQ rq) {
+                          hipStream_t stream) {
 #define CA_PREFILL_DMA(TR, DD)                                                                    \
   if (D == DD) {                                                                                  \
-    return causal ? launch_prefill_dma<TR, DD, true>(q, k, v, o, lse, B, Hq, Hkv, S, scale, stream, rq)  \
-                  : launch_prefill_dma<TR, DD, false>(q, k, v, o, lse, B, Hq, Hkv, S, scale, stream, rq); \
+    return causal ? launch_prefill_dma<TR, DD, true>(q, k, v, o, lse, B, Hq, Hkv, S, scale, stream)  \
+                  : launch_prefill_dma<TR, DD, false>(q, k, v, o, lse, B, Hq, Hkv, S, scale, stream); \
   }
   if (dtype == kDtypeF32) return launch_prefill_f32(q, k, v, o, lse, B, Hq, Hkv, S, D, scale, causal, stream);
-  if ((dtype == kDtypeBF16 || dtype == kDtypeF16) && prefill_w64_supported(D, S, scale, rq.cos != nullptr))
+  if ((dtype == kDtypeBF16 || dtype == kDtypeF16) && prefill_w64_supported(D, S, scale))
     return launch_prefill_w64(dtype == kDtypeF16, q, k, v, o, lse, B, Hq, Hkv, S, scale, causal, stream);
   if (dtype == kDtypeBF16) {
     CA_PREFILL_DMA(BF16, 64)

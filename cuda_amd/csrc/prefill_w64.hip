@@ -143,10 +143,10 @@ void magic_div(uint32_t d, uint32_t* m, uint32_t* sh) {
   *sh = 31 + s;
 }
 
-bool prefill_w64_supported(int D, int S, float scale, bool rope) {
+bool prefill_w64_supported(int D, int S, float scale) {
   const float sl2 = scale * kLog2e;
   // S * 256 bytes per head must fit the 31-bit buffer offsets
-  return D == 128 && !rope && sl2 >= 0.f && sl2 <= 3.0e38f && S > 0 && S < (1 << 22);
+  return D == 128 && sl2 >= 0.f && sl2 <= 3.0e38f && S > 0 && S < (1 << 22);
 }
 
 hipError_t w64_geometry(int B, int Hq, int S, bool causal, PfW64Geom* g) {

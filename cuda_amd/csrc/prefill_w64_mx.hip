@@ -126,7 +126,7 @@ hipError_t launch_prefill_w64_mx(bool out_f16, const uint8_t* q, const uint8_t* 
   const bool neg = scale < 0.f;
   if (neg) scale = -scale;
   // the Q scale words are read at 32-bit offsets from qs
-  if (!prefill_w64_supported(128, S, scale, false) || (long long)B * H * S * 4 > 0xffffffffLL)
+  if (!prefill_w64_supported(128, S, scale) || (long long)B * H * S * 4 > 0xffffffffLL)
     return hipErrorInvalidValue;
   PfW64Geom g;
   const hipError_t ge = w64_geometry(B, H, S, causal, &g);
