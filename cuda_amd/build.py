@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libcuda_llm_amd.so")
-SOURCES = ["prefill.hip", "prefill_w64.hip", "prefill_w64_mx.hip", "decode.hip", "mxfp8.hip", "f32.hip", "backward.hip", "backward_f32.hip",
+SOURCES = ["prefill.hip", "prefill_rows.hip", "prefill_w64.hip", "prefill_w64_mx.hip", "decode.hip", "mxfp8.hip", "f32.hip", "backward.hip", "backward_f32.hip",
            "kv_append.hip", "rope.hip", "stream_read.hip", "abi.cpp"]
 ARCH = os.environ.get("CA_OFFLOAD_ARCH", "gfx950")
 
@@ -29,7 +29,7 @@ COMMON = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-result",
 ]
-# Per-source additions. prefill: the softmax row max runs on v_max/v_max3;
+# Per-source additions. prefill, prefill_rows: the softmax row max runs on v_max/v_max3;
 # with the IEEE mode bit on, every fmaxf operand that does not come from an
 # arithmetic instruction (MFMA results do not count) is first quieted with an
 # extra v_max. The kernels there have no NaN-dependent logic.
@@ -44,6 +44,7 @@ COMMON = [
 # TFLOP/s (two A/B runs); it made the 32-row forward at head dim 64 2-3 %
 # slower, so it stays on the backward only.
 EXTRA = {"prefill.hip": ["-mno-amdgpu-ieee", "-fno-honor-nans"],
+         "prefill_rows.hip": ["-mno-amdgpu-ieee", "-fno-honor-nans"],
          "f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
          "decode.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
          "backward.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]}

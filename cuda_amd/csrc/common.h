@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace ca {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -174,6 +176,15 @@ __device__ __forceinline__ f16x2 e4m3x2_to_f16(uint32_t w) {
 template <bool HI>
 __device__ __forceinline__ bf16x2 e4m3x2_to_bf16_scaled(uint32_t w, float s) {
   return __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, s, HI);
+}
+
+// f(integral constant 0 .. N - 1): loops whose index is an instruction's immediate
+template <int N, typename F, int I = 0>
+__device__ __forceinline__ void for_const(F& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    for_const<N, F, I + 1>(f);
+  }
 }
 
 template <typename V8, typename V4>

@@ -36,7 +36,6 @@
 #include <climits>
 #include <functional>
 #include <mutex>
-#include <type_traits>
 
 #include "common.h"
 #include "launch.h"
@@ -116,15 +115,6 @@ struct DmaCfg {
 };
 constexpr int kDmaPolicy = 2;  // global_load_lds cache policy bits: nt
 constexpr int kStepPages = 2;  // pages per step of a wave
-
-// f(integral constant 0 .. N - 1): loops whose index is an instruction's immediate
-template <int N, typename F, int I = 0>
-__device__ __forceinline__ void for_const(F& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    for_const<N, F, I + 1>(f);
-  }
-}
 
 // The wave's GQA group of query rows (Gc <= 16 heads from `qrow`, D each) as
 // the B operand of S^T = K^T Q^T: lane (head l16, group grp) holds d = 32 ks

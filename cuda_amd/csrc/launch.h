@@ -27,6 +27,12 @@ hipError_t launch_prefill(int dtype, const void* q, const void* k, const void* v
 bool prefill_w64_supported(int D, int S, float scale);
 hipError_t launch_prefill_w64(bool f16, const void* q, const void* k, const void* v, void* o, float* lse, int B,
                               int Hq, int Hkv, int S, float scale, bool causal, hipStream_t stream);
+// Prefill with waves sharing rows (prefill_rows.hip; 16-bit): the row groups of
+// 32 per workgroup that suit a launch (2 or 4), or 0 where the 256-row kernels do.
+int prefill_rows_groups(int B, int Hq, int S, int D, float scale, bool causal);
+hipError_t launch_prefill_rows(int groups, bool f16, const void* q, const void* k, const void* v,
+                               void* o, float* lse, int B, int Hq, int Hkv, int S, int D,
+                               float scale, bool causal, hipStream_t stream);
 void magic_div(uint32_t d, uint32_t* m, uint32_t* sh);
 // Work decomposition of the 64-row kernels (grid 0: nothing to launch).
 struct PfW64Geom {

@@ -37,6 +37,7 @@
 #include "common.h"
 #include "launch.h"
 #include "lds_dma.h"
+#include "prefill_common.h"
 
 namespace ca {
 
@@ -59,22 +60,6 @@ namespace ca {
 // among 16 consecutive rows 8 distinct chunks, and rows r, r+2 opposite
 // 4-chunk halves.
 // ---------------------------------------------------------------------------
-template <int D>
-struct PfGeom {
-  static_assert(D == 64 || D == 128, "head dim");
-  static constexpr int kBN = 64;                     // keys per tile
-  static constexpr int kRowB = D * 2;                // bytes per K/V row
-  static constexpr int kLpr = kRowB / 16;            // 16-byte chunks per row
-  static constexpr int kRpk = 1024 / kRowB;          // rows per 1-KB load
-  static constexpr int kTileB = kBN * kRowB;         // bytes per K (or V) tile
-  static constexpr int kStageB = 2 * kTileB;         // K tile then V tile
-  static constexpr int kNKS = D / 16;                // QK k-steps
-  static constexpr int kNOB = D / 32;                // O^T row blocks
-  __device__ static __forceinline__ int swz(int r) {
-    return D == 128 ? (((r & 3) << 2) | ((r >> 2) & 3)) : ((((r >> 1) & 1) << 2) | ((r >> 2) & 3));
-  }
-};
-
 constexpr int kPfRows = 256;   // query rows per workgroup
 constexpr int kPfWaves = 8;    // waves per workgroup (32 query rows each)
 constexpr int kPfStages = 4;   // K/V tiles in the LDS ring (32 KB each at D = 128; D = 64: 8)
@@ -849,6 +834,9 @@ hipError_t launch_prefill(int dtype, const void* q, const void* k, const void* v
                   : launch_prefill_dma<TR, DD, false>(q, k, v, o, lse, B, Hq, Hkv, S, scale, stream); \
   }
   if (dtype == kDtypeF32) return launch_prefill_f32(q, k, v, o, lse, B, Hq, Hkv, S, D, scale, causal, stream);
+  if (const int groups = prefill_rows_groups(B, Hq, S, D, scale, causal); groups > 0)
+    return launch_prefill_rows(groups, dtype == kDtypeF16, q, k, v, o, lse, B, Hq, Hkv, S, D, scale,
+                               causal, stream);
   if ((dtype == kDtypeBF16 || dtype == kDtypeF16) && prefill_w64_supported(D, S, scale))
     return launch_prefill_w64(dtype == kDtypeF16, q, k, v, o, lse, B, Hq, Hkv, S, scale, causal, stream);
   if (dtype == kDtypeBF16) {

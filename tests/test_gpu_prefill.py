@@ -321,3 +321,56 @@ def test_w64_long_sequences(dev, dtype, s, causal):
     assert torch.isfinite(out).all()
     ref = oracle.attention(to_np(q[:, 1:]), to_np(k[:, 1:]), to_np(v[:, 1:]), is_causal=causal)
     assert_close(to_np(out[:, 1:]), ref, **TOL_16BIT, name=f"{dtype} S={s} causal={causal}")
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("is_causal", [False, True])
+@pytest.mark.parametrize("b,hq,hkv,s", [(1, 3, 1, 1), (1, 3, 1, 31), (1, 3, 1, 33), (1, 3, 1, 65), (1, 4, 4, 127),
+                                        (1, 4, 4, 129), (1, 4, 2, 257), (1, 8, 8, 1025), (4, 12, 12, 400),
+                                        (1, 32, 8, 1000)])
+def test_shared_row_waves(dev, b, hq, hkv, s, is_causal, d):
+    """Launches too small for 256-row tiles, whose waves share rows: lengths at
+    the edges of the 32-row groups, of the key tiles and of a round of the
+    waves' tiles; fewer tiles than waves; pairs of tiles. O and LSE of sampled
+    heads against the oracle, every row written."""
+    import cuda_amd._lib as L
+    from cuda_amd.api import _ptr, _stream
+    gen = torch.Generator(device=dev).manual_seed(s)
+    dtype = torch.float16 if d == 64 else torch.bfloat16
+    q, k, v = qkv(b, hq, s, d, dtype, dev, hkv=hkv, gen=gen)
+    out = torch.full_like(q, float("nan"))
+    lse = torch.full((b, hq, s), float("nan"), device=dev)
+    L.call("ca_flash_attention_fwd_lse", L.CA_F16 if d == 64 else L.CA_BF16, _ptr(q), _ptr(k), _ptr(v),
+           _ptr(out), _ptr(lse), b, hq, hkv, s, d, 0.1, int(is_causal), _stream())
+    torch.cuda.synchronize()
+    assert torch.isfinite(out).all() and torch.isfinite(lse).all()
+    for bi, hi in ((0, 0), (b - 1, hq - 1)):
+        kh = hi // (hq // hkv)
+        args = [to_np(q[bi:bi + 1, hi:hi + 1]), to_np(k[bi:bi + 1, kh:kh + 1])]
+        ref = oracle.attention(*args, to_np(v[bi:bi + 1, kh:kh + 1]), is_causal=is_causal, scale=0.1)
+        assert_close(to_np(out[bi:bi + 1, hi:hi + 1]), ref, **TOL_16BIT, name=f"head {bi},{hi}")
+        lref = oracle.attention_lse(*args, is_causal=is_causal, scale=0.1, dtype=np.float64)
+        assert np.abs(to_np(lse[bi:bi + 1, hi:hi + 1]) - lref).max() <= 1e-3
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("is_causal", [False, True])
+@pytest.mark.parametrize("s,jump", [(1, False), (65, False), (200, False), (600, True)])
+def test_short_sequences_full_grid(dev, s, jump, is_causal, d):
+    """Short sequences of many heads: the 256-row kernels' walks of one to ten
+    key tiles, and (jump) key norms that rise past the stale running max."""
+    gen = torch.Generator(device=dev).manual_seed(s)
+    dtype = torch.float16 if jump else torch.bfloat16
+    q, k, v = qkv(8, 64, s, d, dtype, dev, hkv=32, gen=gen)
+    if jump:
+        u = torch.randn(d, device=dev, generator=gen)
+        u = u / u.norm()
+        q = (8 * u + 0.1 * q).to(dtype)
+        k = (torch.where(torch.arange(s, device=dev) < 300, 1.0, 130.0)[:, None] * u + 0.1 * k).to(dtype)
+    out = cuda_llm.flash_attention(q, k, v, is_causal=is_causal)
+    torch.cuda.synchronize()
+    assert torch.isfinite(out).all()
+    for bi, hi in ((0, 0), (7, 63)):
+        ref = oracle.attention(to_np(q[bi:bi + 1, hi:hi + 1]), to_np(k[bi:bi + 1, hi // 2:hi // 2 + 1]),
+                               to_np(v[bi:bi + 1, hi // 2:hi // 2 + 1]), is_causal=is_causal)
+        assert_close(to_np(out[bi:bi + 1, hi:hi + 1]), ref, **TOL_16BIT, name=f"head {bi},{hi}")
