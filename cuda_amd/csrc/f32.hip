@@ -9,9 +9,8 @@
 //
 // Two kernels. prefill_f32_kernel: one workgroup = 4 waves x 32 query rows of
 // one (b, h); K/V tiles of 32 keys, double-buffered in LDS (register-staged
-// loads, one barrier per tile). prefill_f32_split_kernel (launches with fewer
-// 128-row tiles than CUs): one workgroup per pair of 32-row query blocks, its
-// 4 waves splitting the pair's key tiles and merging their softmax states
+// loads, one barrier per tile). prefill_f32_split_kernel (few or unequal tiles,
+// f32_splits): one workgroup per pair of 32-row query blocks, its 4 waves splitting the pair's key tiles and merging their softmax states
 // (described at the kernel). Per wave and tile, both on
 // v_mfma_f32_32x32x2_f32 (one fp32 element of each operand per lane,
 // k = lane / 32):
@@ -532,6 +531,27 @@ __global__ __launch_bounds__(64 * SplitStage<D>::NW, 1) void prefill_f32_split_k
   if (p2 >= 0) prefill_f32_split_merge<D>(O, Lse, S, bh, p2, 1, stg);
 }
 
+// Whether a launch of `grid` work items of 128-row tiles (n_qt per head, n_bh
+// heads) splits each 32-row block's key walk instead (prefill_f32_split_kernel):
+// - fewer tiles than three quarters of the CUs (2 x 8 heads x 1024 x 64,
+//   causal: 27 us against 91; at 192 tiles, not causal, D = 64, 55 against 48);
+// - not causal, D = 128: up to two tiles per CU (32 heads x 1500: 453 -> 354 us);
+//   D = 64 runs two workgroups per CU well (179 us against 195 at 16 x 2048);
+// - causal, too few tiles to pair: the walks differ in length, the split ones
+//   do not. D = 128 always (16 heads x 2048: 344 -> 169 us; 256 x 300: 151 ->
+//   112) but for heads of one full tile (256 x 128: 31 against 37), D = 64 where the longest walk is 1.2 times the mean load or more (16 x
+//   2048: 180 -> 105 us; 256 x 300, 1.1 times: 57 against 61).
+static bool f32_splits(long long grid, bool paired, bool causal, int D, int S, long long n_qt,
+                       long long n_bh) {
+  const long long cus = device_cus();
+  if (4 * grid < 3 * cus) return true;
+  if (grid > 0x1fffffff) return false;  // (the split grid is up to twice as large)
+  if (!causal) return D == 128 && grid < 2 * cus;
+  if (paired) return false;
+  if (D == 128) return n_qt > 1 || S <= 64;
+  return 10 * 2 * cus > 6 * n_bh * (n_qt + 1);
+}
+
 template <int D, bool CAUSAL>
 static hipError_t launch_prefill_f32_t(const void* q, const void* k, const void* v, void* o, float* lse,
                                        int B, int Hq, int Hkv, int S, float scale,
@@ -542,8 +562,7 @@ static hipError_t launch_prefill_f32_t(const void* q, const void* k, const void*
   const long long grid = prefill_grid(B, Hq, n_qt, CAUSAL, 2, &paired);
   if (grid == 0) return hipSuccess;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  if (grid < device_cus()) {
-    // fewer 128-row tiles than CUs: split each 32-row block's key walk
+  if (f32_splits(grid, paired, CAUSAL, D, S, n_qt, (long long)B * Hq)) {
     const int n_qb = (S + 31) / 32;
     const bool two = CAUSAL || (long long)B * Hq * n_qb > device_cus();
     const int per_head = two ? (n_qb + 1) / 2 : n_qb;

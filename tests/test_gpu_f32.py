@@ -163,6 +163,26 @@ def test_split_key_walk_f32(dev, head_dim, is_causal, b, hq, hkv, s):
 
 @pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize("is_causal", [False, True])
+@pytest.mark.parametrize("b,hq,hkv,s", [(2, 48, 12, 255), (1, 32, 8, 1000), (3, 16, 16, 700), (1, 256, 64, 130),
+                                        (4, 32, 8, 1000)])
+def test_prefill_dispatch_edges_f32(dev, head_dim, is_causal, b, hq, hkv, s):
+    """Grids on both sides of the lines between the split key walk and whole
+    tiles: 192 and 256 tiles, more, several rounds of short tiles, and enough
+    to pair. Sampled heads against the oracle, every row finite."""
+    gen = torch.Generator(device=dev).manual_seed(s)
+    q, k, v = qkv(b, hq, s, head_dim, F32, dev, hkv=hkv, gen=gen)
+    out = cuda_llm.flash_attention(q, k, v, is_causal=is_causal)
+    torch.cuda.synchronize()
+    assert torch.isfinite(out).all()
+    for bi, hi in ((0, 0), (b - 1, hq - 1)):
+        kh = hi // (hq // hkv)
+        ref = oracle.attention(to_np(q[bi:bi + 1, hi:hi + 1]), to_np(k[bi:bi + 1, kh:kh + 1]),
+                               to_np(v[bi:bi + 1, kh:kh + 1]), is_causal=is_causal, dtype=np.float64)
+        assert_close(to_np(out[bi:bi + 1, hi:hi + 1]), ref, **TOL_F32, name=f"head {bi},{hi}")
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("is_causal", [False, True])
 @pytest.mark.parametrize("s", [300, 1111])
 def test_zero_scale_is_running_mean_f32(dev, head_dim, is_causal, s):
     """softmax_scale = 0 weighs every visible key equally: row i is the mean
