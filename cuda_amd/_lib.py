@@ -86,3 +86,33 @@ def call(name, *args):
                 CA_LAUNCH_FAILED: "launch failed"}.get(st, f"status {st}")
         raise RuntimeError(f"{msg} [{kind}]")
     return st
+
+
+class _General:
+    """Stands in for the extension module while the library is not built: every
+    call is the general path's, which raises as it always has."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+#: functions whose addresses the extension module takes, in its order (csrc/pyfast.cpp, Abi)
+NATIVE_FUNCTIONS = (
+    "ca_flash_attention_fwd", "ca_flash_attention_fwd_lse", "ca_flash_attention_bwd",
+    "ca_flash_attention_bwd_workspace_bytes", "ca_fused_rope_flash_attention", "ca_rope_workspace_bytes",
+    "ca_flash_decode", "ca_paged_attention", "ca_fp8_paged_attention", "ca_decode_workspace_bytes",
+    "ca_paged_kv_append", "ca_fused_microscaled_attention", "ca_mx_workspace_bytes")
+
+
+def native():
+    """The extension module of the plain calls (csrc/pyfast.cpp), bound to the
+    library that load() gives."""
+    if not os.path.exists(LIB_PATH):
+        return _General()
+    lib = load()
+    try:
+        from . import _native
+    except ImportError as e:
+        raise LibraryNotBuilt(f"cuda_amd._native is missing: build it with `python -m cuda_amd.build` ({e})") from e
+    _native.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in NATIVE_FUNCTIONS))
+    return _native

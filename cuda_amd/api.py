@@ -42,6 +42,22 @@ def _check(cond, msg):
         raise RuntimeError(msg)
 
 
+_native_module = None
+
+
+def _native():
+    """The extension module (csrc/pyfast.cpp): a function per entry point, which
+    makes the call if its arguments are the plain case and returns None, having
+    done nothing, if they are not; the code after it here is the general path."""
+    global _native_module
+    if _native_module is None:
+        m = _lib.native()
+        if isinstance(m, _lib._General):
+            return m
+        _native_module = m
+    return _native_module
+
+
 if hasattr(torch._C, "_cuda_getCurrentRawStream") and hasattr(torch._C, "_cuda_getDevice"):
     def _stream():
         # The current device's current stream, as torch.cuda.current_stream()
@@ -104,6 +120,9 @@ def flash_attention_forward(q, k, v, is_causal=False, softmax_scale=None):
     q: [B, Hq, S, D]; k, v: [B, Hkv, S, D] (Hkv == Hq in the reference; any
     divisor of Hq here). Reference: fused_softmax_binding.cpp:49-103.
     """
+    out = _native().flash_attention_forward(q, k, v, is_causal, softmax_scale)
+    if out is not None:
+        return out
     _prefill_checks(q, k, v)
     b, hq, s, d = q.shape
     dt = _dtype_code(q, "FlashAttention")
@@ -120,6 +139,9 @@ def flash_attention_forward_lse(q, k, v, is_causal=False, softmax_scale=None):
     no visible key). No reference counterpart: the reference's forward returns
     O only; its backward takes this LSE (fused_softmax_binding.cpp:367-376),
     which its tests build with ref_lse (tests/_utils.py:56-64)."""
+    res = _native().flash_attention_forward_lse(q, k, v, is_causal, softmax_scale)
+    if res is not None:
+        return res
     _prefill_checks(q, k, v)
     b, hq, s, d = q.shape
     dt = _dtype_code(q, "FlashAttention")
@@ -139,6 +161,9 @@ def flash_attention_backward(dout, q, k, v, out, lse, is_causal=False, softmax_s
     S, D]; k, v: [B, Hkv, S, D] (GQA: dk, dv sum over the q heads of a kv
     head). fp16 / bf16 / float32; lse is converted to contiguous float32 as
     the reference does."""
+    res = _native().flash_attention_backward(dout, q, k, v, out, lse, is_causal, softmax_scale)
+    if res is not None:
+        return res
     _check(dout.is_cuda and q.is_cuda and k.is_cuda and v.is_cuda and out.is_cuda,
            "Inputs must be on CUDA")
     _check(lse.is_cuda, "LSE tensor must be on CUDA")
@@ -208,6 +233,9 @@ def fused_rope_flash_attention(q, k, v, cos_tab, sin_tab, is_causal=True, softma
     rotate-half convention, cos_tab / sin_tab [seq_len, head_dim] (converted
     to contiguous float32 as the reference does); q, k, v as
     flash_attention_forward (GQA allowed)."""
+    out = _native().fused_rope_flash_attention(q, k, v, cos_tab, sin_tab, is_causal, softmax_scale)
+    if out is not None:
+        return out
     _check(cos_tab.is_cuda and sin_tab.is_cuda, "RoPE tables must be on CUDA")
     _prefill_checks(q, k, v)
     b, hq, s, d = q.shape
@@ -231,6 +259,9 @@ def fused_rope_flash_attention(q, k, v, cos_tab, sin_tab, is_causal=True, softma
 def async_flash_decode(q, k, v, softmax_scale=None):
     """q: [B, Hq, 1, D]; k, v: [B, Hkv, S_kv, D] -> [B, Hq, 1, D].
     Reference: fused_softmax_binding.cpp:308-360."""
+    out = _native().async_flash_decode(q, k, v, softmax_scale)
+    if out is not None:
+        return out
     _check(q.is_cuda and k.is_cuda and v.is_cuda, "Inputs must be on CUDA")
     _check(q.dim() == 4 and k.dim() == 4 and v.dim() == 4,
            "Inputs must be 4D [batch, heads, seq, dim]")
@@ -295,6 +326,10 @@ def paged_attention_forward(query, key_cache, value_cache, block_tables, context
     query [N, Hq, D]; caches [num_blocks, Hkv, D, 16] of the query dtype;
     block_tables int32 [N, max_blocks]; context_lens int32 [N] -> [N, Hq, D].
     """
+    out = _native().paged_attention_forward(query, key_cache, value_cache, block_tables, context_lens,
+                                            softmax_scale)
+    if out is not None:
+        return out
     n, hq, hkv, d = _paged_checks(query, key_cache, value_cache, block_tables, context_lens)
     _check(key_cache.dtype == query.dtype and value_cache.dtype == query.dtype,
            "Caches must have the query dtype")
@@ -323,6 +358,10 @@ def fp8_paged_attention_forward(query, key_cache_fp8, value_cache_fp8, k_scale, 
     Scales: fp32-convertible, [Hkv] per head or [num_blocks, Hkv] per block
     (``k_scale.dim() == 2`` selects per-block, :671). Output in query dtype.
     """
+    out = _native().fp8_paged_attention_forward(query, key_cache_fp8, value_cache_fp8, k_scale, v_scale,
+                                                block_tables, context_lens, softmax_scale)
+    if out is not None:
+        return out
     _check(k_scale.is_cuda and v_scale.is_cuda, "Scale tensors must be on CUDA")
     n, hq, hkv, d = _paged_checks(query, key_cache_fp8, value_cache_fp8, block_tables, context_lens)
     _check(key_cache_fp8.dtype in _FP8_CACHE_DTYPES and value_cache_fp8.dtype in _FP8_CACHE_DTYPES,
@@ -374,6 +413,9 @@ def paged_kv_append(key, value, key_cache, value_cache, block_tables, context_le
     py:52-55 per page). Positions past the table and block ids outside the
     pool are skipped.
     """
+    if _native().paged_kv_append(key, value, key_cache, value_cache, block_tables, context_lens, new_lens,
+                                 k_scale, v_scale):
+        return
     _check(key.is_cuda and value.is_cuda and key_cache.is_cuda and value_cache.is_cuda,
            "Inputs must be on CUDA")
     _check(block_tables.is_cuda and context_lens.is_cuda, "Metadata tensors must be on CUDA")
@@ -458,6 +500,11 @@ def fused_microscaled_attention(q_fp8, q_scale, k_fp8, k_scale, v_fp8, v_scale,
     Mixed forms are brought to e8m0 bytes here, which checks them. Output
     [B, H, S, 128] bf16/fp16.
     """
+    if out_dtype in (torch.bfloat16, torch.float16):
+        out = _native().fused_microscaled_attention(q_fp8, q_scale, k_fp8, k_scale, v_fp8, v_scale, is_causal,
+                                                    softmax_scale, out_dtype is torch.float16)
+        if out is not None:
+            return out
     for t in (q_fp8, k_fp8, v_fp8, q_scale, k_scale, v_scale):
         _check(t.is_cuda, "Inputs must be on CUDA")
     _check(q_fp8.dim() == 4, "Expected 4D tensor: [batch, num_heads, seq_len, head_dim]")

@@ -3,7 +3,8 @@
 Usage: ``python -m cuda_amd.build`` (or ``__graft_entry__.build()``).
 Each HIP source is compiled to an object in ``cuda_amd/_build/`` (in
 parallel), then linked into the in-tree shared library that
-``cuda_amd._lib`` loads. Nothing is hipified: the sources are written for
+``cuda_amd._lib`` loads; ``csrc/pyfast.cpp`` becomes the extension module
+``cuda_amd._native``. Nothing is hipified: the sources are written for
 gfx950 directly.
 """
 import os
@@ -15,6 +16,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libcuda_llm_amd.so")
+NATIVE = os.path.join(HERE, "_native.so")
 SOURCES = ["prefill.hip", "prefill_rows.hip", "prefill_w64.hip", "prefill_w64_mx.hip", "decode.hip", "mxfp8.hip", "f32.hip", "backward.hip", "backward_f32.hip",
            "kv_append.hip", "rope.hip", "stream_read.hip", "abi.cpp"]
 ARCH = os.environ.get("CA_OFFLOAD_ARCH", "gfx950")
@@ -77,11 +79,34 @@ def _compile(src):
     return obj
 
 
+def _build_native():
+    """The extension module: host C++ against this interpreter and torch."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(os.path.abspath(torch.__file__))
+    lib = os.path.join(root, "lib")
+    rocm = os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM",
+           "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", os.path.join(root, "include"), "-isystem", rocm,
+           "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, "pyfast.cpp"),
+           "-o", NATIVE + ".tmp", f"-L{lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python",
+           f"-Wl,-rpath,{lib}"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"pyfast.cpp failed:\n{r.stderr}")
+    os.replace(NATIVE + ".tmp", NATIVE)
+
+
 def build(verbose=True):
-    """Compile every HIP source and link the shared library. Returns its path."""
+    """Compile every HIP source, link the shared library and build the extension
+    module. Returns the library's path."""
     os.makedirs(BUILD, exist_ok=True)
     with ThreadPoolExecutor(max_workers=min(4, len(SOURCES))) as ex:
+        native = ex.submit(_build_native)
         objs = list(ex.map(_compile, SOURCES))
+        native.result()
     tmp = LIB + ".tmp"
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp]
     r = subprocess.run(cmd, capture_output=True, text=True)
