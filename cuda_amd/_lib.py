@@ -41,6 +41,8 @@ SIGNATURES = {
                                             _I, _P, _Z, _P]),
     "ca_mx_workspace_bytes": (_Z, [_I, _I, _I, _I, _I]),
     "ca_decode_workspace_bytes": (_Z, [_I, _I, _I, _I]),
+    "ca_paged_decode_workspace_bytes": (_Z, [_I, _I, _I, _I, _I, _I, _I]),
+    "ca_flash_decode_workspace_bytes": (_Z, [_I, _I, _I, _I, _I, _I]),
     "ca_check_block_tables": (_I, [_P, _P, _I, _I, _I, _I, _P]),
     "ca_check_mx_scales": (_I, [_P, _P, _P, _I, _I, _I, _I, _P]),
     "ca_last_error": (ctypes.c_char_p, []),
@@ -100,7 +102,8 @@ class _General:
 NATIVE_FUNCTIONS = (
     "ca_flash_attention_fwd", "ca_flash_attention_fwd_lse", "ca_flash_attention_bwd",
     "ca_flash_attention_bwd_workspace_bytes", "ca_fused_rope_flash_attention", "ca_rope_workspace_bytes",
-    "ca_flash_decode", "ca_paged_attention", "ca_fp8_paged_attention", "ca_decode_workspace_bytes",
+    "ca_flash_decode", "ca_flash_decode_workspace_bytes", "ca_paged_attention", "ca_fp8_paged_attention",
+    "ca_paged_decode_workspace_bytes",
     "ca_paged_kv_append", "ca_fused_microscaled_attention", "ca_mx_workspace_bytes")
 
 

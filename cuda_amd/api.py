@@ -276,7 +276,7 @@ def async_flash_decode(q, k, v, softmax_scale=None):
     q, k, v = (_aligned(t.contiguous()) for t in (q, k, v))
     hkv, s_kv = k.size(1), k.size(2)
     out = torch.empty_like(q)
-    ws, nbytes = _workspace(_lib.load().ca_decode_workspace_bytes(b, hq, d, s_kv), q.device)
+    ws, nbytes = _workspace(_lib.load().ca_flash_decode_workspace_bytes(dt, b, hq, hkv, s_kv, d), q.device)
     _lib.call("ca_flash_decode", dt, _ptr(q), _ptr(k), _ptr(v), _ptr(out), b, hq, hkv, s_kv, d,
               _scale(softmax_scale, d), _ptr(ws), nbytes, _stream())
     return out
@@ -339,7 +339,7 @@ def paged_attention_forward(query, key_cache, value_cache, block_tables, context
     _debug_check_tables(block_tables, context_lens, key_cache.size(0))
     out = torch.empty_like(query)
     max_blocks = block_tables.size(1)
-    ws, nbytes = _workspace(_lib.load().ca_decode_workspace_bytes(n, hq, d, max_blocks * 16),
+    ws, nbytes = _workspace(_lib.load().ca_paged_decode_workspace_bytes(dt, 0, n, hq, hkv, d, max_blocks),
                             query.device)
     _lib.call("ca_paged_attention", dt, _ptr(query), _ptr(key_cache), _ptr(value_cache),
               _ptr(block_tables), _ptr(context_lens), _ptr(out), n, hq, hkv, d, max_blocks, 16,
@@ -384,7 +384,7 @@ def fp8_paged_attention_forward(query, key_cache_fp8, value_cache_fp8, k_scale, 
     _debug_check_tables(block_tables, context_lens, num_blocks)
     out = torch.empty_like(query)
     max_blocks = block_tables.size(1)
-    ws, nbytes = _workspace(_lib.load().ca_decode_workspace_bytes(n, hq, d, max_blocks * 16),
+    ws, nbytes = _workspace(_lib.load().ca_paged_decode_workspace_bytes(dt, 1, n, hq, hkv, d, max_blocks),
                             query.device)
     _lib.call("ca_fp8_paged_attention", dt, _ptr(query), _ptr(kc), _ptr(vc), _ptr(k_scale),
               _ptr(v_scale), int(per_block), _ptr(block_tables), _ptr(context_lens), _ptr(out),

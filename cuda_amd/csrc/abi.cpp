@@ -108,6 +108,30 @@ size_t ca_decode_workspace_bytes(int num_seqs, int num_q_heads, int head_dim, in
   return ca::decode_workspace_bytes(num_seqs, num_q_heads, head_dim, max_tokens);
 }
 
+size_t ca_paged_decode_workspace_bytes(ca_dtype dtype, int fp8_cache, int num_seqs, int num_q_heads,
+                                       int num_kv_heads, int head_dim, int max_blocks_per_seq) {
+  if (num_seqs <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 ||
+      (head_dim != 64 && head_dim != 128) || max_blocks_per_seq <= 0 ||
+      max_blocks_per_seq > INT_MAX / ca::kDecodePage ||
+      !product_at_most(1LL << 40, {num_seqs, num_q_heads, max_blocks_per_seq}))
+    return 0;
+  return std::max(ca::decode_workspace_bytes(num_seqs, num_q_heads, head_dim,
+                                             max_blocks_per_seq * ca::kDecodePage),
+                  ca::paged_decode_partials_bytes((int)dtype, fp8_cache != 0, num_seqs, num_q_heads,
+                                                  num_kv_heads, head_dim, max_blocks_per_seq, SIZE_MAX));
+}
+
+size_t ca_flash_decode_workspace_bytes(ca_dtype dtype, int batch, int num_q_heads, int num_kv_heads,
+                                       int kv_len, int head_dim) {
+  if (batch <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads != 0 ||
+      (head_dim != 64 && head_dim != 128) || kv_len <= 0 ||
+      !product_at_most(1LL << 40, {batch, num_q_heads, kv_len}))
+    return 0;
+  return std::max(ca::decode_workspace_bytes(batch, num_q_heads, head_dim, kv_len),
+                  ca::flash_decode_partials_bytes((int)dtype, batch, num_q_heads, num_kv_heads, head_dim,
+                                                  kv_len));
+}
+
 static ca_status prefill_entry(const char* what, ca_dtype dtype, const void* q, const void* k,
                                const void* v, void* o, float* lse, int batch, int num_q_heads,
                                int num_kv_heads, int seq_len, int head_dim, float softmax_scale,
@@ -307,7 +331,8 @@ ca_status ca_fp8_paged_attention_noalloc(ca_dtype dtype, const void* query,
   if (num_seqs == 0) return CA_OK;
   if (!k_scale || !v_scale) return fail(CA_INVALID_ARGUMENT, "%s: null scale pointer", what);
   const size_t need = ca::paged_decode_partials_bytes((int)dtype, 1, num_seqs, num_q_heads,
-                                                      num_kv_heads, head_dim, max_blocks_per_seq);
+                                                      num_kv_heads, head_dim, max_blocks_per_seq,
+                                                      ca::kNoAllocScratchBytes);
   if (need > ca::kNoAllocScratchBytes)
     return fail(CA_INVALID_ARGUMENT,
                 "%s: these sizes need %zu bytes of split partials, more than the %zu bytes of "

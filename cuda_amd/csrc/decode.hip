@@ -837,22 +837,6 @@ __global__ __launch_bounds__(64) void decode_sk_merge_kernel(
                     ws_o, ws_lse, O, orow);
 }
 
-// Splits per (sequence, kv head, chunk) of a contiguous decode of `segs` of
-// them, `pages` pages each: enough for two workgroups per CU (160 heads of
-// 3000 tokens, head dim 128: 43 us against 51 with one split, 43 with twice as
-// many), as far as the workspace goes; none when the heads alone are about one
-// workgroup per CU, which saves the merge (256 heads of 4096 tokens, head dim
-// 64: 47 us against 52 with two splits).
-static int contig_splits(long long segs, int pages) {
-  const int cus = device_cus();
-  if (segs <= cus && segs >= cus - cus / 8) return 1;
-  const int most = std::max(1, pages / kPagesPerWave + (pages % kPagesPerWave != 0));
-  int s = 1;
-  while (s < most && segs * s < 2 * cus) ++s;
-  const int per = std::max(1, (pages + s - 1) / s);
-  return std::max(1, (pages + per - 1) / per);
-}
-
 // Bytes of split partials for max_splits splits per (sequence, query head):
 // [N][Hq][max_splits] x D floats of o / l, then [N][Hq][max_splits] floats
 // of log2-sum-exp; none when every context fits one split.
@@ -902,22 +886,53 @@ static size_t sk_partials_bytes(int grid, int N, int Gq, int D) {
          (size_t)N * sizeof(int32_t);
 }
 
+// Splits of the split grid's longest context, pages per split, and the bytes of
+// partials it writes.
+struct SplitGrid {
+  int max_splits = 1, pages = 1;
+  size_t bytes = 0;
+};
+// `segs` walks of `pages` pages in splits of `coarse`, or finer where those
+// leave most CUs idle and the workspace holds the partials: up to four
+// workgroups per CU, 16 pages or more per split (a step of two for each of 8
+// waves) and 16 splits, which the merge loads at once. Measured against the
+// coarse splits: 3 bf16 sequences of 90-3000 tokens with their append 20.4 ->
+// 15.6 us, 1 of 1100 14.7 -> 9.7, contiguous 1 x 8 x 4001 16.1 -> 11.2, 24 FP8
+// sequences (head dim 64) 26.9 -> 23.5. Where the coarse 16-bit splits already
+// fill half the CUs (64 walks of 256 pages 21.6 -> 22.4 us) or the FP8 ones one
+// and a half (800 workgroups 47 -> 51) they stay, as with more than 16 splits
+// (8 walks of 1024 pages 20.9 -> 33).
+static SplitGrid split_grid(long long segs, int N, int Hq, int D, int pages, int coarse, bool fp8, size_t ws_bytes) {
+  SplitGrid g;
+  g.pages = coarse;
+  g.max_splits = std::max(1, pages / coarse + (pages % coarse != 0));
+  g.bytes = split_partials_bytes(N, Hq, D, g.max_splits);
+  const long long cus = device_cus();
+  if (pages <= kPagesPerWave || 2 * segs * g.max_splits > (fp8 ? 3 : 1) * cus) return g;
+  const int fine = (int)std::max<long long>({16, (segs * pages + 4 * cus - 1) / (4 * cus), (pages + 15) / 16});
+  if (fine >= coarse) return g;
+  const int s = pages / fine + (pages % fine != 0);
+  const size_t bytes = split_partials_bytes(N, Hq, D, s);
+  if (bytes > std::min(ws_bytes, kFineSplitBytes)) return g;
+  return {s, fine, bytes};
+}
+
 // How a paged decode launch splits its work: stream-K (grid > 0) when its
 // partials fit the workspace every caller provides (decode_workspace_bytes)
-// and the sequences fit the prefix registers; otherwise the split grid.
+// and the sequences fit the prefix registers; otherwise the split grid, finer
+// where the workspace given (ws_bytes) holds its partials.
 struct PagedPlan {
   int grid = 0;          // stream-K waves, 0 for the split grid
-  int max_splits = 1;    // split grid: splits of the longest context
+  SplitGrid split;
   size_t bytes = 0;      // partials the launch writes
 };
 template <typename Tr, int D, int KIND>
-static PagedPlan paged_plan(int N, int Hq, int Hkv, int max_blocks) {
+static PagedPlan paged_plan(int N, int Hq, int Hkv, int max_blocks, size_t ws_bytes) {
   PagedPlan p;
   constexpr int kPages = DmaCfg<KIND>::kPages;
-  p.max_splits = std::max(1, max_blocks / kPages + (max_blocks % kPages != 0));
   const int Gq = Hq / Hkv;
   const int n_hc = (Gq + 15) / 16;
-  if (p.max_splits > 1 && N <= kSkMaxSeqs &&
+  if (max_blocks > kPages && N <= kSkMaxSeqs &&
       (long long)N * max_blocks * Hkv * n_hc <= (long long)INT_MAX) {
     const int g = sk_grid<Tr, D, KIND>();
     const size_t need = sk_partials_bytes(g, N, Gq, D);
@@ -927,18 +942,23 @@ static PagedPlan paged_plan(int N, int Hq, int Hkv, int max_blocks) {
       return p;
     }
   }
-  p.bytes = split_partials_bytes(N, Hq, D, p.max_splits);
+  p.split = split_grid((long long)N * Hkv * n_hc, N, Hq, D, max_blocks, kPages,
+                       KIND == kKindPagedFp8, ws_bytes);
+  p.bytes = p.split.bytes;
   return p;
 }
 
 // Waves per workgroup of a split grid of `grid` workgroups, at most `pages`
-// pages each. A share of a few pages does not pay for the merge in LDS (128
-// sequences of up to 200 tokens: one wave 15.4 us, four 19.4); up to one
-// workgroup per CU, eight waves shorten the chain further (one sequence of
-// 1000 tokens, 8 kv heads: 9.0 us against 10.7 with four).
+// pages each: eight while the workgroups are few (one sequence of 1000 tokens, 8
+// kv heads: 9.0 us against 10.7 with four; 384 splits of 16 pages 15.6 against
+// 17.7), and one where a share of a few pages would not pay for the merge in
+// LDS (1024 of up to 13 pages: 15.4 us, four waves 19.4).
 static int mw_waves(long long grid, int pages) {
-  if (pages <= 16) return 1;
-  return grid <= device_cus() && pages >= 32 ? 8 : 4;
+  const long long cus = device_cus();
+  if (pages <= 4) return 1;
+  if (grid <= cus) return 8;
+  if (pages <= 16) return grid <= 2 * cus ? 8 : 1;
+  return 4;
 }
 template <typename Tr, int D, int KIND>
 static auto mw_kernel(int nw) {
@@ -957,7 +977,7 @@ static hipError_t launch_paged_decode_t(const void* q, const void* kc, const voi
   const int max_tokens = max_blocks * kDecodePage;
   const int Gq = Hq / Hkv;
   const int n_hc = (Gq + 15) / 16;
-  const PagedPlan plan = paged_plan<Tr, D, KIND>(N, Hq, Hkv, max_blocks);
+  const PagedPlan plan = paged_plan<Tr, D, KIND>(N, Hq, Hkv, max_blocks, ws_bytes);
   if (ws_bytes < plan.bytes) return hipErrorInvalidValue;
   if (plan.grid > 0) {
     const size_t rows = (size_t)2 * plan.grid * std::min(16, Gq);
@@ -974,22 +994,44 @@ static hipError_t launch_paged_decode_t(const void* q, const void* kc, const voi
                        stream, ws_prefix, ws_o, ws_lse, out, N, Hq, Hkv, n_hc, plan.grid);
     return hipGetLastError();
   }
-  const int max_splits = plan.max_splits;
+  const int max_splits = plan.split.max_splits, pages_per_split = plan.split.pages;
   float* ws_o = (float*)ws;
   float* ws_lse = plan.bytes ? ws_o + (size_t)N * Hq * max_splits * D : nullptr;
-  const long long total_waves = (long long)N * Hkv * n_hc * max_splits;
-  if (total_waves == 0) return hipSuccess;
-  if (total_waves > 0x7fffffffLL) return hipErrorInvalidValue;
-  const int nw = mw_waves(total_waves, std::min(max_blocks, DmaCfg<KIND>::kPages));
-  const auto kernel = mw_kernel<Tr, D, KIND>(nw);
-  hipLaunchKernelGGL(kernel, dim3((unsigned)total_waves), dim3(64 * nw), 0, stream, (const uint16_t*)q, kc, vc, k_scale, v_scale, per_block, bt, lens,
+  const long long grid = (long long)N * Hkv * n_hc * max_splits;
+  if (grid == 0) return hipSuccess;
+  if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+  const int nw = mw_waves(grid, std::min(max_blocks, pages_per_split));
+  hipLaunchKernelGGL((mw_kernel<Tr, D, KIND>(nw)), dim3((unsigned)grid), dim3(64 * nw), 0, stream,
+                     (const uint16_t*)q, kc, vc, k_scale, v_scale, per_block, bt, lens,
                      (uint16_t*)out, ws_o, ws_lse, Hq, Hkv, max_blocks, 0, num_blocks, max_splits,
-                     DmaCfg<KIND>::kPages, n_hc, scale * kLog2e);
+                     pages_per_split, n_hc, scale * kLog2e);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || max_splits <= 1) return e;
   hipLaunchKernelGGL((decode_merge_kernel<Tr, D>), dim3((unsigned)(N * Hq)), dim3(64), 0, stream,
-                     lens, max_tokens, ws_o, ws_lse, out, Hq, max_splits, DmaCfg<KIND>::kPages);
+                     lens, max_tokens, ws_o, ws_lse, out, Hq, max_splits, pages_per_split);
   return hipGetLastError();
+}
+
+// The contiguous cache's split grid: as a paged one's, in equal splits; one
+// split when the heads alone are about one workgroup per CU, which saves the
+// merge (256 heads of 4096 tokens, head dim 64: 47 us against 52 with two).
+static SplitGrid contig_grid(int N, int Hq, int Hkv, int D, int S, size_t ws_bytes) {
+  const int cus = device_cus();
+  const int pages = S / kDecodePage + (S % kDecodePage != 0);
+  const long long segs = (long long)N * Hkv * ((Hq / Hkv + 15) / 16);
+  SplitGrid g;
+  g.pages = std::max(1, pages);
+  if (segs <= cus && segs >= cus - cus / 8) return g;
+  // at least two workgroups per CU, as far as every caller's workspace goes
+  const int most = std::max(1, pages / kPagesPerWave + (pages % kPagesPerWave != 0));
+  int s = (int)std::max(1LL, std::min<long long>(most, (2LL * cus + segs - 1) / std::max(1LL, segs)));
+  const SplitGrid fine =
+      split_grid(segs, N, Hq, D, pages, std::max(1, (pages + s - 1) / s), false, ws_bytes);
+  s = fine.max_splits;
+  g.pages = std::max(1, (pages + s - 1) / s);
+  g.max_splits = std::max(1, (pages + g.pages - 1) / g.pages);
+  g.bytes = split_partials_bytes(N, Hq, D, g.max_splits);
+  return g;
 }
 
 template <typename Tr, int D>
@@ -997,27 +1039,24 @@ static hipError_t launch_contig_decode_t(const void* q, const void* k, const voi
                                          int N, int Hq, int Hkv, int S, float scale, void* ws,
                                          size_t ws_bytes, hipStream_t stream) {
   constexpr int KIND = kKindContig16;
-  const int pages = S / kDecodePage + (S % kDecodePage != 0);
   const int Gq = Hq / Hkv;
   const int n_hc = (Gq + 15) / 16;
-  const size_t need = decode_workspace_bytes(N, Hq, D, S);
-  if (ws_bytes < need) return hipErrorInvalidValue;
-  const int max_splits = contig_splits((long long)N * Hkv * n_hc, pages);
-  const int pages_per_split = std::max(1, (pages + max_splits - 1) / max_splits);
+  if (ws_bytes < decode_workspace_bytes(N, Hq, D, S)) return hipErrorInvalidValue;
+  const SplitGrid plan = contig_grid(N, Hq, Hkv, D, S, ws_bytes);
+  const int max_splits = plan.max_splits;
   float* ws_o = (float*)ws;
-  float* ws_lse = need ? ws_o + (size_t)N * Hq * max_splits * D : nullptr;
+  float* ws_lse = plan.bytes ? ws_o + (size_t)N * Hq * max_splits * D : nullptr;
   const long long grid = (long long)N * Hkv * n_hc * max_splits;
   if (grid == 0) return hipSuccess;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  const int nw = mw_waves(grid, pages_per_split);
-  const auto kernel = mw_kernel<Tr, D, KIND>(nw);
-  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * nw), 0, stream, (const uint16_t*)q, k, v, nullptr, nullptr, 0, nullptr, nullptr,
-                     (uint16_t*)out, ws_o, ws_lse, Hq, Hkv, 0, S, 1, max_splits, pages_per_split,
-                     n_hc, scale * kLog2e);
+  const int nw = mw_waves(grid, plan.pages);
+  hipLaunchKernelGGL((mw_kernel<Tr, D, KIND>(nw)), dim3((unsigned)grid), dim3(64 * nw), 0, stream,
+                     (const uint16_t*)q, k, v, nullptr, nullptr, 0, nullptr, nullptr, (uint16_t*)out,
+                     ws_o, ws_lse, Hq, Hkv, 0, S, 1, max_splits, plan.pages, n_hc, scale * kLog2e);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || max_splits <= 1) return e;
   hipLaunchKernelGGL((decode_merge_kernel<Tr, D>), dim3((unsigned)(N * Hq)), dim3(64), 0, stream,
-                     nullptr, S, ws_o, ws_lse, out, Hq, max_splits, pages_per_split);
+                     nullptr, S, ws_o, ws_lse, out, Hq, max_splits, plan.pages);
   return hipGetLastError();
 }
 
@@ -1398,12 +1437,12 @@ hipError_t with_noalloc_scratch(hipStream_t stream, const std::function<hipError
 }
 
 size_t paged_decode_partials_bytes(int dtype, int cache_kind, int N, int Hq, int Hkv, int D,
-                                   int max_blocks_per_seq) {
+                                   int max_blocks_per_seq, size_t ws_bytes) {
   if (dtype == kDtypeF32)
     return split_partials_bytes(N, Hq, D, max_blocks_per_seq / kPagesPerWave +
                                               (max_blocks_per_seq % kPagesPerWave != 0));
 #define CA_PLAN(TR, DD, KIND) \
-  if (D == DD) return paged_plan<TR, DD, KIND>(N, Hq, Hkv, max_blocks_per_seq).bytes;
+  if (D == DD) return paged_plan<TR, DD, KIND>(N, Hq, Hkv, max_blocks_per_seq, ws_bytes).bytes;
   if (cache_kind == 0) {
     if (dtype == kDtypeBF16) { CA_PLAN(BF16, 64, kKindPaged16) CA_PLAN(BF16, 128, kKindPaged16) }
     if (dtype == kDtypeF16) { CA_PLAN(F16, 64, kKindPaged16) CA_PLAN(F16, 128, kKindPaged16) }
@@ -1413,6 +1452,10 @@ size_t paged_decode_partials_bytes(int dtype, int cache_kind, int N, int Hq, int
   }
 #undef CA_PLAN
   return 0;
+}
+
+size_t flash_decode_partials_bytes(int dtype, int N, int Hq, int Hkv, int D, int S) {
+  return dtype == kDtypeF32 ? decode_workspace_bytes(N, Hq, D, S) : contig_grid(N, Hq, Hkv, D, S, SIZE_MAX).bytes;
 }
 
 hipError_t launch_flash_decode(int dtype, const void* q, const void* k, const void* v, void* o,

@@ -115,11 +115,15 @@ hipError_t launch_paged_decode(int dtype, int cache_kind, const void* q, const v
                                int D, int max_blocks_per_seq, int num_blocks, float scale,
                                void* ws, size_t ws_bytes, hipStream_t stream);
 
-// Bytes of partials a paged decode launch writes on the current device (the
-// exact minimum of its workspace; the entry points require
-// decode_workspace_bytes, which is at least this).
+// Bytes of partials a paged decode launch writes on the current device when it
+// is given a workspace of ws_bytes (small launches split finer where theirs
+// fits it, up to kFineSplitBytes; the entry points require
+// decode_workspace_bytes, which is at least what the others write).
+constexpr size_t kFineSplitBytes = 8u << 20;
 size_t paged_decode_partials_bytes(int dtype, int cache_kind, int N, int Hq, int Hkv, int D,
-                                   int max_blocks_per_seq);
+                                   int max_blocks_per_seq, size_t ws_bytes);
+// ... and a contiguous-cache decode with all the workspace it can use.
+size_t flash_decode_partials_bytes(int dtype, int N, int Hq, int Hkv, int D, int S);
 
 // The allocation-free paged decode's scratch (decode.hip): a file-scope
 // device array of kNoAllocScratchBytes per device; *ptr receives its address

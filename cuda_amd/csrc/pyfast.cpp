@@ -36,9 +36,10 @@ struct Abi {
   decltype(&ca_fused_rope_flash_attention) fused_rope_flash_attention;
   decltype(&ca_rope_workspace_bytes) rope_workspace_bytes;
   decltype(&ca_flash_decode) flash_decode;
+  decltype(&ca_flash_decode_workspace_bytes) flash_decode_workspace_bytes;
   decltype(&ca_paged_attention) paged_attention;
   decltype(&ca_fp8_paged_attention) fp8_paged_attention;
-  decltype(&ca_decode_workspace_bytes) decode_workspace_bytes;
+  decltype(&ca_paged_decode_workspace_bytes) paged_decode_workspace_bytes;
   decltype(&ca_paged_kv_append) paged_kv_append;
   decltype(&ca_fused_microscaled_attention) fused_microscaled_attention;
   decltype(&ca_mx_workspace_bytes) mx_workspace_bytes;
@@ -212,7 +213,7 @@ PyObject* async_flash_decode(PyObject* const* a) {
       (q->size(3) != 64 && q->size(3) != 128) || !scale_of(a[3], n(*q, 3), &scale))
     return nullptr;
   const at::Tensor o = like(*q);
-  const Workspace ws(abi.decode_workspace_bytes(n(*q, 0), n(*q, 1), n(*q, 3), n(*k, 2)), *q);
+  const Workspace ws(abi.flash_decode_workspace_bytes(dt, n(*q, 0), n(*q, 1), n(*k, 1), n(*k, 2), n(*q, 3)), *q);
   if (!ok([&] {
         return abi.flash_decode(dt, in(*q), in(*k), in(*v), out(o), n(*q, 0), n(*q, 1), n(*k, 1), n(*k, 2), n(*q, 3),
                                 scale, ws.ptr(), ws.bytes, stream());
@@ -255,7 +256,7 @@ PyObject* paged_attention_forward(PyObject* const* a) {
       debug_asked("CUDA_LLM_CHECK_BLOCK_TABLES"))
     return nullptr;
   const at::Tensor o = like(*q);
-  const Workspace ws(abi.decode_workspace_bytes(n(*q, 0), n(*q, 1), n(*q, 2), n(*bt, 1) * 16), *q);
+  const Workspace ws(abi.paged_decode_workspace_bytes(dt, 0, n(*q, 0), n(*q, 1), n(*kc, 1), n(*q, 2), n(*bt, 1)), *q);
   if (!ok([&] {
         return abi.paged_attention(dt, in(*q), in(*kc), in(*vc), (const int32_t*)in(*bt), (const int32_t*)in(*cl),
                                    out(o), n(*q, 0), n(*q, 1), n(*kc, 1), n(*q, 2), n(*bt, 1), 16, n(*kc, 0), scale,
@@ -276,7 +277,7 @@ PyObject* fp8_paged_attention_forward(PyObject* const* a) {
       debug_asked("CUDA_LLM_CHECK_BLOCK_TABLES"))
     return nullptr;
   const at::Tensor o = like(*q);
-  const Workspace ws(abi.decode_workspace_bytes(n(*q, 0), n(*q, 1), n(*q, 2), n(*bt, 1) * 16), *q);
+  const Workspace ws(abi.paged_decode_workspace_bytes(dt, 1, n(*q, 0), n(*q, 1), n(*kc, 1), n(*q, 2), n(*bt, 1)), *q);
   if (!ok([&] {
         return abi.fp8_paged_attention(dt, in(*q), (const uint8_t*)in(*kc), (const uint8_t*)in(*vc),
                                        (const float*)in(*ks), (const float*)in(*vs), ks->dim() == 2,

@@ -282,6 +282,18 @@ ca_status ca_check_block_tables(const int32_t* block_tables, const int32_t* cont
  * entry points. No counterpart in the reference (its decode is not split). */
 size_t ca_decode_workspace_bytes(int num_seqs, int num_q_heads, int head_dim, int max_tokens);
 
+/* Bytes with which a 16-bit decode runs at its best: at least
+ * ca_decode_workspace_bytes(), which stays the least that is accepted. Small
+ * launches (few sequences and heads) split each context finer when the
+ * workspace they are given holds the partials (at most 8 MiB); the split, and
+ * so the rounding of a result, follows from the sizes and workspace_bytes.
+ * 0 for sizes that are not valid. fp8_cache: 0 for ca_paged_attention, 1 for
+ * ca_fp8_paged_attention. */
+size_t ca_paged_decode_workspace_bytes(ca_dtype dtype, int fp8_cache, int num_seqs, int num_q_heads,
+                                       int num_kv_heads, int head_dim, int max_blocks_per_seq);
+size_t ca_flash_decode_workspace_bytes(ca_dtype dtype, int batch, int num_q_heads, int num_kv_heads,
+                                       int kv_len, int head_dim);
+
 /* Thread-local description of the last non-OK status of this thread. */
 const char* ca_last_error(void);
 

@@ -304,6 +304,49 @@ def test_flash_decode_waves_and_splits(dev, head_dim, b, hq, hkv, kv_len):
                  name=f"decode {kv_len}")
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+def test_least_workspace_takes_coarse_splits(dev, fp8):
+    """ca_decode_workspace_bytes stays enough: with it the small launches keep
+    their coarse splits, with ca_*_decode_workspace_bytes they split finer (the
+    guard bytes after either workspace stay as they were); both against the
+    oracle, the paged and the contiguous cache."""
+    import ctypes
+    import cuda_amd._lib as L
+    lib = L.load()
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    case = build_paged([2500, 1, 0, 1040], 8, 2, 128, torch.bfloat16, dev, fp8=fp8, per_block=True, seed=9)
+    q, kc, vc = case["query"], case["key_cache"], case["value_cache"]
+    n, hq, d = q.shape
+    width = case["block_tables"].shape[1]
+    least = lib.ca_decode_workspace_bytes(n, hq, d, width * 16)
+    best = lib.ca_paged_decode_workspace_bytes(L.CA_BF16, int(fp8), n, hq, 2, d, width)
+    assert best > least > 0
+    scales = (p(case["k_scale"]), p(case["v_scale"]), 1) if fp8 else ()
+    name = "ca_fp8_paged_attention" if fp8 else "ca_paged_attention"
+    ref = paged_oracle(case)
+    kk, vv = (torch.randn(1, 2, 1500, d, device=dev).bfloat16() for _ in range(2))
+    qq = torch.randn(1, hq, 1, d, device=dev).bfloat16()
+    cref = oracle.attention(to_np(qq), to_np(kk), to_np(vv))
+    cleast = lib.ca_decode_workspace_bytes(1, hq, d, 1500)
+    cbest = lib.ca_flash_decode_workspace_bytes(L.CA_BF16, 1, hq, 2, 1500, d)
+    assert cbest > cleast > 0
+    for size, csize in ((least, cleast), (best, cbest)):
+        ws = torch.full((max(size, csize) + 64,), 0x5A, dtype=torch.uint8, device=dev)
+        out = torch.empty_like(q)
+        L.call(name, L.CA_BF16, p(q), p(kc), p(vc), *scales, p(case["block_tables"]), p(case["context_lens"]),
+               p(out), n, hq, 2, d, width, 16, kc.shape[0], d ** -0.5, p(ws), size, None)
+        torch.cuda.synchronize()
+        assert (ws[size:] == 0x5A).all()
+        assert_close(to_np(out), ref, **(TOL_FP8 if fp8 else TOL_16BIT), name=f"paged {size}")
+        ws.fill_(0x5A)
+        out = torch.empty_like(qq)
+        L.call("ca_flash_decode", L.CA_BF16, p(qq), p(kk), p(vv), p(out), 1, hq, 2, 1500, d, d ** -0.5, p(ws),
+               csize, None)
+        torch.cuda.synchronize()
+        assert (ws[csize:] == 0x5A).all()
+        assert_close(to_np(out), cref, **TOL_16BIT, name=f"contiguous {csize}")
+
+
 def test_baseline_c3_shape(dev):
     """C3: N=64, Hq=32/Hkv=8, D=128, L ~ U[512, 8192], 40k-page pool,
     permuted; every sequence against the oracle."""

@@ -42,6 +42,21 @@ def test_refuses_what_is_not_plain():
         n.bind(1)
 
 
+def test_decode_workspace_sizes():
+    """The best workspace is never less than the least one; invalid sizes are 0."""
+    lib = L.load()
+    for n, hq, hkv, d, blocks in ((1, 32, 8, 128, 3), (3, 32, 8, 128, 256), (64, 32, 8, 64, 512), (1, 1, 1, 64, 2 ** 26)):
+        least = lib.ca_decode_workspace_bytes(n, hq, d, 16 * blocks)
+        for dt in (L.CA_F32, L.CA_F16, L.CA_BF16):
+            for fp8 in (0, 1):
+                assert lib.ca_paged_decode_workspace_bytes(dt, fp8, n, hq, hkv, d, blocks) >= least
+            assert lib.ca_flash_decode_workspace_bytes(dt, n, hq, hkv, 16 * blocks, d) >= least
+    big = 2 ** 31 - 1
+    for bad in ((0, 32, 8, 128, 4), (1, 32, 5, 128, 4), (1, 32, 8, 96, 4), (1, 32, 8, 128, -1), (big, big, 1, 128, big)):
+        assert lib.ca_paged_decode_workspace_bytes(L.CA_BF16, 0, *bad) == 0
+        assert lib.ca_flash_decode_workspace_bytes(L.CA_BF16, *bad[:3], bad[4], bad[3]) == 0
+
+
 def _same(a, b):
     a, b = ([x] if torch.is_tensor(x) else list(x) for x in (a, b))
     assert len(a) == len(b)
