@@ -424,9 +424,9 @@ __global__ __launch_bounds__(64 * bwdma::kNW) void bwd_dq_dma_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ dO,
     const float* __restrict__ LD, uint16_t* __restrict__ dQ, int S, int Hq, int Hkv, float scale,
-    int n_qt, int n_bh, int n_work, int paired) {
+    int n_qt, int n_bh, int n_work, int order) {
   const QTileWork wk =
-      prefill_work(xcd_remap(__builtin_amdgcn_workgroup_id_x(), n_work), n_qt, n_bh, paired);
+      prefill_item(__builtin_amdgcn_workgroup_id_x(), n_work, n_qt, n_bh, order);
   const int n_pass = wk.qt1 < 0 ? 1 : 2;
 #pragma clang loop unroll(disable)
   for (int pass = 0; pass < n_pass; ++pass) {
@@ -692,11 +692,11 @@ __global__ __launch_bounds__(64 * bwdma::kNW) void bwd_dkv_dma_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ dO,
     const float* __restrict__ LD, uint16_t* __restrict__ dK, uint16_t* __restrict__ dV, int S,
-    int Hq, int Hkv, float scale, int n_kt, int n_bh, int n_work, int paired) {
+    int Hq, int Hkv, float scale, int n_kt, int n_bh, int n_work, int order) {
   // key tile kt walks n_kt - kt query stretches: kt = n_kt - 1 - qt gives the
-  // longest walks first (unpaired) and pairs of equal total length (paired)
+  // longest walks first (single) and pairs of equal total length
   const QTileWork wk =
-      prefill_work(xcd_remap(__builtin_amdgcn_workgroup_id_x(), n_work), n_kt, n_bh, paired);
+      prefill_item(__builtin_amdgcn_workgroup_id_x(), n_work, n_kt, n_bh, order);
   const int n_pass = wk.qt1 < 0 ? 1 : 2;
 #pragma clang loop unroll(disable)
   for (int pass = 0; pass < n_pass; ++pass) {
@@ -719,7 +719,7 @@ __global__ __launch_bounds__(64 * bwdma::kNW) void bwd_dkv_dma_kernel(
 // equal pairs with 4 (dK/dV 827 -> 605 us); 8 kv heads of 1000, forward and dQ
 // aside, are 32 workgroups with 8 groups and 128 with 2 (backward 243 -> 114 us).
 struct BwdSplit {
-  int groups, n_tiles, paired;
+  int groups, n_tiles, order;
   long long grid;
 };
 BwdSplit bwd_split(int B, int heads, int S, bool causal, int cost4, int cost2) {
@@ -730,10 +730,10 @@ BwdSplit bwd_split(int B, int heads, int S, bool causal, int cost4, int cost2) {
     BwdSplit s{};
     s.groups = groups;
     s.n_tiles = (S + 32 * groups - 1) / (32 * groups);
-    s.grid = prefill_grid(B, heads, s.n_tiles, causal, 1, &s.paired);
+    s.grid = prefill_grid(B, heads, s.n_tiles, causal, 1, &s.order);
     // walk lengths in tiles of the busiest CU, times the work of a tile
     const long long tiles = (long long)B * heads * s.n_tiles;
-    const long long walks = causal ? (s.paired ? (s.grid + cus - 1) / cus * (s.n_tiles + 1)
+    const long long walks = causal ? (s.order == kOrderPairs ? (s.grid + cus - 1) / cus * (s.n_tiles + 1)
                                                : std::max<long long>(s.n_tiles, tiles * (s.n_tiles + 1) / 2 / cus))
                                    : (tiles + cus - 1) / cus * s.n_tiles;
     const long long cost = walks * groups * groups * (groups == 8 ? 100 : groups == 4 ? cost4 : cost2);
@@ -766,14 +766,14 @@ hipError_t launch_bwd_t(const void* q, const void* k, const void* v, const void*
                                     : &bwd_dkv_dma_kernel<Tr, D, CAUSAL, 2>;
   hipLaunchKernelGGL(dkv, dim3((unsigned)sk.grid), block, 0, stream, (const uint16_t*)q,
                      (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)dout, ws, (uint16_t*)dk,
-                     (uint16_t*)dv, S, Hq, Hkv, scale, sk.n_tiles, B * Hkv, (int)sk.grid, sk.paired);
+                     (uint16_t*)dv, S, Hq, Hkv, scale, sk.n_tiles, B * Hkv, (int)sk.grid, sk.order);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   const auto dqk = sq.groups == 8 ? &bwd_dq_dma_kernel<Tr, D, CAUSAL, 8>
                                   : &bwd_dq_dma_kernel<Tr, D, CAUSAL, 4>;
   hipLaunchKernelGGL(dqk, dim3((unsigned)sq.grid), block, 0, stream, (const uint16_t*)q,
                      (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)dout, ws, (uint16_t*)dq,
-                     S, Hq, Hkv, scale, sq.n_tiles, B * Hq, (int)sq.grid, sq.paired);
+                     S, Hq, Hkv, scale, sq.n_tiles, B * Hq, (int)sq.grid, sq.order);
   return hipGetLastError();
 }
 

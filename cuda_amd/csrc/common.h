@@ -215,7 +215,7 @@ __device__ __forceinline__ int xcd_remap(int w, int total) {
   return (x < r) ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
 }
 
-// Query tiles of one prefill workgroup (work index after xcd_remap; n_bh =
+// Orders 0 and 1 of prefill_item (work index after xcd_remap; n_bh =
 // B * Hq heads, n_qt tiles per head). Unpaired: one tile; the work index runs
 // over heads and, within a head, over its tiles longest causal walk first.
 // Paired (causal launches, n_qt > 1): tiles n_qt-1-p and p of one head, whose
@@ -250,6 +250,21 @@ __device__ __forceinline__ QTileWork prefill_work(int work, int n_qt, int n_bh, 
       w.qt1 = half;
     }
   }
+  return w;
+}
+// Query tiles of workgroup v of a launch in one of prefill_grid's orders
+// (launch.h). 0 (kOrderHeads): single tiles, head by head; 1 (kOrderPairs):
+// pairs; 2 (kOrderLongest): single tiles, the longest walks of all heads first,
+// where an XCD (v mod 8) keeps its n_bh / 8 heads if 8 divides n_bh.
+__device__ __forceinline__ QTileWork prefill_item(int v, int n_work, int n_qt, int n_bh, int order) {
+  if (order != 2) return prefill_work(xcd_remap(v, n_work), n_qt, n_bh, order);
+  const int sh = n_bh % 8 == 0 ? 3 : 0;
+  const int per = n_bh >> sh, i = v >> sh;
+  QTileWork w;
+  w.bh0 = (v - (i << sh)) * per + i % per;
+  w.qt0 = n_qt - 1 - i / per;
+  w.bh1 = 0;
+  w.qt1 = -1;
   return w;
 }
 

@@ -206,8 +206,8 @@ template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(
     const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
     float* __restrict__ O, float* __restrict__ Lse, int S, int Hq, int Hkv, float scale_log2, int n_qt, int n_bh,
-    int n_work, int paired) {
-  const QTileWork wk = prefill_work(xcd_remap(blockIdx.x, n_work), n_qt, n_bh, paired);
+    int n_work, int order) {
+  const QTileWork wk = prefill_item(blockIdx.x, n_work, n_qt, n_bh, order);
   const int n_pass = wk.qt1 < 0 ? 1 : 2;
 #pragma clang loop unroll(disable)
   for (int pass = 0; pass < n_pass; ++pass) {
@@ -537,17 +537,17 @@ __global__ __launch_bounds__(64 * SplitStage<D>::NW, 1) void prefill_f32_split_k
 //   causal: 27 us against 91; at 192 tiles, not causal, D = 64, 55 against 48);
 // - not causal, D = 128: up to two tiles per CU (32 heads x 1500: 453 -> 354 us);
 //   D = 64 runs two workgroups per CU well (179 us against 195 at 16 x 2048);
-// - causal, too few tiles to pair: the walks differ in length, the split ones
+// - causal, fewer than two pairs of tiles per CU: the walks differ in length, the split ones
 //   do not. D = 128 always (16 heads x 2048: 344 -> 169 us; 256 x 300: 151 ->
 //   112) but for heads of one full tile (256 x 128: 31 against 37), D = 64 where the longest walk is 1.2 times the mean load or more (16 x
 //   2048: 180 -> 105 us; 256 x 300, 1.1 times: 57 against 61).
-static bool f32_splits(long long grid, bool paired, bool causal, int D, int S, long long n_qt,
+static bool f32_splits(long long grid, bool causal, int D, int S, long long n_qt,
                        long long n_bh) {
   const long long cus = device_cus();
   if (4 * grid < 3 * cus) return true;
   if (grid > 0x1fffffff) return false;  // (the split grid is up to twice as large)
   if (!causal) return D == 128 && grid < 2 * cus;
-  if (paired) return false;
+  if (n_qt > 1 && (n_bh * n_qt + 1) / 2 >= 2 * cus) return false;
   if (D == 128) return n_qt > 1 || S <= 64;
   return 10 * 2 * cus > 6 * n_bh * (n_qt + 1);
 }
@@ -558,11 +558,11 @@ static hipError_t launch_prefill_f32_t(const void* q, const void* k, const void*
                                        hipStream_t stream) {
   constexpr int BM = 128;
   const int n_qt = (S + BM - 1) / BM;
-  int paired = 0;
-  const long long grid = prefill_grid(B, Hq, n_qt, CAUSAL, 2, &paired);
+  int order = 0;
+  const long long grid = prefill_grid(B, Hq, n_qt, CAUSAL, 2, &order);
   if (grid == 0) return hipSuccess;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  if (f32_splits(grid, paired, CAUSAL, D, S, n_qt, (long long)B * Hq)) {
+  if (f32_splits(grid, CAUSAL, D, S, n_qt, (long long)B * Hq)) {
     const int n_qb = (S + 31) / 32;
     const bool two = CAUSAL || (long long)B * Hq * n_qb > device_cus();
     const int per_head = two ? (n_qb + 1) / 2 : n_qb;
@@ -574,7 +574,7 @@ static hipError_t launch_prefill_f32_t(const void* q, const void* k, const void*
   }
   hipLaunchKernelGGL((prefill_f32_kernel<D, CAUSAL>), dim3((unsigned)grid), dim3(256), 0, stream,
                      (const float*)q, (const float*)k, (const float*)v, (float*)o, lse, S, Hq, Hkv,
-                     scale * kLog2e, n_qt, B * Hq, (int)grid, paired);
+                     scale * kLog2e, n_qt, B * Hq, (int)grid, order);
   return hipGetLastError();
 }
 

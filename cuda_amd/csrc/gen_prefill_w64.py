@@ -552,7 +552,7 @@ INV = {nm: Sym(nm) for nm in IN_V}
 
 # SGPRs: kernel arguments
 KARG = dict(QP=s(0, 2), KP=s(2, 2), VP=s(4, 2), OP=s(6, 2), LP=s(8, 2), SEQ=s(10), NQT=s(11),
-            NWORK=s(12), PAIRED=s(13), QSHIFT=s(14), SCALE=s(15), NBH=s(16), NFULL=s(17),
+            NWORK=s(12), ORDER=s(13), QSHIFT=s(14), SCALE=s(15), NBH=s(16), NFULL=s(17),
             HALF=s(18), HQ=s(19), HKV=s(20), MNQT=s(21), SHNQT=s(22), MHALF=s(23), SHHALF=s(24),
             MHQ=s(25), SHHQ=s(26), MRATIO=s(27), SHRATIO=s(28), XQ=s(29), XR=s(30))
 globals().update(KARG)
@@ -2169,14 +2169,16 @@ class Gen:
 
     def decode(self, tag):
         """Work item ITEMV -> (BH0, QT0) and (BH1, QT1) (QT1 = -1: no second
-        tile): work = xcd_remap(ITEMV), then prefill_work's pairing."""
+        tile): as prefill_item does (common.h; ORDER 0, 1, 2).
+        In order 2 the host passes the heads of an XCD as HALF and its shift as NFULL."""
         L = lambda n: self.L(f"{n}_{tag}")
         t = T
         out = [S("s_and_b32", t[0], ITEMV, 7), S("s_lshr_b32", t[1], ITEMV, 3), S("s_add_u32", t[2], XQ, 1),
                S("s_mul_i32", t[3], t[0], t[2]), S("s_sub_u32", t[4], t[0], XR), S("s_mul_i32", t[4], t[4], XQ),
                S("s_mul_i32", t[5], XR, t[2]), S("s_add_u32", t[4], t[4], t[5]), S("s_cmp_lt_u32", t[0], XR),
                S("s_cselect_b32", t[3], t[3], t[4]), S("s_add_u32", WORK, t[3], t[1])]
-        out += [S("s_cmp_eq_u32", PAIRED, 0), CBR("s_cbranch_scc1", L("unpaired")),
+        out += [S("s_cmp_eq_u32", ORDER, 0), CBR("s_cbranch_scc1", L("unpaired")),
+                S("s_cmp_eq_u32", ORDER, 2), CBR("s_cbranch_scc1", L("longest")),
                 S("s_cmp_lt_u32", WORK, NFULL), CBR("s_cbranch_scc0", L("pair_tail"))]
         out += div_magic(t[0], WORK, MHALF, SHHALF)
         out += [S("s_mul_i32", t[1], t[0], HALF), S("s_sub_u32", t[1], WORK, t[1]),
@@ -2185,6 +2187,13 @@ class Gen:
         out += [LABEL(L("pair_tail")), S("s_sub_u32", t[0], WORK, NFULL), S("s_lshl_b32", BH0, t[0], 1),
                 S("s_mov_b32", QT0, HALF), S("s_add_u32", BH1, BH0, 1), S("s_mov_b32", QT1, HALF),
                 S("s_cmp_lt_u32", BH1, NBH), CBR("s_cbranch_scc1", L("decoded")), S("s_mov_b32", QT1, -1),
+                BR(L("decoded"))]
+        out += [LABEL(L("longest")), S("s_lshr_b32", WORK, ITEMV, NFULL), S("s_lshl_b32", t[1], WORK, NFULL),
+                S("s_sub_u32", t[2], ITEMV, t[1])]
+        out += div_magic(t[0], WORK, MHALF, SHHALF)
+        out += [S("s_mul_i32", t[1], t[0], HALF), S("s_sub_u32", t[1], WORK, t[1]),
+                S("s_mul_i32", t[2], t[2], HALF), S("s_add_u32", BH0, t[2], t[1]),
+                S("s_sub_u32", QT0, NQT, 1), S("s_sub_u32", QT0, QT0, t[0]), S("s_mov_b32", QT1, -1),
                 BR(L("decoded"))]
         out += [LABEL(L("unpaired"))] + div_magic(t[0], WORK, MNQT, SHNQT)
         out += [S("s_mul_i32", t[1], t[0], NQT), S("s_sub_u32", t[1], WORK, t[1]), S("s_mov_b32", BH0, t[0]),

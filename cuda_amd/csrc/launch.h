@@ -37,7 +37,7 @@ void magic_div(uint32_t d, uint32_t* m, uint32_t* sh);
 // Work decomposition of the 64-row kernels (grid 0: nothing to launch).
 struct PfW64Geom {
   long long grid;
-  int n_qt, n_work, paired, q_shift, n_bh, n_full, half;
+  int n_qt, n_work, order, q_shift, n_bh, n_full, half;
   uint32_t m_nqt, sh_nqt, m_half, sh_half;
   int xcd_q, xcd_r;
 };
@@ -84,17 +84,26 @@ inline int device_cus() {
   return n;
 }
 
-// Workgroups of a prefill launch of n_qt query tiles per (b, h). A causal
-// launch pairs query tiles (prefill_work: n_qt-1-p with p of a head, the
-// middle tiles of an odd n_qt two heads at a time) when the paired grid still
-// gives every workgroup slot of the device at least one workgroup; otherwise
-// each workgroup takes one tile.
-inline long long prefill_grid(int B, int Hq, int n_qt, bool causal, int wg_per_cu, int* paired) {
+// Workgroups of a prefill launch of n_qt query tiles per (b, h), and the order
+// of its tiles (prefill_item). Causal tiles differ in length, so a launch with
+// more of them than workgroup slots pairs them (n_qt-1-p with p of a head, the
+// middle tiles of an odd n_qt two heads at a time: equal work for everyone)
+// where the pairs fill whole rounds of the slots, to a twentieth; otherwise a
+// workgroup takes one tile, the longest of all heads first, and the short ones
+// fill the ends: bf16, head dim 128, 2 x 24 heads x 4096 (384 pairs) 192 -> 175
+// us, 3 x 24 x 2000 (288) 101 -> 79, 1 x 32 x 3000 (192; single tiles head by
+// head before) 85 -> 71, 3 x 12 x 3000 (216) 98 -> 80, but 2 x 32 x 4096 (512)
+// 243 against 237 paired and 1 x 24 x 5127 (252) 137 against 134.
+constexpr int kOrderHeads = 0, kOrderPairs = 1, kOrderLongest = 2;
+inline long long prefill_grid(int B, int Hq, int n_qt, bool causal, int wg_per_cu, int* order) {
   const long long n_bh = (long long)B * Hq;
-  const long long single = n_bh * n_qt;
-  const long long pairs = n_bh * (n_qt / 2) + ((n_qt & 1) ? (n_bh + 1) / 2 : 0);
-  *paired = (causal && n_qt > 1 && pairs >= (long long)device_cus() * wg_per_cu) ? 1 : 0;
-  return *paired ? pairs : single;
+  const long long single = n_bh * n_qt, pairs = (single + 1) / 2;
+  const long long slots = (long long)device_cus() * wg_per_cu;
+  *order = kOrderHeads;
+  if (!causal || n_qt <= 1 || single <= slots) return single;
+  const long long rounds = slots > 0 ? (pairs + slots - 1) / slots : 0;
+  *order = 20 * pairs >= 19 * rounds * slots ? kOrderPairs : kOrderLongest;
+  return *order == kOrderPairs ? pairs : single;
 }
 
 // Split-K geometry of the decode kernels: pages of 16 tokens. The workspace

@@ -738,7 +738,7 @@ struct PfArgs {
 
 template <typename Tr, int D, bool CAUSAL, bool POS>
 __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_dma_kernel(
-    PfArgs a, int S, int Hq, int Hkv, float scale_log2, int n_qt, int n_bh, int n_work, int paired,
+    PfArgs a, int S, int Hq, int Hkv, float scale_log2, int n_qt, int n_bh, int n_work, int order,
     int q_shift) {
   // Work items v = blockIdx.x, + gridDim.x, ... (a persistent launch when the
   // grid is smaller than n_work; gridDim.x is then a multiple of 8, so every
@@ -750,7 +750,7 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_dma_kernel(
   int g0 = 0;  // ring tiles taken by the earlier query tiles
   bool pre = false;
   int v = __builtin_amdgcn_workgroup_id_x(), pass = 0;
-  QTileWork wk = prefill_work(xcd_remap(v, n_work), n_qt, n_bh, paired);
+  QTileWork wk = prefill_item(v, n_work, n_qt, n_bh, order);
 #pragma clang loop unroll(disable)
   for (;;) {
     // the tile after this one: the pair's second, else the next item's first
@@ -759,7 +759,7 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_dma_kernel(
     if (pass2 == 2 || wk.qt1 < 0) {
       v2 = v + (int)gridDim.x;
       pass2 = 0;
-      if (v2 < n_work) wk2 = prefill_work(xcd_remap(v2, n_work), n_qt, n_bh, paired);
+      if (v2 < n_work) wk2 = prefill_item(v2, n_work, n_qt, n_bh, order);
     }
     // Item indices and g0 are uniform; readfirstlane says so (else the
     // compiler may keep them in vector registers and wrap every buffer load
@@ -791,26 +791,26 @@ static hipError_t launch_prefill_kernel(const PfArgs& a, int B, int Hq, int Hkv,
   // wave's causal diagonal still lies in one key tile): the partial tile is
   // the first one, whose causal key walk is the shortest
   const int q_shift = (n_qt * kPfRows - S) / Gm::kBN * Gm::kBN;
-  int paired = 0;
-  const long long n_work = prefill_grid(B, Hq, n_qt, CAUSAL, 1, &paired);
+  int order = 0;
+  const long long n_work = prefill_grid(B, Hq, n_qt, CAUSAL, 1, &order);
   if (n_work == 0) return hipSuccess;
   if (n_work > 0x7fffffffLL) return hipErrorInvalidValue;
   // Items of equal work (non-causal tiles, causal pairs): one workgroup per
   // CU (the ring's LDS admits one) takes items v, v + grid, ..., so a
   // workgroup's next tile streams into the ring behind its current one.
-  // Unpaired causal tiles differ in length and keep one workgroup each,
-  // longest first, for the hardware dispatcher to balance.
+  // Single causal tiles differ in length and keep one workgroup each, for the
+  // hardware dispatcher to balance.
   const long long slots = device_cus() / 8 * 8;
-  const long long grid = ((!CAUSAL || paired) && slots > 0 && n_work > slots) ? slots : n_work;
+  const long long grid = ((!CAUSAL || order == kOrderPairs) && slots > 0 && n_work > slots) ? slots : n_work;
   const float sl2 = scale * kLog2e;
   const dim3 block(64 * kPfWaves);
   if (sl2 >= 0.f) {
     hipLaunchKernelGGL((prefill_dma_kernel<Tr, D, CAUSAL, true>), dim3((unsigned)grid),
-                       block, 0, stream, a, S, Hq, Hkv, sl2, n_qt, B * Hq, (int)n_work, paired,
+                       block, 0, stream, a, S, Hq, Hkv, sl2, n_qt, B * Hq, (int)n_work, order,
                        q_shift);
   } else {
     hipLaunchKernelGGL((prefill_dma_kernel<Tr, D, CAUSAL, false>), dim3((unsigned)grid),
-                       block, 0, stream, a, S, Hq, Hkv, sl2, n_qt, B * Hq, (int)n_work, paired,
+                       block, 0, stream, a, S, Hq, Hkv, sl2, n_qt, B * Hq, (int)n_work, order,
                        q_shift);
   }
   return hipGetLastError();

@@ -37,7 +37,7 @@ struct RowsArgs {
   float* lse;
   int S, Hq, Hkv;
   float scale_log2;
-  int n_qt, n_bh, n_work, paired;
+  int n_qt, n_bh, n_work, order;
 };
 
 template <typename Tr, int D, bool CAUSAL, int QG>
@@ -338,13 +338,7 @@ __device__ CA_INLINE void prefill_rows_tile(const RowsArgs& a, int bh, int qt) {
 template <typename Tr, int D, bool CAUSAL, int QG>
 __global__ __launch_bounds__(64 * kRowsWaves) void prefill_rows_kernel(RowsArgs a) {
   const int wg = __builtin_amdgcn_workgroup_id_x();
-  QTileWork wk = prefill_work(xcd_remap(wg, a.n_work), a.n_qt, a.n_bh, a.paired);
-  if (!a.paired && a.n_bh % 8 == 0) {
-    // single tiles of unequal length: the longest of all the XCD's heads first
-    const int per_xcd = a.n_bh / 8, i = wg / 8;
-    wk.bh0 = (wg % 8) * per_xcd + i % per_xcd;
-    wk.qt0 = a.n_qt - 1 - i / per_xcd;
-  }
+  const QTileWork wk = prefill_item(wg, a.n_work, a.n_qt, a.n_bh, a.order);
   const int n_pass = wk.qt1 < 0 ? 1 : 2;
 #pragma clang loop unroll(disable)
   for (int pass = 0; pass < n_pass; ++pass) {
@@ -372,7 +366,9 @@ hipError_t launch_t(RowsArgs a, int groups, long long grid, hipStream_t stream) 
 //   4       128             17, 12               28
 //   2       128, 256        13, 10.5             39
 // A launch takes its busiest CU's time: tiles in rounds (equal tiles, pairs), or
-// the longest walk or the mean load. Waves share rows where that is estimated a
+// the longest walk or the mean load, with a tenth for its end (2 groups: 45 %,
+// they fetch K and V most often: 12 heads x 3500 x 64, 660 tiles, 38 us against
+// 34 with 4). Waves share rows where that is estimated a
 // tenth or more shorter, as measured for 32/8 heads, one sequence, causal: 333
 // keys 12.3 -> 9.4 us at D = 128, 10.0 -> 7.1 at 64; 1000 keys 23.6 -> 20.5, 18.9
 // -> 13.6; 8 heads of 2500 keys 44.5 -> 28.5, 35.6 -> 17.4; for 2048 keys of 32
@@ -382,22 +378,22 @@ int prefill_rows_groups(int B, int Hq, int S, int D, float scale, bool causal) {
   if (!(sl2 >= 0.f && sl2 <= 3.0e38f)) return 0;
   const double cus = std::max(device_cus(), 1);
   const double bh = (double)B * Hq;
-  auto estimate = [&](int groups, int keys, double step, double tile) {
+  auto estimate = [&](int groups, int keys, double step, double tile, double slack = 1.1) {
     const int rows = 32 * groups, n_qt = (S + rows - 1) / rows;
-    int paired = 0;
-    const double grid = (double)prefill_grid(B, Hq, n_qt, causal, 1, &paired);
+    int order = 0;
+    const double grid = (double)prefill_grid(B, Hq, n_qt, causal, 1, &order);
     auto walk = [&](int n) { return tile + step * ((n + keys - 1) / keys); };
     const double longest = walk(S);
     if (!causal) return std::ceil(grid / cus) * longest;
     // the mean of a causal tile's steps: half the longest's and a half step
     const double mean = tile + step * (0.5 * S / keys + 0.5);
-    if (paired) return std::ceil(grid / cus) * 2 * mean;
-    return std::max(longest, 1.1 * bh * n_qt * mean / cus);
+    if (order == kOrderPairs) return std::ceil(grid / cus) * 2 * mean;
+    return std::max(longest, slack * bh * n_qt * mean / cus);
   };
   const bool d64 = D == 64;
   const double base = estimate(8, 64, d64 ? 9 : 11, 30);
   const double four = estimate(4, 128, d64 ? 12 : 17, 28);
-  const double two = estimate(2, d64 ? 256 : 128, d64 ? 10.5 : 13, 39);
+  const double two = estimate(2, d64 ? 256 : 128, d64 ? 10.5 : 13, 39, 1.45);
   if (std::min(four, two) > 0.9 * base) return 0;
   return two < four ? 2 : 4;
 }
@@ -408,7 +404,7 @@ hipError_t launch_prefill_rows(int groups, bool f16, const void* q, const void* 
   RowsArgs a{(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o, lse, S, Hq,
              Hkv, scale * kLog2e, 0, B * Hq, 0, 0};
   a.n_qt = (S + 32 * groups - 1) / (32 * groups);
-  const long long grid = prefill_grid(B, Hq, a.n_qt, causal, 1, &a.paired);
+  const long long grid = prefill_grid(B, Hq, a.n_qt, causal, 1, &a.order);
   if (grid == 0) return hipSuccess;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
   a.n_work = (int)grid;

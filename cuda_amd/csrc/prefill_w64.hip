@@ -9,10 +9,10 @@
 // dims and element types).
 //
 // Work decomposition: one query tile = 256 rows of one (b, h), taken by the
-// 4 waves of a workgroup (64 rows each); causal launches pair query tiles n-1-p
-// and p of a head; with more items than CUs one workgroup per CU takes items
-// g, g + grid, ... (prefill_work, xcd_remap in common.h, restated in the
-// kernel body with magic-number divisions). K and V tiles of 64 keys travel
+// 4 waves of a workgroup (64 rows each), in prefill_grid's order; of equal
+// items (pairs, non-causal tiles), where there are more than CUs, one workgroup
+// per CU takes items g, g + grid, ... (prefill_item in common.h, restated in
+// the kernel body with magic-number divisions). K and V tiles of 64 keys travel
 // HBM -> LDS by buffer loads into two rings of 4 tiles (K tile t is read by
 // QK in iteration t - 1, V tile t by PV in iteration t + 1, so the rings
 // release their slots at different times), every wave loading a quarter of
@@ -56,7 +56,7 @@ struct PfW64Args {
   const void* v;
   void* o;
   float* lse;
-  int S, n_qt, n_work, paired, q_shift;
+  int S, n_qt, n_work, order, q_shift;
   float scale_log2;
   int n_bh, n_full, half, hq, hkv;
   // x / d = (x * m) >> sh for 0 <= x < 2^31 (magic division), per divisor
@@ -156,16 +156,20 @@ hipError_t w64_geometry(int B, int Hq, int S, bool causal, PfW64Geom* g) {
   // padding rows of a ragged S go before row 0, in whole key tiles, so every
   // wave's causal diagonal is its last key tile
   g->q_shift = (n_qt * kRows - S) / kBN * kBN;
-  const long long n_work = prefill_grid(B, Hq, n_qt, causal, 1, &g->paired);
+  const long long n_work = prefill_grid(B, Hq, n_qt, causal, 1, &g->order);
   if (n_work == 0) return hipSuccess;
   if (n_work > 0x7fffffffLL || (long long)B * Hq > 0x7fffffffLL) return hipErrorInvalidValue;
   const long long slots = device_cus() / 8 * 8;
-  g->grid = ((!causal || g->paired) && slots > 0 && n_work > slots) ? slots : n_work;
+  g->grid = ((!causal || g->order == kOrderPairs) && slots > 0 && n_work > slots) ? slots : n_work;
   g->n_qt = n_qt;
   g->n_work = (int)n_work;
   g->n_bh = B * Hq;
   g->half = n_qt >> 1;
   g->n_full = g->n_bh * g->half;
+  if (g->order == kOrderLongest) {  // what the body's decode takes here: heads per XCD, their shift
+    g->n_full = g->n_bh % 8 == 0 ? 3 : 0;
+    g->half = g->n_bh >> g->n_full;
+  }
   magic_div((uint32_t)n_qt, &g->m_nqt, &g->sh_nqt);
   magic_div((uint32_t)(g->half > 0 ? g->half : 1), &g->m_half, &g->sh_half);
   g->xcd_q = (int)(n_work / 8);
@@ -188,7 +192,7 @@ hipError_t launch_prefill_w64(bool f16, const void* q, const void* k, const void
   a.S = S;
   a.n_qt = g.n_qt;
   a.n_work = g.n_work;
-  a.paired = g.paired;
+  a.order = g.order;
   a.q_shift = g.q_shift;
   a.scale_log2 = scale * kLog2e;
   a.n_bh = g.n_bh;

@@ -41,7 +41,7 @@ struct PfW64MxArgs {
   const void* v;
   void* o;
   const void* qs;
-  int S, n_qt, n_work, paired, q_shift;
+  int S, n_qt, n_work, order, q_shift;
   float scale_log2;
   int n_bh, n_full, half, hq, unused0;
   uint32_t m_nqt, sh_nqt, m_half, sh_half;
@@ -140,7 +140,7 @@ hipError_t launch_prefill_w64_mx(bool out_f16, const uint8_t* q, const uint8_t* 
   a.S = S;
   a.n_qt = g.n_qt;
   a.n_work = g.n_work;
-  a.paired = g.paired;
+  a.order = g.order;
   a.q_shift = g.q_shift;
   a.scale_log2 = scale * kLog2e;
   a.n_bh = g.n_bh;

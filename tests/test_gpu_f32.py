@@ -264,3 +264,20 @@ def test_fp8_paged_f32_nan_tail_does_not_leak(dev):
                                                case["context_lens"])
     torch.cuda.synchronize()
     assert_close(to_np(out), ref, **TOL_F32, name="fp8 paged f32 nan tail")
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("b,h,s", [(1, 203, 600), (8, 32, 300), (3, 43, 600)])
+def test_causal_tile_orders_f32(dev, head_dim, b, h, s):
+    """508 pairs of 128-row tiles (two workgroups per CU), middle tiles and a
+    lone one; 768 and 645 single tiles, the longest of all heads first. Row 0 of
+    every head is V's row 0, sampled heads against the oracle."""
+    q, k, v = qkv(b, h, s, head_dim, F32, dev)
+    out = cuda_llm.flash_attention(q, k, v, is_causal=True)
+    torch.cuda.synchronize()
+    assert torch.isfinite(out).all()
+    assert (out[:, :, 0] - v[:, :, 0]).abs().max().item() <= 1e-5
+    for bi, hi in ((0, 0), (b - 1, h - 1)):
+        sel = [to_np(t[bi:bi + 1, hi:hi + 1]) for t in (q, k, v)]
+        ref = oracle.attention(*sel, is_causal=True, dtype=np.float64)
+        assert_close(to_np(out[bi:bi + 1, hi:hi + 1]), ref, **TOL_F32, name=f"head {bi},{hi}")

@@ -265,3 +265,19 @@ def test_mx_scale_check_opt_in(dev, monkeypatch):
     monkeypatch.setenv("CUDA_LLM_CHECK_MX_SCALES", "1")
     with pytest.raises(RuntimeError, match="powers of two"):
         cuda_llm.fused_microscaled_attention(x["q"], f32[0], x["k"], f32[1], x["v"], f32[2], is_causal=True)
+
+
+@pytest.mark.parametrize("b,h,s", [(1, 101, 1200), (3, 12, 2300), (4, 16, 1500)])
+def test_mx_causal_tile_orders(dev, b, h, s):
+    """253 pairs of 256-row tiles; single tiles, the longest of all heads first,
+    for head counts that 8 does not and does divide: row 0 of every head is
+    V's row 0, sampled heads against the oracle."""
+    x = mx_inputs(b, h, s, 128, dev, seed=s)
+    out = _run(x, True)
+    torch.cuda.synchronize()
+    v0 = oracle.mx_dequantize(x["v"][:, :, :1].cpu().numpy(), x["v_scale"][:, :, :1].cpu().numpy())
+    assert_close(to_np(out[:, :, :1]), v0, **TOL_FP8, name="row 0")
+    for heads in ((0, 0), (b - 1, h - 1)):
+        d = _ref(x, heads)
+        ref = oracle.attention(d["q"], d["k"], d["v"], is_causal=True)
+        assert_close(to_np(out[heads[0]:heads[0] + 1, heads[1]:heads[1] + 1]), ref, **TOL_FP8, name=f"head {heads}")

@@ -374,3 +374,38 @@ def test_short_sequences_full_grid(dev, s, jump, is_causal, d):
         ref = oracle.attention(to_np(q[bi:bi + 1, hi:hi + 1]), to_np(k[bi:bi + 1, hi // 2:hi // 2 + 1]),
                                to_np(v[bi:bi + 1, hi // 2:hi // 2 + 1]), is_causal=is_causal)
         assert_close(to_np(out[bi:bi + 1, hi:hi + 1]), ref, **TOL_16BIT, name=f"head {bi},{hi}")
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("b,hq,hkv,s", [
+    (7, 29, 29, 1200),  # 508 pairs of 256-row tiles, two rounds of 256: middle tiles, a lone one
+    (7, 29, 1, 1088),   # the same with a first tile of 64 rows
+    (3, 24, 4, 1000),   # 288 single tiles, longest first, nine heads per XCD
+    (3, 12, 12, 2200),  # 324, 36 heads over all XCDs
+    (1, 257, 257, 300),  # 514, an odd count of heads
+    (1, 12, 4, 3500),   # 336 tiles of 128 rows (head dim 64)
+    (1, 32, 8, 1500),   # 384 tiles of 128 rows
+])
+def test_causal_tile_orders(dev, b, hq, hkv, s, d):
+    """Causal launches in the orders of their tiles on 256 CUs: pairs where
+    they fill rounds of the device, else single tiles, the longest of all heads
+    first. O and LSE of sampled heads against the oracle, every row written."""
+    import cuda_amd._lib as L
+    from cuda_amd.api import _ptr, _stream
+    dtype = torch.float16 if d == 64 else torch.bfloat16
+    q, k, v = qkv(b, hq, s, d, dtype, dev, hkv=hkv, gen=torch.Generator(device=dev).manual_seed(s))
+    out = torch.full_like(q, float("nan"))
+    lse = torch.full((b, hq, s), float("nan"), device=dev)
+    L.call("ca_flash_attention_fwd_lse", L.CA_F16 if d == 64 else L.CA_BF16, _ptr(q), _ptr(k), _ptr(v),
+           _ptr(out), _ptr(lse), b, hq, hkv, s, d, 0.1, 1, _stream())
+    torch.cuda.synchronize()
+    assert torch.isfinite(out).all() and torch.isfinite(lse).all()
+    kv0 = v[:, :, 0].float().repeat_interleave(hq // hkv, dim=1)
+    assert (out[:, :, 0].float() - kv0).abs().max().item() <= 1e-2
+    for bi, hi in ((0, 0), (b - 1, hq - 1)):
+        kh = hi // (hq // hkv)
+        args = [to_np(q[bi:bi + 1, hi:hi + 1]), to_np(k[bi:bi + 1, kh:kh + 1])]
+        ref = oracle.attention(*args, to_np(v[bi:bi + 1, kh:kh + 1]), is_causal=True, scale=0.1)
+        assert_close(to_np(out[bi:bi + 1, hi:hi + 1]), ref, **TOL_16BIT, name=f"head {bi},{hi}")
+        lref = oracle.attention_lse(*args, is_causal=True, scale=0.1, dtype=np.float64)
+        assert np.abs(to_np(lse[bi:bi + 1, hi:hi + 1]) - lref).max() <= 1e-3
