@@ -155,7 +155,8 @@ hipError_t launch_kv_append(int dtype, int kind, const void* key, const void* va
                             const int32_t* context_lens, const int32_t* new_lens, int N, int Hkv,
                             int D, int T, int max_blocks, int num_blocks, hipStream_t stream);
 
-// RoPE + prefill (rope.hip): q and k rotated into ws, then launch_prefill.
+// RoPE + prefill (rope.hip): k rotated into ws, q into o (float32: into ws),
+// then launch_prefill.
 size_t rope_workspace_bytes(int dtype, int B, int Hq, int Hkv, int S, int D);
 hipError_t launch_rope_prefill(int dtype, const void* q, const void* k, const void* v,
                                const float* cos_tab, const float* sin_tab, void* o, int B, int Hq,
