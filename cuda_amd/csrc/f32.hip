@@ -10,8 +10,9 @@
 // Two kernels. prefill_f32_kernel: one workgroup = 4 waves x 32 query rows of
 // one (b, h); K/V tiles of 32 keys, double-buffered in LDS (register-staged
 // loads, one barrier per tile). prefill_f32_split_kernel (few or unequal tiles,
-// f32_splits): one workgroup per pair of 32-row query blocks, its 4 waves splitting the pair's key tiles and merging their softmax states
-// (described at the kernel). Per wave and tile, both on
+// f32_splits): one workgroup per pair of 32-row query blocks, its 4 waves
+// splitting the pair's key tiles and merging their softmax states (described
+// at the kernel). Per wave and tile, both on
 // v_mfma_f32_32x32x2_f32 (one fp32 element of each operand per lane,
 // k = lane / 32):
 //   S^T[32 keys x 32 q] = K Q^T   over D/2 steps; lane half h contracts
@@ -222,9 +223,9 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(
 // Small grids: the key walk of one 32-row query block split over the waves
 // of a workgroup.
 //
-// When (b, h) x 128-row tiles would not give every CU a workgroup (BASELINE
-// C1: 16 heads x 8 tiles = 128 workgroups on 256 CUs, the longest walking 32
-// key tiles on each SIMD), a workgroup takes one 32-row query block and its
+// When (b, h) x 128-row tiles would not give every CU a workgroup (2 x 8 heads
+// x 1024: 128 workgroups on 256 CUs, the longest walking 32 key tiles on each
+// SIMD), a workgroup takes one 32-row query block and its
 // four waves (one per SIMD) take key tiles w, w + 4, ... of it, each with its
 // own online-softmax state; the states are merged through LDS at the end (O =
 // sum_w a_w O_w / sum_w a_w l_w with a_w = 2^(m_w - max m)). Causal launches
