@@ -18,7 +18,8 @@ constexpr int kDtypeF16 = 1;
 constexpr int kDtypeBF16 = 2;
 
 // Prefill; lse (may be null) receives the natural-log row logsumexp [B, Hq, S].
-// q may be o itself (16-bit: every row is read as Q before it is written).
+// q may be o itself (16-bit: a workgroup reads Q rows of the tiles that it
+// writes only, each before it writes that row).
 hipError_t launch_prefill(int dtype, const void* q, const void* k, const void* v, void* o,
                           float* lse, int B, int Hq, int Hkv, int S, int D, float scale,
                           bool causal, hipStream_t stream);

@@ -161,11 +161,11 @@ __device__ CA_INLINE bool prefill_dma_qtile(const void* Qv, const void* __restri
 
   // Q as the B operand of S^T = K Q^T: qv, k-step ks: d = 16 ks + 8 hl +
   // [0, 8). Loaded after the first K/V tiles' loads, so that
-  // their latencies overlap: the lane's row of tile (bx, qtx), row 0 for
-  // rows outside [0, S) ...
+  // their latencies overlap: the lane's row of tile (bx, qtx), the nearest
+  // row (of the same tile: q may be o itself) for rows outside [0, S) ...
   auto load_q_raw = [&](int bx, int qtx) CA_INLINE {
     const int r = qtx * kBM - q_shift + wave * 32 + l32;
-    const size_t row = (size_t)bx * S + ((r >= 0 && r < S) ? r : 0);
+    const size_t row = (size_t)bx * S + min(max(r, 0), S - 1);
     const uint16_t* Qr = (const uint16_t*)Qv + row * D;
 #pragma unroll
     for (int ks = 0; ks < Gv::kNKS; ++ks) qv[ks] = *(const vec8*)(Qr + 16 * ks + 8 * hl);

@@ -106,10 +106,12 @@ __device__ CA_INLINE void prefill_rows_tile(const RowsArgs& a, int bh, int qt) {
 #pragma unroll
   for (int g = 0; g < kGroups - 1; ++g) issue(g);
 
-  // Q as the B operand of S^T = K Q^T: k-step ks holds d = 16 ks + 8 hl + [0, 8)
+  // Q as the B operand of S^T = K Q^T: k-step ks holds d = 16 ks + 8 hl + [0, 8).
+  // Lanes past S take row S - 1 of their own tile, whose vote in the tiles below
+  // is that row's (q may be o itself: other tiles' rows may be written already).
   vec8 qv[kNKS];
   {
-    const uint16_t* Qr = a.q + ((size_t)bh * S + (q_in ? myq : 0)) * D;
+    const uint16_t* Qr = a.q + ((size_t)bh * S + min(myq, S - 1)) * D;
 #pragma unroll
     for (int ks = 0; ks < kNKS; ++ks) qv[ks] = *(const vec8*)(Qr + 16 * ks + 8 * hl);
   }

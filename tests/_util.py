@@ -146,3 +146,41 @@ def balanced_walk_taken(n, hq, hkv, d, max_blocks, fp8):
     sk = 2 * grid * min(16, hq // hkv) * (d + 1) * 4 + 4 * n
     contract = n * hq * (-(-max_blocks // 64)) * (d + 1) * 4
     return max_blocks > split_pages and n <= 1024 and sk <= contract
+
+
+def prefill_order(b, hq, n_qt, causal):
+    """(grid, order) of a 16-bit prefill launch of n_qt query tiles per head
+    (prefill_grid in launch.h, one workgroup per CU): order "pairs" or
+    "longest" for causal launches of more tiles than CUs, else "heads"."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    single = b * hq * n_qt
+    pairs = (single + 1) // 2
+    if not causal or n_qt <= 1 or single <= cus:
+        return single, "heads"
+    return (pairs, "pairs") if 20 * pairs >= 19 * -(-pairs // cus) * cus else (single, "longest")
+
+
+def prefill_rows_groups(b, hq, s, d, causal):
+    """The rule of prefill_rows.hip for scale >= 0 (prefill_rows_groups there):
+    32-row groups per workgroup, 2 or 4, where waves share rows; 0 where the
+    256-row kernels run (head dim 128: the 64-row kernel)."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+
+    def estimate(groups, keys, step, tile, slack=1.1):
+        n_qt = -(-s // (32 * groups))
+        grid, order = prefill_order(b, hq, n_qt, causal)
+        longest = tile + step * -(-s // keys)
+        if not causal:
+            return math.ceil(grid / cus) * longest
+        mean = tile + step * (0.5 * s / keys + 0.5)
+        if order == "pairs":
+            return math.ceil(grid / cus) * 2 * mean
+        return max(longest, slack * b * hq * n_qt * mean / cus)
+
+    d64 = d == 64
+    base = estimate(8, 64, 9 if d64 else 11, 30)
+    four = estimate(4, 128, 12 if d64 else 17, 28)
+    two = estimate(2, 256 if d64 else 128, 10.5 if d64 else 13, 39, 1.45)
+    if min(four, two) > 0.9 * base:
+        return 0
+    return 2 if two < four else 4

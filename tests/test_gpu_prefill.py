@@ -14,7 +14,7 @@ import torch
 
 import cuda_llm
 import oracle
-from _util import TOL_16BIT, assert_close, qkv, to_np
+from _util import TOL_16BIT, assert_close, prefill_rows_groups, qkv, to_np
 
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "golden.npz")
@@ -351,6 +351,30 @@ def test_shared_row_waves(dev, b, hq, hkv, s, is_causal, d):
         assert_close(to_np(out[bi:bi + 1, hi:hi + 1]), ref, **TOL_16BIT, name=f"head {bi},{hi}")
         lref = oracle.attention_lse(*args, is_causal=is_causal, scale=0.1, dtype=np.float64)
         assert np.abs(to_np(lse[bi:bi + 1, hi:hi + 1]) - lref).max() <= 1e-3
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("is_causal", [False, True])
+def test_shared_row_waves_lanes_past_the_end(dev, dtype, d, is_causal):
+    """The last 32-row group of a length that 32 does not divide has lanes
+    without a row: row 0 of the head, whose logits pass the stale max at every
+    tile here, must not reach the bits of the group's rows."""
+    b, h, s = 1, 8, 1000
+    assert prefill_rows_groups(b, h, s, d, is_causal) > 0
+    g = torch.Generator(device=dev).manual_seed(3)
+    u = torch.randn(d, device=dev, generator=g)
+    u = u / u.norm()
+    rows, noise, v = (torch.randn(b, h, s, d, device=dev, generator=g) for _ in range(3))
+    rows -= (rows @ u)[..., None] * u
+    k = (0.5 * torch.arange(s, device=dev)[:, None] * u + 0.1 * noise).to(dtype)
+    q, v = rows.to(dtype), v.to(dtype)
+    q0 = q.clone()
+    q0[:, :, 0] = (8 * u).to(dtype)
+    a = cuda_llm.flash_attention(q, k, v, is_causal=is_causal)
+    c = cuda_llm.flash_attention(q0, k, v, is_causal=is_causal)
+    torch.cuda.synchronize()
+    assert torch.equal(a[:, :, s // 32 * 32:], c[:, :, s // 32 * 32:])
 
 
 @pytest.mark.parametrize("d", [64, 128])

@@ -12,7 +12,7 @@ import torch
 
 import cuda_llm
 import oracle
-from _util import TOL_16BIT, assert_close, qkv, to_np
+from _util import TOL_16BIT, assert_close, prefill_rows_groups, qkv, to_np
 
 pytestmark = pytest.mark.gpu
 TOL_F32 = dict(max_abs=1e-4, mean_abs=1e-5)
@@ -74,6 +74,26 @@ def test_rope_identity_tables_equal_flash_attention(dev, dtype, d):
         assert_close(to_np(a), to_np(b), **TOL_16BIT, name="identity rope")
     else:
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("is_causal", [False, True])
+def test_rope_ragged_is_reproducible(dev, d, is_causal):
+    """16-bit q is rotated into the output, which the prefill reads as Q: with
+    lanes past S in the last row group (S = 1000, waves sharing rows) equal
+    calls still give equal bits, also where a row's logits outgrow the running
+    max in every tile."""
+    s = 1000
+    assert prefill_rows_groups(1, 8, s, d, is_causal) > 0
+    q, k, v = qkv(1, 8, s, d, torch.bfloat16, dev)
+    q[:, :, 0] = 8
+    k += 0.05 * torch.arange(s, device=dev, dtype=k.dtype)[:, None]
+    cos, sin = torch.ones(s, d, device=dev), torch.zeros(s, d, device=dev)
+    want = cuda_llm.flash_attention(q, k, v, is_causal=is_causal)
+    for _ in range(3):
+        out = cuda_llm.fused_rope_flash_attention(q, k, v, cos, sin, is_causal=is_causal)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
 
 
 def test_rope_rejects_bad_tables(dev):
