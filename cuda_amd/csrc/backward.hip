@@ -155,6 +155,9 @@ constexpr int dkv_stages() {
 struct TrOfs {
   uint32_t a, b;
 };
+struct TrHalves {
+  u32x2 lo, hi;
+};
 template <int D>
 struct Geom {
   static constexpr int kRowB = 2 * D;        // bytes per row
@@ -189,12 +192,19 @@ struct Geom {
     t.b = (row + 4) * kRowB + 16 * (c0 ^ swz(row + 4)) + 8 * (s16 & 1);
     return t;
   }
-  // A operand (32 dims x 16 rows) of k-step kk of a tile at `base`, dims block ob.
-  template <typename Tr, int KK>
-  __device__ static __forceinline__ typename Tr::vec8 tr_operand(uint32_t base, TrOfs t, int ob) {
-    const u32x2 lo = lds_read_tr16<16 * kRowB * KK>((base + t.a) ^ (64 * ob));
-    const u32x2 hi = lds_read_tr16<16 * kRowB * KK>((base + t.b) ^ (64 * ob));
-    const u32x4 w = {lo[0], lo[1], hi[0], hi[1]};
+  // A operand (32 dims x 16 rows) of k-step KK of a tile at `base`, dims block
+  // ob: its halves' reads, and after their wait the operand (joining them
+  // earlier could copy registers that a read in flight has yet to write).
+  template <int KK>
+  __device__ static __forceinline__ TrHalves tr_read(uint32_t base, TrOfs t, int ob) {
+    return {lds_read_tr16<16 * kRowB * KK>((base + t.a) ^ (64 * ob)),
+            lds_read_tr16<16 * kRowB * KK>((base + t.b) ^ (64 * ob))};
+  }
+  template <typename Tr>
+  __device__ static __forceinline__ typename Tr::vec8 tr_operand(TrHalves& h) {
+    after_wait(h.lo);
+    after_wait(h.hi);
+    const u32x4 w = {h.lo[0], h.lo[1], h.hi[0], h.hi[1]};
     return __builtin_bit_cast(typename Tr::vec8, w);
   }
 };
@@ -386,12 +396,10 @@ __device__ CA_INLINE void bwd_dq_dma_tile(const uint16_t* __restrict__ Q,
     // dQ^T[d x q] += K^T[d x keys] dS^T[keys x q]
 #pragma unroll
     for (int ob = 0; ob < kNOB; ++ob) {
-      const vec8 a0 = Gm::template tr_operand<Tr, 0>(hb, tofs, ob);
-      const vec8 a1 = Gm::template tr_operand<Tr, 1>(hb, tofs, ob);
+      TrHalves h0 = Gm::template tr_read<0>(hb, tofs, ob);
+      TrHalves h1 = Gm::template tr_read<1>(hb, tofs, ob);
       wait_lgkm<0>();
-      vec8 x0 = a0, x1 = a1;
-      after_wait(x0);
-      after_wait(x1);
+      const vec8 x0 = Gm::template tr_operand<Tr>(h0), x1 = Gm::template tr_operand<Tr>(h1);
       acc[ob] = Tr::mfma32(x0, pb[0], acc[ob]);
       acc[ob] = Tr::mfma32(x1, pb[1], acc[ob]);
     }
@@ -640,16 +648,13 @@ __device__ CA_INLINE void bwd_dkv_dma_tile(const uint16_t* __restrict__ Q,
     // dV^T[d x keys] += dO^T P and dK^T[d x keys] += Q^T dS
 #pragma unroll
     for (int ob = 0; ob < kNOB; ++ob) {
-      const vec8 g0 = Gm::template tr_operand<Tr, 0>(sb + kTileB, tofs, ob);
-      const vec8 g1 = Gm::template tr_operand<Tr, 1>(sb + kTileB, tofs, ob);
-      const vec8 x0 = Gm::template tr_operand<Tr, 0>(sb, tofs, ob);
-      const vec8 x1 = Gm::template tr_operand<Tr, 1>(sb, tofs, ob);
+      TrHalves g0 = Gm::template tr_read<0>(sb + kTileB, tofs, ob);
+      TrHalves g1 = Gm::template tr_read<1>(sb + kTileB, tofs, ob);
+      TrHalves h0 = Gm::template tr_read<0>(sb, tofs, ob);
+      TrHalves h1 = Gm::template tr_read<1>(sb, tofs, ob);
       wait_lgkm<0>();
-      vec8 a0 = g0, a1 = g1, b0 = x0, b1 = x1;
-      after_wait(a0);
-      after_wait(a1);
-      after_wait(b0);
-      after_wait(b1);
+      const vec8 a0 = Gm::template tr_operand<Tr>(g0), a1 = Gm::template tr_operand<Tr>(g1);
+      const vec8 b0 = Gm::template tr_operand<Tr>(h0), b1 = Gm::template tr_operand<Tr>(h1);
       acc[kNOB + ob] = Tr::mfma32(a0, pp[0], acc[kNOB + ob]);
       acc[ob] = Tr::mfma32(b0, pd[0], acc[ob]);
       acc[kNOB + ob] = Tr::mfma32(a1, pp[1], acc[kNOB + ob]);
