@@ -378,8 +378,14 @@ __device__ __forceinline__ void dma_walk(const typename Tr::vec8 (&qv)[D / 32], 
     if (wave_any(need)) {
       const float m_new = __builtin_fmaxf(m_run, tmax);
       const float alpha = (m_new == kNegInf) ? 1.f : fast_exp2(m_run - m_new);
+      if (wave_any(m_run != kNegInf)) {  // (in a walk's first step o is zero)
+        // m, l and alpha are head l16's; row r of o is head 4 grp + r
+        f32x4 alpha_o;
 #pragma unroll
-      for (int i = 0; i < NB; ++i) o[i] *= alpha;
+        for (int r = 0; r < 4; ++r) alpha_o[r] = __shfl(alpha, 4 * grp + r, 64);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) o[i] *= alpha_o;
+      }
       l_run *= alpha;
       m_run = m_new;
     }

@@ -38,7 +38,7 @@ def qkv(b, hq, s, d, dtype, device, hkv=None, gen=None):
 
 
 def build_paged(lens, hq, hkv, d, dtype, device, fp8=False, per_block=True, pool=None,
-                page=16, seed=0):
+                page=16, seed=0, edit=None):
     """Paged GQA decode inputs in the reference layout [blocks, Hkv, D, page].
 
     A pool of ``pool`` pages (default: exactly the pages needed) ~N(0,1) is
@@ -46,6 +46,8 @@ def build_paged(lens, hq, hkv, d, dtype, device, fp8=False, per_block=True, pool
     random permutation of the pool (tests/_utils.py:105-133 generalised to a
     shared pool and GQA). FP8: per-(page, kv-head) scale amax/448 (or one per
     kv head if ``per_block`` is False) and e4m3 codes (tests/test_kernels_misc.py:52-55).
+    ``edit(q, kf, tables)`` may change the float queries and keys before they are
+    converted.
     """
     g = torch.Generator(device=device)
     g.manual_seed(seed)
@@ -61,10 +63,12 @@ def build_paged(lens, hq, hkv, d, dtype, device, fp8=False, per_block=True, pool
         if p:
             tables[i, :p] = perm[cur:cur + p]
         cur += p
-    q = torch.randn(n, hq, d, device=device, generator=g).to(dtype)
+    q = torch.randn(n, hq, d, device=device, generator=g)
     kf = torch.randn(pool, hkv, d, page, device=device, generator=g)
     vf = torch.randn(pool, hkv, d, page, device=device, generator=g)
-    case = dict(query=q, block_tables=tables,
+    if edit is not None:
+        edit(q, kf, tables)
+    case = dict(query=q.to(dtype), block_tables=tables,
                 context_lens=torch.tensor(lens, dtype=torch.int32, device=device))
     if not fp8:
         case.update(key_cache=kf.to(dtype), value_cache=vf.to(dtype))

@@ -14,6 +14,7 @@
   ragged and empty contexts, a context cut into more partials than the merge
   loads at once (and more than 64), fewer pages than waves, GQA groups above
   16, head dim 64, both cache kinds and scale forms;
+* logits that grow along the context, on every walk;
 * the committed golden vectors.
 """
 import os
@@ -302,6 +303,78 @@ def test_flash_decode_waves_and_splits(dev, head_dim, b, hq, hkv, kv_len):
     torch.cuda.synchronize()
     assert_close(to_np(out), oracle.attention(to_np(q), to_np(k), to_np(v)), **TOL_16BIT,
                  name=f"decode {kv_len}")
+
+
+def _growing(hkv, group, d, tokens, profile, dev):
+    """Queries [Hkv, G, D] and keys [Hkv, tokens, D] whose logits grow along the
+    tokens, each head of a group at its own: "ramp", by up to half a nat a token
+    from a start of the head's, and "jump", by about 90 nats at one token."""
+    g = torch.Generator(device=dev).manual_seed(group)
+    u = torch.randn(hkv, group, d, device=dev, generator=g)
+    u = u / u.norm(dim=-1, keepdim=True)
+    t = torch.arange(tokens, device=dev, dtype=torch.float32)
+    h = torch.arange(group, device=dev, dtype=torch.float32)[:, None]
+    if profile == "ramp":
+        amp = 0.5 * (t - 29 * h).clamp(0, 1500)
+    else:
+        amp = torch.where(t >= tokens * (h + 1) / (group + 2), 130.0, 1.0)
+    k = torch.einsum("gt,hgd->htd", amp, u) + 0.1 * torch.randn(hkv, tokens, d, device=dev, generator=g)
+    return 8 * u + 0.1 * torch.randn(hkv, group, d, device=dev, generator=g), k
+
+
+@pytest.mark.parametrize("profile", ["ramp", "jump"])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("n,hkv,group,width", [
+    (140, 4, 4, 16),    # one wave walks 16 pages
+    (66, 4, 1, 40),     # four waves, ten pages each
+    (6, 2, 16, 64),     # eight waves, eight pages each
+    (64, 8, 4, 512),    # the balanced walk
+])
+def test_paged_running_max_growth(dev, n, hkv, group, width, head_dim, fp8, profile):
+    """Maxima that grow after a wave's first step, by head: the rescale of the
+    accumulator rows is each head's own."""
+    q, k = _growing(hkv, group, head_dim, 16 * width, profile, dev)
+    page = k.view(hkv, width, 16, head_dim).permute(1, 0, 3, 2)
+
+    def edit(qf, kf, tables):
+        qf[:] = q.reshape(hkv * group, head_dim)
+        for i in range(n):
+            kf[tables[i].long()] = page
+
+    lens = [16 * width - 5 * i % (8 * width) for i in range(n)]
+    dtype = torch.float16 if head_dim == 64 else torch.bfloat16
+    case = build_paged([16 * width] * n, hkv * group, hkv, head_dim, dtype, dev, fp8=fp8, edit=edit)
+    case["context_lens"].copy_(torch.tensor(lens))
+    assert balanced_walk_taken(n, hkv * group, hkv, head_dim, width, fp8) == (width == 512)
+    out = _run_paged(case)
+    torch.cuda.synchronize()
+    assert torch.isfinite(out).all()
+    seqs = sorted({0, 1, n // 2, n - 1})
+    assert_close(to_np(out)[seqs], paged_oracle(case, seqs), **(TOL_FP8 if fp8 else TOL_16BIT), name=profile)
+
+
+@pytest.mark.parametrize("profile", ["ramp", "jump"])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("b,hkv,group,kv_len", [
+    (260, 2, 4, 250),   # one wave
+    (129, 2, 1, 300),   # four waves
+    (8, 32, 1, 1024),   # eight waves
+    (1, 2, 16, 5000),   # splits
+])
+def test_flash_decode_running_max_growth(dev, b, hkv, group, kv_len, head_dim, profile):
+    """The same over the contiguous cache."""
+    q, k = _growing(hkv, group, head_dim, kv_len, profile, dev)
+    dtype = torch.float16 if head_dim == 64 else torch.bfloat16
+    q = q.reshape(1, hkv * group, 1, head_dim).expand(b, -1, -1, -1).to(dtype).contiguous()
+    k = k.expand(b, -1, -1, -1).to(dtype).contiguous()
+    v = torch.randn(b, hkv, kv_len, head_dim, device=dev).to(dtype)
+    out = cuda_llm.flash_decode(q, k, v)
+    torch.cuda.synchronize()
+    assert torch.isfinite(out).all()
+    for i in (0, b - 1):
+        ref = oracle.attention(to_np(q[i:i + 1]), to_np(k[i:i + 1]), to_np(v[i:i + 1]))
+        assert_close(to_np(out[i:i + 1]), ref, **TOL_16BIT, name=profile)
 
 
 @pytest.mark.parametrize("fp8", [False, True])
