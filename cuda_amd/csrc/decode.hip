@@ -429,6 +429,10 @@ __device__ __forceinline__ void dma_walk(const typename Tr::vec8 (&qv)[D / 32], 
   wait_vmcnt<0>();  // no load may still target this workgroup's LDS when it exits
 }
 
+// log2-sum-exp of a partial: -inf where it has no token, NaN where its logits
+// are (a NaN or infinite query or key), which the merges carry into the output.
+__device__ __forceinline__ float partial_lse(float m, float l) { return l == 0.f ? kNegInf : m + __log2f(l); }
+
 // The wave's Gc query heads normalised by their sums: written to the output
 // (`out_rows`, head g at + g D) or, when out_rows is null, as a partial for a
 // merge (o / l at po + g po_stride, log2-sum-exp at plse + g plse_stride).
@@ -458,7 +462,7 @@ __device__ __forceinline__ void dma_finish(const f32x4 (&o)[D / 16], float m_run
     } else {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) po[g * po_stride + 16 * nb + l16] = o[nb][r] * inv;
-      if (l16 == 0) plse[g * plse_stride] = (lg > 0.f) ? mg + __log2f(lg) : kNegInf;
+      if (l16 == 0) plse[g * plse_stride] = partial_lse(mg, lg);
     }
   }
 }
@@ -569,14 +573,13 @@ __global__ __launch_bounds__(64 * NW) void decode_mw_kernel(
     float M = red_m[0][g];
 #pragma unroll
     for (int j = 1; j < NW; ++j) M = __builtin_fmaxf(M, red_m[j][g]);
+    const float msub = M == kNegInf ? 0.f : M;  // (no token, or only NaN logits: l says which)
     float l = 0.f, acc = 0.f;
-    if (M != kNegInf) {
 #pragma unroll
-      for (int j = 0; j < NW; ++j) {
-        const float a = fast_exp2(red_m[j][g] - M);
-        l += a * red_l[j][g];
-        acc += a * ((const float*)(lds + j * kRingB))[g * D + d];
-      }
+    for (int j = 0; j < NW; ++j) {
+      const float a = fast_exp2(red_m[j][g] - msub);
+      l += a * red_l[j][g];
+      acc += a * ((const float*)(lds + j * kRingB))[g * D + d];
     }
     const float inv = l > 0.f ? 1.f / l : 0.f;
     const size_t hq = (size_t)n * Hq + hq0 + g;
@@ -585,7 +588,7 @@ __global__ __launch_bounds__(64 * NW) void decode_mw_kernel(
     } else {
       const size_t sl = hq * max_splits + split;
       ws_o[sl * D + d] = acc * inv;
-      if (d == 0) ws_lse[sl] = l > 0.f ? M + __log2f(l) : kNegInf;
+      if (d == 0) ws_lse[sl] = partial_lse(M, l);
     }
   }
 }
@@ -753,36 +756,35 @@ __device__ __forceinline__ void merge_rows(int n_parts, Idx idx, const float* __
   for (int s = lane + 64; s < n_parts; s += 64) M = __builtin_fmaxf(M, ws_lse[idx(s)]);
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) M = __builtin_fmaxf(M, __shfl_xor(M, off, 64));
+  const float msub = M == kNegInf ? 0.f : M;  // (M passes over a NaN; its weight is one)
   float wsum = 0.f;
   float acc[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) acc[i] = 0.f;
-  if (M != kNegInf) {
-    for (int s0 = 0; s0 < n_parts; s0 += 64) {
-      const int s = s0 + lane;
-      const float lse = s0 == 0 ? lse0 : (s < n_parts) ? ws_lse[idx(s)] : kNegInf;
-      const float wl = (lse == kNegInf) ? 0.f : fast_exp2(lse - M);
-      const int cnt = min(64, n_parts - s0);
-      int j0 = 0;
-      if (s0 == 0) {
+  for (int s0 = 0; s0 < n_parts; s0 += 64) {
+    const int s = s0 + lane;
+    const float lse = s0 == 0 ? lse0 : (s < n_parts) ? ws_lse[idx(s)] : kNegInf;
+    const float wl = fast_exp2(lse - msub);
+    const int cnt = min(64, n_parts - s0);
+    int j0 = 0;
+    if (s0 == 0) {
 #pragma unroll
-        for (int j = 0; j < kMergeAhead; ++j)
-          if (j < n_ahead) {
-            const float wj = __shfl(wl, j, 64);
-            wsum += wj;
+      for (int j = 0; j < kMergeAhead; ++j)
+        if (j < n_ahead) {
+          const float wj = __shfl(wl, j, 64);
+          wsum += wj;
 #pragma unroll
-            for (int i = 0; i < PER; ++i) acc[i] += wj * part[j][i];
-          }
-        j0 = n_ahead;
-      }
+          for (int i = 0; i < PER; ++i) acc[i] += wj * part[j][i];
+        }
+      j0 = n_ahead;
+    }
 #pragma unroll 4
-      for (int j = j0; j < cnt; ++j) {
-        const float wj = __shfl(wl, j, 64);
-        wsum += wj;
-        const float* src = ws_o + idx(s0 + j) * D + lane * PER;
+    for (int j = j0; j < cnt; ++j) {
+      const float wj = __shfl(wl, j, 64);
+      wsum += wj;
+      const float* src = ws_o + idx(s0 + j) * D + lane * PER;
 #pragma unroll
-        for (int i = 0; i < PER; ++i) acc[i] += wj * src[i];
-      }
+      for (int i = 0; i < PER; ++i) acc[i] += wj * src[i];
     }
   }
   const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
@@ -1216,7 +1218,7 @@ __global__ __launch_bounds__(64) void decode_f32_kernel(
       const float sm = valid ? s[g] : kNegInf;
       const float m_new = __builtin_fmaxf(m_run[g], wave_max_f(sm));
       const float alpha = (m_run[g] == kNegInf) ? 0.f : fast_exp2(m_run[g] - m_new);
-      const float p = valid ? fast_exp2(sm - m_new) : 0.f;
+      const float p = valid ? fast_exp2(sm - (m_new == kNegInf ? 0.f : m_new)) : 0.f;
       l_run[g] = l_run[g] * alpha + p;
 #pragma unroll
       for (int i = 0; i < PER; ++i) o[g][i] *= alpha;
@@ -1286,7 +1288,7 @@ __global__ __launch_bounds__(64) void decode_f32_kernel(
       const size_t sl = ((size_t)n * Hq + hq) * max_splits + split;
 #pragma unroll
       for (int i = 0; i < PER; ++i) ws_o[sl * D + lane + 64 * i] = o[g][i] * inv;
-      if (lane == 0) ws_lse[sl] = (lt > 0.f) ? m_run[g] + __log2f(lt) : kNegInf;
+      if (lane == 0) ws_lse[sl] = partial_lse(m_run[g], lt);
     }
   }
 }

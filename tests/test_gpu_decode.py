@@ -377,6 +377,37 @@ def test_flash_decode_running_max_growth(dev, b, hkv, group, kv_len, head_dim, p
         assert_close(to_np(out[i:i + 1]), ref, **TOL_16BIT, name=profile)
 
 
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("cache", ["paged", "fp8", "contiguous"])
+@pytest.mark.parametrize("n,hkv,width", [
+    (2, 2, 4),      # one wave
+    (66, 4, 40),    # four waves
+    (2, 2, 60),     # eight
+    (2, 2, 250),    # splits
+    (64, 8, 512),   # the balanced walk
+])
+def test_not_a_number_stays(dev, n, hkv, width, cache, dtype, value):
+    """A NaN or an infinity in a query head makes all of that head's output NaN,
+    as softmax does, and leaves the other heads' as they are."""
+    lens = [16 * width - 3 - i % 16 for i in range(n)]
+    if cache == "contiguous":
+        q = torch.randn(n, 2 * hkv, 1, 64, device=dev).to(dtype)
+        k, v = (torch.randn(n, hkv, lens[0], 64, device=dev).to(dtype) for _ in range(2))
+        run = lambda: cuda_llm.flash_decode(q, k, v)
+    else:
+        case = build_paged(lens, 2 * hkv, hkv, 64, dtype, dev, fp8=cache == "fp8")
+        q = case["query"]
+        run = lambda: _run_paged(case)
+    clean = run()
+    q[1, 1].view(-1)[5] = value
+    out = run()
+    torch.cuda.synchronize()
+    assert torch.isnan(out[1, 1]).all()
+    out[1, 1] = clean[1, 1]
+    assert_close(to_np(out), to_np(clean), **TOL_16BIT, name="other heads")
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 def test_least_workspace_takes_coarse_splits(dev, fp8):
     """ca_decode_workspace_bytes stays enough: with it the small launches keep
