@@ -14,7 +14,7 @@ import torch
 
 import cuda_llm
 import oracle
-from _util import TOL_16BIT, assert_close, prefill_rows_groups, qkv, to_np
+from _util import TOL_16BIT, assert_close, prefill_order, prefill_rows_groups, qkv, to_np
 
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "golden.npz")
@@ -90,13 +90,18 @@ def test_zero_scale_is_running_mean(dev, dtype, head_dim, is_causal):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize("is_causal", [False, True])
-def test_long_ragged_sequence_zero_scale(dev, dtype, head_dim, is_causal):
-    """One head of 65573 rows (a ragged end far past the sizes the oracle
-    checks; 1025 key tiles, so the head-dim-64 walk's groups of four end
-    mid-group): with softmax_scale = 0 the output is the running mean of V,
-    checked on every row."""
+@pytest.mark.parametrize("heads", [1, 4])
+def test_long_ragged_sequence_zero_scale(dev, dtype, head_dim, is_causal, heads):
+    """Heads of 65573 rows (a ragged end far past the sizes the oracle checks;
+    1025 key tiles, so with four heads, which take the 256-row kernels, the
+    head-dim-64 walk's groups of four end mid-group; one head's waves share
+    rows, except not causal at head dim 128): with softmax_scale = 0 the output
+    is the running mean of V, checked on every row."""
     s = 65573
-    q, k, v = qkv(1, 1, s, head_dim, dtype, dev)
+    if dtype != torch.float32:
+        assert (prefill_rows_groups(1, heads, s, head_dim, is_causal) > 0) == \
+            (heads == 1 and (is_causal or head_dim == 64))
+    q, k, v = qkv(1, heads, s, head_dim, dtype, dev)
     out = cuda_llm.flash_attention(q, k, v, is_causal=is_causal, softmax_scale=0.0)
     torch.cuda.synchronize()
     v64 = v.double()
@@ -122,31 +127,39 @@ def test_negative_scale(dev, dtype, head_dim, is_causal):
     assert_close(to_np(out), ref, **TOL_16BIT, name=f"negative scale {dtype}")
 
 
-def test_custom_scale_and_large_logits(dev):
+@pytest.mark.parametrize("heads", [2, 64])
+def test_custom_scale_and_large_logits(dev, heads):
     """Scaled-up queries drive the lazy-rescale path (row max jumps by > 8 in
-    log2 units between tiles)."""
-    q, k, v = qkv(1, 2, 700, 128, torch.bfloat16, dev)
+    log2 units between tiles): two heads' waves share rows, 64 heads take the
+    64-row kernel."""
+    q, k, v = qkv(1, heads, 700, 128, torch.bfloat16, dev)
     q = (q.float() * 6).to(torch.bfloat16)
+    # weights and result are each rounded to bf16 once, by at most 2^-8 of max |V|
+    tol = TOL_16BIT if heads == 2 else dict(max_abs=2 * 2.0 ** -8 * v.abs().max().item(), mean_abs=2e-3)
     for causal in (False, True):
+        assert (prefill_rows_groups(1, heads, 700, 128, causal) > 0) == (heads == 2)
         out = cuda_llm.flash_attention(q, k, v, is_causal=causal, softmax_scale=0.3)
         torch.cuda.synchronize()
         ref = oracle.attention(to_np(q), to_np(k), to_np(v), is_causal=causal, scale=0.3)
-        assert_close(to_np(out), ref, **TOL_16BIT, name=f"large logits causal={causal}")
+        assert_close(to_np(out), ref, **tol, name=f"large logits causal={causal}")
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("is_causal", [False, True])
 @pytest.mark.parametrize("profile", ["ramp", "jump"])
 @pytest.mark.parametrize("d", [64, 128])
-def test_running_max_growth(dev, dtype, is_causal, profile, d):
+@pytest.mark.parametrize("b,h", [(1, 2), (2, 32)])
+def test_running_max_growth(dev, dtype, is_causal, profile, d, b, h):
     """Logits that grow along the keys. Tiles after a wave's first take their
     exponentials against the running max as it stands; a tile whose sums
     pass the bound of the P operand type (bf16 2^48, fp16 2^15; ramp: about
     +33 log2 units per 64-key tile) or overflow to infinity (jump: +130 log2
     units at key 512) takes the full max, rescales O and l, and takes the
-    exponentials again."""
+    exponentials again. Two heads' waves share rows; 2 x 32 heads take the
+    256-row kernel at head dim 64 and the 64-row one at 128."""
     g = torch.Generator(device=dev).manual_seed(11)
-    b, h, s = 1, 2, 1024
+    s = 1024
+    assert (prefill_rows_groups(b, h, s, d, is_causal) > 0) == (h == 2)
     u = torch.randn(d, device=dev, generator=g)
     u = u / u.norm()
     j = torch.arange(s, device=dev, dtype=torch.float32)
@@ -158,8 +171,9 @@ def test_running_max_growth(dev, dtype, is_causal, profile, d):
     out = cuda_llm.flash_attention(q, k, v, is_causal=is_causal)
     torch.cuda.synchronize()
     assert torch.isfinite(out).all()
-    ref = oracle.attention(to_np(q), to_np(k), to_np(v), is_causal=is_causal)
-    assert_close(to_np(out), ref, **TOL_16BIT, name=f"{profile} causal={is_causal}")
+    for bi, hi in ((0, 0), (b - 1, h - 1)):
+        ref = oracle.attention(*(to_np(t[bi:bi + 1, hi:hi + 1]) for t in (q, k, v)), is_causal=is_causal)
+        assert_close(to_np(out[bi:bi + 1, hi:hi + 1]), ref, **TOL_16BIT, name=f"{profile} causal={is_causal}")
 
 
 def test_every_row_written(dev):
@@ -223,24 +237,26 @@ def test_baseline_c2_shapes(dev, cfg):
 
 
 @pytest.mark.parametrize("dtype,d,b,hq,hkv,s", [
-    (torch.bfloat16, 128, 2, 32, 8, 3072),   # 12 query tiles of 256 rows: 6 pairs per head
-    (torch.float16, 128, 2, 32, 32, 3456),   # 14 tiles (first one 128 rows): 7 pairs
-    (torch.bfloat16, 128, 2, 32, 8, 3800),   # 15 tiles: 7 pairs + middle tiles of 2 heads
+    (torch.bfloat16, 128, 3, 28, 7, 3072),   # 12 query tiles of 256 rows: 6 pairs per head
+    (torch.float16, 128, 2, 36, 36, 3456),   # 14 tiles (first one 128 rows): 7 pairs
+    (torch.bfloat16, 128, 2, 33, 11, 3800),  # 15 tiles: 7 pairs + middle tiles of 2 heads
     (torch.float16, 128, 2, 32, 32, 4096),   # 16 tiles: 8 pairs
-    (torch.bfloat16, 128, 7, 7, 1, 2800),    # 11 tiles, 49 heads: one lone middle tile
+    (torch.bfloat16, 128, 7, 13, 1, 2800),   # 11 tiles, 91 heads: one lone middle tile
     (torch.bfloat16, 64, 4, 32, 8, 1900),    # head dim 64: 8 tiles (first one 128 rows)
-    (torch.bfloat16, 128, 2, 24, 8, 3640),   # 15 tiles, the first one 64 rows (one key tile)
-    (torch.float16, 64, 2, 24, 8, 3640),     # the same at head dim 64
+    (torch.bfloat16, 128, 2, 33, 11, 3640),  # 15 tiles, the first one 64 rows (one key tile)
+    (torch.float16, 64, 2, 33, 11, 3640),    # the same at head dim 64
 ])
 def test_causal_paired_query_tiles(dev, dtype, d, b, hq, hkv, s):
-    """Causal grids big enough that each workgroup takes two query tiles
-    (tiles n_qt-1-p and p of a head; for an odd n_qt the middle tiles of two
-    heads), for equal work per workgroup on a 256-CU device; every grid here
-    also exceeds 256 such items, so each workgroup of the persistent launch
-    takes several, its key ring running on from one tile into the next (a
-    one-key-tile first tile, S = 3640, stops that). Sampled heads (including
-    the last head, whose middle tile may be alone) against the oracle, every
-    head through row 0 (which sees key 0 only) and through finiteness."""
+    """Causal grids that fill rounds of a 256-CU device with pairs of query
+    tiles (tiles n_qt-1-p and p of a head; for an odd n_qt the middle tiles of
+    two heads), for equal work per workgroup; every grid here exceeds 256 such
+    items, so each workgroup of the persistent launch takes several, its key
+    ring running on from one tile into the next (a one-key-tile first tile,
+    S = 3640, stops that). Sampled heads (including the last head, whose middle
+    tile may be alone) against the oracle, every head through row 0 (which sees
+    key 0 only) and through finiteness."""
+    grid, order = prefill_order(b, hq, -(-s // 256), True)
+    assert prefill_rows_groups(b, hq, s, d, True) == 0 and order == "pairs" and grid > 256
     q, k, v = qkv(b, hq, s, d, dtype, dev, hkv=hkv)
     out = cuda_llm.flash_attention(q, k, v, is_causal=True)
     torch.cuda.synchronize()
@@ -277,23 +293,26 @@ def test_persistent_noncausal(dev, dtype, s, d):
 def _random_w64_cases(n=12, seed=1234):
     """Seeded shapes for the 64-row kernel (head dim 128, bf16 and fp16):
     ragged lengths (a first query tile of 64-192 rows), GQA ratios, causal
-    and not, with and without the LSE output."""
+    and not, with and without the LSE output; 130 heads or more, which take
+    that kernel at these lengths."""
     rng = np.random.default_rng(seed)
     out = []
     for i in range(n):
         hkv = int(rng.choice([1, 2, 4, 8]))
         g = int(rng.choice([1, 2, 4]))
         s = int(rng.integers(65, 2600))
-        out.append((torch.float16 if i % 2 else torch.bfloat16, int(rng.integers(1, 3)), hkv * g, hkv, s,
+        b = -(-int(rng.integers(130, 260)) // (hkv * g))
+        out.append((torch.float16 if i % 2 else torch.bfloat16, b, hkv * g, hkv, s,
                     bool(rng.integers(0, 2)), bool(rng.integers(0, 2)), float(rng.choice([0.05, 0.0884, 0.2]))))
     return out
 
 
 @pytest.mark.parametrize("dtype,b,hq,hkv,s,causal,lse,scale", _random_w64_cases())
 def test_w64_random_shapes(dev, dtype, b, hq, hkv, s, causal, lse, scale):
-    """The 64-row kernel on seeded random shapes: every head of the first
+    """The 64-row kernel on seeded random shapes: every head of the last
     batch against the oracle; the LSE, where asked for, against the oracle's
     logsumexp."""
+    assert prefill_rows_groups(b, hq, s, 128, causal) == 0
     gen = torch.Generator(device=dev).manual_seed(s)
     q, k, v = qkv(b, hq, s, 128, dtype, dev, hkv=hkv, gen=gen)
     if lse:
@@ -302,37 +321,42 @@ def test_w64_random_shapes(dev, dtype, b, hq, hkv, s, causal, lse, scale):
         out = cuda_llm.flash_attention(q, k, v, is_causal=causal, softmax_scale=scale)
     torch.cuda.synchronize()
     assert torch.isfinite(out).all()
-    ref = oracle.attention(to_np(q[:1]), to_np(k[:1]), to_np(v[:1]), is_causal=causal, scale=scale)
-    assert_close(to_np(out[:1]), ref, **TOL_16BIT, name=f"{dtype} {b}x{hq}/{hkv}x{s} causal={causal}")
+    ref = oracle.attention(to_np(q[-1:]), to_np(k[-1:]), to_np(v[-1:]), is_causal=causal, scale=scale)
+    assert_close(to_np(out[-1:]), ref, **TOL_16BIT, name=f"{dtype} {b}x{hq}/{hkv}x{s} causal={causal}")
     if lse:
-        lref = oracle.attention_lse(to_np(q[:1]), to_np(k[:1]), is_causal=causal, scale=scale, dtype=np.float64)
-        assert np.abs(to_np(l[:1]) - lref).max() <= 1e-3
+        lref = oracle.attention_lse(to_np(q[-1:]), to_np(k[-1:]), is_causal=causal, scale=scale, dtype=np.float64)
+        assert np.abs(to_np(l[-1:]) - lref).max() <= 1e-3
 
 
 @pytest.mark.parametrize("dtype,s,causal", [(torch.bfloat16, 16384, True), (torch.float16, 16384, False),
                                             (torch.bfloat16, 12345, False)])
 def test_w64_long_sequences(dev, dtype, s, causal):
     """Long walks of the 64-row kernel (up to 256 key tiles per query tile,
-    64 query tiles per head) on one head against the oracle."""
+    64 query tiles per head) on one of eight heads against the oracle."""
+    assert prefill_rows_groups(1, 8, s, 128, causal) == 0
     gen = torch.Generator(device=dev).manual_seed(s)
-    q, k, v = qkv(1, 2, s, 128, dtype, dev, gen=gen)
+    q, k, v = qkv(1, 8, s, 128, dtype, dev, gen=gen)
     out = cuda_llm.flash_attention(q, k, v, is_causal=causal)
     torch.cuda.synchronize()
     assert torch.isfinite(out).all()
-    ref = oracle.attention(to_np(q[:, 1:]), to_np(k[:, 1:]), to_np(v[:, 1:]), is_causal=causal)
-    assert_close(to_np(out[:, 1:]), ref, **TOL_16BIT, name=f"{dtype} S={s} causal={causal}")
+    ref = oracle.attention(to_np(q[:, 7:]), to_np(k[:, 7:]), to_np(v[:, 7:]), is_causal=causal)
+    assert_close(to_np(out[:, 7:]), ref, **TOL_16BIT, name=f"{dtype} S={s} causal={causal}")
 
 
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("is_causal", [False, True])
-@pytest.mark.parametrize("b,hq,hkv,s", [(1, 3, 1, 1), (1, 3, 1, 31), (1, 3, 1, 33), (1, 3, 1, 65), (1, 4, 4, 127),
-                                        (1, 4, 4, 129), (1, 4, 2, 257), (1, 8, 8, 1025), (4, 12, 12, 400),
-                                        (1, 32, 8, 1000)])
-def test_shared_row_waves(dev, b, hq, hkv, s, is_causal, d):
-    """Launches too small for 256-row tiles, whose waves share rows: lengths at
-    the edges of the 32-row groups, of the key tiles and of a round of the
-    waves' tiles; fewer tiles than waves; pairs of tiles. O and LSE of sampled
-    heads against the oracle, every row written."""
+@pytest.mark.parametrize("b,hq,hkv,s,dims", [
+    (1, 3, 1, 65, (64, 128)), (1, 4, 2, 95, (64, 128)), (1, 3, 1, 97, (64, 128)), (1, 4, 4, 127, (64, 128)),
+    (1, 4, 4, 193, (64, 128)), (1, 4, 2, 256, (64, 128)), (1, 3, 1, 321, (64, 128)), (1, 8, 8, 1025, (64, 128)),
+    (4, 12, 12, 400, (64, 128)), (1, 32, 8, 1000, (64, 128)), (1, 4, 4, 129, (64,)), (1, 4, 2, 257, (64,)),
+    (1, 3, 1, 1, ()), (1, 3, 1, 31, ()), (1, 3, 1, 33, ())])
+def test_shared_row_waves(dev, b, hq, hkv, s, dims, is_causal, d):
+    """Launches too small for 256-row tiles, whose waves share rows (at the head
+    dims `dims`; the others' run the 256-row kernels): lengths at the edges of the
+    32-row groups, of the key tiles and of a round of the waves' tiles; fewer
+    tiles than waves; pairs of tiles. O and LSE of sampled heads against the
+    oracle, every row written."""
+    assert (prefill_rows_groups(b, hq, s, d, is_causal) > 0) == (d in dims)
     import cuda_amd._lib as L
     from cuda_amd.api import _ptr, _stream
     gen = torch.Generator(device=dev).manual_seed(s)
@@ -379,10 +403,12 @@ def test_shared_row_waves_lanes_past_the_end(dev, dtype, d, is_causal):
 
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("is_causal", [False, True])
-@pytest.mark.parametrize("s,jump", [(1, False), (65, False), (200, False), (600, True)])
+@pytest.mark.parametrize("s,jump", [(1, False), (65, False), (129, False), (200, False), (600, True)])
 def test_short_sequences_full_grid(dev, s, jump, is_causal, d):
     """Short sequences of many heads: the 256-row kernels' walks of one to ten
-    key tiles, and (jump) key norms that rise past the stale running max."""
+    key tiles (two: causal only, the others' waves share rows), and (jump) key
+    norms that rise past the stale running max."""
+    assert (prefill_rows_groups(8, 64, s, d, is_causal) > 0) == (s == 65 and not is_causal)
     gen = torch.Generator(device=dev).manual_seed(s)
     dtype = torch.float16 if jump else torch.bfloat16
     q, k, v = qkv(8, 64, s, d, dtype, dev, hkv=32, gen=gen)
@@ -407,7 +433,7 @@ def test_short_sequences_full_grid(dev, s, jump, is_causal, d):
     (3, 24, 4, 1000),   # 288 single tiles, longest first, nine heads per XCD
     (3, 12, 12, 2200),  # 324, 36 heads over all XCDs
     (1, 257, 257, 300),  # 514, an odd count of heads
-    (1, 12, 4, 3500),   # 336 tiles of 128 rows (head dim 64)
+    (1, 12, 4, 3500),   # 336 tiles of 128 rows
     (1, 32, 8, 1500),   # 384 tiles of 128 rows
 ])
 def test_causal_tile_orders(dev, b, hq, hkv, s, d):
@@ -416,6 +442,9 @@ def test_causal_tile_orders(dev, b, hq, hkv, s, d):
     first. O and LSE of sampled heads against the oracle, every row written."""
     import cuda_amd._lib as L
     from cuda_amd.api import _ptr, _stream
+    groups = prefill_rows_groups(b, hq, s, d, True)
+    assert groups == (4 if b == 1 and hq < 257 else 0)
+    assert prefill_order(b, hq, -(-s // (32 * groups or 256)), True)[1] == ("pairs" if b == 7 else "longest")
     dtype = torch.float16 if d == 64 else torch.bfloat16
     q, k, v = qkv(b, hq, s, d, dtype, dev, hkv=hkv, gen=torch.Generator(device=dev).manual_seed(s))
     out = torch.full_like(q, float("nan"))

@@ -41,11 +41,13 @@ def test_rope_reference_grid(dev, dtype, head_dim, is_causal):
 
 
 @pytest.mark.parametrize("b,hq,hkv,s,d", [(2, 8, 2, 1024, 128), (1, 4, 4, 777, 64), (2, 32, 8, 2048, 128),
-                                           (2, 32, 8, 4096, 128)])
+                                           (2, 32, 8, 4096, 128), (2, 32, 8, 4096, 64)])
 def test_rope_longer_and_gqa(dev, b, hq, hkv, s, d):
-    """Longer sequences and GQA; at S = 4096 the grid is persistent (512
-    causal pairs), so the rotated Q of a query tile is often loaded by the
-    workgroup's previous tile, of another head."""
+    """Longer sequences and GQA: waves that share rows (up to S = 1024) and the
+    64-row and 256-row kernels; at S = 4096 the grid is persistent (512 causal
+    pairs), so the rotated Q of a query tile is often loaded by the workgroup's
+    previous tile, of another head."""
+    assert (prefill_rows_groups(b, hq, s, d, True) > 0) == (s <= 1024)
     q, k, v = qkv(b, hq, s, d, torch.bfloat16, dev, hkv=hkv)
     cos, sin = rope_tables(s, d, dev)
     out = cuda_llm.fused_rope_flash_attention(q, k, v, cos, sin)  # default causal
@@ -59,21 +61,22 @@ def test_rope_longer_and_gqa(dev, b, hq, hkv, s, d):
 
 
 @pytest.mark.parametrize("dtype,d", [(torch.float16, 128), (torch.bfloat16, 64), (torch.bfloat16, 128)])
-def test_rope_identity_tables_equal_flash_attention(dev, dtype, d):
-    """Identity tables leave Q and K as they are. Where both calls run the
-    same kernel the outputs are equal bit for bit; at head dim 128 without
-    rope both 16-bit types run the 64-row kernel, whose summation order
-    differs, so there the two agree to the 16-bit tolerance."""
-    q, k, v = qkv(2, 4, 300, d, dtype, dev)
-    ones = torch.ones(300, d, device=dev)
-    zeros = torch.zeros(300, d, device=dev)
-    a = cuda_llm.fused_rope_flash_attention(q, k, v, ones, zeros, is_causal=True)
-    b = cuda_llm.flash_attention(q, k, v, is_causal=True)
+@pytest.mark.parametrize("is_causal", [False, True])
+@pytest.mark.parametrize("scale", [None, -0.1])
+@pytest.mark.parametrize("b,hq,hkv,s", [(2, 4, 4, 300), (2, 32, 8, 4096), (2, 33, 11, 3800)])
+def test_rope_identity_tables_equal_flash_attention(dev, dtype, d, is_causal, scale, b, hq, hkv, s):
+    """Identity tables leave Q and K as they are, and the same kernel runs, only
+    with Q in the buffer that it writes: equal bit for bit. The larger grids are
+    persistent (pairs or equal tiles, several per workgroup, ragged at 3800); a
+    negative scale takes the 256-row kernel at both head dims, which loads the
+    next tile's Q before it stores a tile."""
+    q, k, v = qkv(b, hq, s, d, dtype, dev, hkv=hkv)
+    ones = torch.ones(s, d, device=dev)
+    zeros = torch.zeros(s, d, device=dev)
+    a = cuda_llm.fused_rope_flash_attention(q, k, v, ones, zeros, is_causal=is_causal, softmax_scale=scale)
+    c = cuda_llm.flash_attention(q, k, v, is_causal=is_causal, softmax_scale=scale)
     torch.cuda.synchronize()
-    if d == 128:
-        assert_close(to_np(a), to_np(b), **TOL_16BIT, name="identity rope")
-    else:
-        assert torch.equal(a, b)
+    assert torch.equal(a, c)
 
 
 @pytest.mark.parametrize("d", [64, 128])
