@@ -462,17 +462,22 @@ __device__ CA_INLINE bool prefill_dma_qtile(const void* Qv, const void* __restri
   // the first kNPF PV steps of M(s + 1) are read during softmax(s) (tile s
   // is resident from barrier s until barrier s + 2, which follows M(s + 1)).
   constexpr int kNPF = 4;
-  u32x4 pvf[kNPF];
+  // A V^T fragment's halves, joined after their wait (joining them earlier could
+  // copy registers that a read in flight has yet to write).
+  struct Halves {
+    u32x2 a, c;
+  };
+  Halves pvf[kNPF];
   auto pv_read = [&](uint32_t va1, uint32_t va2, int i) CA_INLINE {
     const uint32_t x = 64 * (i >> 2);
-    u32x2 a, c;
+    Halves h;
     switch (i & 3) {
-      case 0: a = lds_read_tr16<0>(va1 ^ x); c = lds_read_tr16<0>(va2 ^ x); break;
-      case 1: a = lds_read_tr16<kKK>(va1 ^ x); c = lds_read_tr16<kKK>(va2 ^ x); break;
-      case 2: a = lds_read_tr16<2 * kKK>(va1 ^ x); c = lds_read_tr16<2 * kKK>(va2 ^ x); break;
-      default: a = lds_read_tr16<3 * kKK>(va1 ^ x); c = lds_read_tr16<3 * kKK>(va2 ^ x); break;
+      case 0: h.a = lds_read_tr16<0>(va1 ^ x); h.c = lds_read_tr16<0>(va2 ^ x); break;
+      case 1: h.a = lds_read_tr16<kKK>(va1 ^ x); h.c = lds_read_tr16<kKK>(va2 ^ x); break;
+      case 2: h.a = lds_read_tr16<2 * kKK>(va1 ^ x); h.c = lds_read_tr16<2 * kKK>(va2 ^ x); break;
+      default: h.a = lds_read_tr16<3 * kKK>(va1 ^ x); h.c = lds_read_tr16<3 * kKK>(va2 ^ x); break;
     }
-    return u32x4{a[0], a[1], c[0], c[1]};
+    return h;
   };
   auto pv_prefetch = [&](int t) CA_INLINE {
     const uint32_t va1 = stage(t) + vofs1, va2 = stage(t) + vofs2;
@@ -491,7 +496,8 @@ __device__ CA_INLINE bool prefill_dma_qtile(const void* Qv, const void* __restri
 #pragma unroll
         for (int r = 0; r < 16; ++r) sacc[mb][r] = 0.f;
     }
-    u32x4 fr[kMD + 1][kRQK];
+    Halves fv[kMD + 1];   // fragments of PV steps
+    u32x4 fr[kMD + 1];    // ... and of QK steps
     // steps [0, P0) take the fragments read during the softmax; the ring
     // streams steps [P0, N)
     constexpr int P0 = DPV ? kNPF : 0;
@@ -499,13 +505,13 @@ __device__ CA_INLINE bool prefill_dma_qtile(const void* Qv, const void* __restri
     auto fread = [&](int i) CA_INLINE {
       const int b = i % (kMD + 1);
       if (i < NPV) {
-        fr[b][0] = pv_read(va1, va2, i);
+        fv[b] = pv_read(va1, va2, i);
       } else {
         const int j = i - NPV, mb = j & 1, ks = j >> 1;
         if (mb == 0) {
-          fr[b][0] = lds_read_b128<0>(ka ^ (32 * ks));
+          fr[b] = lds_read_b128<0>(ka ^ (32 * ks));
         } else {
-          fr[b][0] = lds_read_b128<32 * kKRowB>(ka ^ (32 * ks));
+          fr[b] = lds_read_b128<32 * kKRowB>(ka ^ (32 * ks));
         }
       }
     };
@@ -517,7 +523,10 @@ __device__ CA_INLINE bool prefill_dma_qtile(const void* Qv, const void* __restri
       for (int k = P0; k < P0 + kMD && k < N; ++k) pending += nreads(k);
       wait_lgkm_n(pending);
 #pragma unroll
-      for (int i = 0; i < P0; ++i) after_wait(pvf[i]);
+      for (int i = 0; i < P0; ++i) {
+        after_wait(pvf[i].a);
+        after_wait(pvf[i].c);
+      }
     }
 #pragma unroll
     for (int i = 0; i < N; ++i) {
@@ -528,16 +537,21 @@ __device__ CA_INLINE bool prefill_dma_qtile(const void* Qv, const void* __restri
 #pragma unroll
         for (int k = i + 1; k <= i + kMD && k < N; ++k) pending += nreads(k);
         wait_lgkm_n(pending);
-#pragma unroll
-        for (int r = 0; r < kRQK; ++r) after_wait(fr[b][r]);
+        if (i < NPV) {
+          after_wait(fv[b].a);
+          after_wait(fv[b].c);
+        } else {
+          after_wait(fr[b]);
+        }
       }
       if (i < NPV) {
         const int ob = i >> 2, kk = i & 3;
-        const u32x4 va = i < P0 ? pvf[i < P0 ? i : 0] : fr[b][0];
+        const Halves h = i < P0 ? pvf[i < P0 ? i : 0] : fv[b];
+        const u32x4 va = {h.a[0], h.a[1], h.c[0], h.c[1]};
         o[ob] = Tr::mfma32(__builtin_bit_cast(vec8, va), pb[kk], o[ob]);
       } else {
         const int j = i - NPV, mb = j & 1, ks = j >> 1;
-        sacc[mb] = Tr::mfma32(__builtin_bit_cast(vec8, fr[b][0]), qv[ks], sacc[mb]);
+        sacc[mb] = Tr::mfma32(__builtin_bit_cast(vec8, fr[b]), qv[ks], sacc[mb]);
         if (j % (kNQK / kLoads) == kNQK / kLoads - 1) issue_one(s + kPpAhead, j / (kNQK / kLoads));
       }
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
