@@ -1,8 +1,8 @@
 // Shared device helpers for the gfx950 attention kernels.
 //
 // Everything here is written for CDNA4 (gfx950, wave64): MFMA operand vector
-// types, 16-bit element traits (bf16 / fp16), LDS transpose reads, fp8 e4m3
-// conversions and wave reductions.
+// types, 16-bit element traits (bf16 / fp16), fp8 e4m3 conversions and wave
+// reductions.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -48,15 +48,6 @@ struct BF16 {
   static __device__ __forceinline__ f32x4 mfma16(vec8 a, vec8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
-  // 16x16x16: 4 elements of k per lane (k = 4 * (lane / 16) + 0..3)
-  static __device__ __forceinline__ f32x4 mfma16k16(vec4 a, vec4 b, f32x4 c) {
-    typedef short s16x4 __attribute__((ext_vector_type(4)));
-    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a),
-                                                     __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ vec4 tr_read(const CA_LDS void* p) {
-    return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((CA_LDS vec4*)p);
-  }
   // round-to-nearest-even pack of two floats
   static __device__ __forceinline__ vec2 pack2(float a, float b) {
     vec2 r;
@@ -82,13 +73,6 @@ struct F16 {
   }
   static __device__ __forceinline__ f32x4 mfma16(vec8 a, vec8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ f32x4 mfma16k16(vec4 a, vec4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ vec4 tr_read(const CA_LDS void* p) {
-    typedef __fp16 fp16x4_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
-    return __builtin_bit_cast(vec4, __builtin_amdgcn_ds_read_tr16_b64_v4f16((CA_LDS fp16x4_t*)p));
   }
   static __device__ __forceinline__ vec2 pack2(float a, float b) {
     vec2 r;
@@ -156,11 +140,6 @@ __device__ __forceinline__ float pair16_sum(float x) {
 
 __device__ __forceinline__ bool wave_any(bool p) { return __ballot(p) != 0ull; }
 
-// LDS transpose read of 8 bytes (gfx950 ds_read_b64_tr_b8).
-__device__ __forceinline__ i32x2 tr8_read(const CA_LDS void* p) {
-  return __builtin_amdgcn_ds_read_tr8_b64_v2i32((CA_LDS i32x2*)p);
-}
-
 // fp8 e4m3 (OCP) x2 -> bf16 x2, exact (e4m3 values are bf16 values); HI
 // selects bytes 2-3 instead of 0-1 of the dword.
 template <bool HI>
@@ -185,14 +164,6 @@ __device__ __forceinline__ void for_const(F& f) {
     f(std::integral_constant<int, I>{});
     for_const<N, F, I + 1>(f);
   }
-}
-
-template <typename V8, typename V4>
-__device__ __forceinline__ V8 cat4(V4 lo, V4 hi) {
-  V8 r;
-  r[0] = lo[0]; r[1] = lo[1]; r[2] = lo[2]; r[3] = lo[3];
-  r[4] = hi[0]; r[5] = hi[1]; r[6] = hi[2]; r[7] = hi[3];
-  return r;
 }
 
 // The lane index (0..63) recomputed where it is used, from v_mbcnt rather

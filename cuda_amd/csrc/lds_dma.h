@@ -42,12 +42,6 @@ __device__ __forceinline__ u32x2 lds_read_tr16(uint32_t a) {
   return r;
 }
 template <int OFF>
-__device__ __forceinline__ uint32_t lds_read_b32(uint32_t a) {
-  uint32_t r = a;
-  CA_DEVICE_ASM("ds_read_b32 %0, %1 offset:%2" : "=v"(r) : "v"(a), "n"(OFF));
-  return r;
-}
-template <int OFF>
 __device__ __forceinline__ u32x2 lds_read_b64(uint32_t a) {
   u32x2 r = {a, a};
   CA_DEVICE_ASM("ds_read_b64 %0, %1 offset:%2" : "=v"(r) : "v"(a), "n"(OFF));

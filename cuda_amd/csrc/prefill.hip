@@ -453,7 +453,6 @@ __device__ CA_INLINE bool prefill_dma_qtile(const void* Qv, const void* __restri
   // kAhead go out between the QK steps.
   constexpr int kNPV = 4 * kNOB;
   constexpr int kNQK = 2 * Gv::kNKS;
-  constexpr int kRQK = 1;           // LDS reads per QK step
   constexpr int kMD = 4;            // steps read ahead
   static_assert(kNQK % kLoads == 0, "loads spread over the QK steps");
   constexpr int kKK = 16 * kVRowB;  // bytes per P^T k-step of V rows
@@ -501,7 +500,7 @@ __device__ CA_INLINE bool prefill_dma_qtile(const void* Qv, const void* __restri
     // steps [0, P0) take the fragments read during the softmax; the ring
     // streams steps [P0, N)
     constexpr int P0 = DPV ? kNPF : 0;
-    auto nreads = [&](int i) CA_INLINE { return i < NPV ? 2 : kRQK; };
+    auto nreads = [&](int i) CA_INLINE { return i < NPV ? 2 : 1; };
     auto fread = [&](int i) CA_INLINE {
       const int b = i % (kMD + 1);
       if (i < NPV) {
@@ -816,6 +815,7 @@ static hipError_t launch_prefill_kernel(const PfArgs& a, int B, int Hq, int Hkv,
   // hardware dispatcher to balance.
   const long long slots = device_cus() / 8 * 8;
   const long long grid = ((!CAUSAL || order == kOrderPairs) && slots > 0 && n_work > slots) ? slots : n_work;
+  // (at head dim 128 POS serves sl2 in (3e38, inf] only: prefill_w64_supported)
   const float sl2 = scale * kLog2e;
   const dim3 block(64 * kPfWaves);
   if (sl2 >= 0.f) {
@@ -837,7 +837,6 @@ static hipError_t launch_prefill_dma(const void* q, const void* k, const void* v
   const PfArgs a{q, k, (const uint16_t*)v, o, lse};
   return launch_prefill_kernel<Tr, D, CAUSAL>(a, B, Hq, Hkv, S, scale, stream);
 }
-
 
 hipError_t launch_prefill(int dtype, const void* q, const void* k, const void* v, void* o, float* lse,
                           int B, int Hq, int Hkv, int S, int D, float scale, bool causal,

@@ -127,6 +127,22 @@ def test_negative_scale(dev, dtype, head_dim, is_causal):
     assert_close(to_np(out), ref, **TOL_16BIT, name=f"negative scale {dtype}")
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("is_causal", [False, True])
+def test_largest_scales(dev, head_dim, is_causal):
+    """A softmax_scale whose base-2 image passes 3e38 stays with the 256-row
+    kernel at both head dims: bf16 q and k of 2^-61 and above, whose products
+    are normal floats and whose logits are of order 2^11."""
+    q, k, v = qkv(2, 4, 700, head_dim, torch.bfloat16, dev)
+    q, k = ((t.sign() * (1 + t.float().abs()) * 2.0 ** -61).bfloat16() for t in (q, k))
+    out = cuda_llm.flash_attention(q, k, v, is_causal=is_causal, softmax_scale=2.3e38)
+    torch.cuda.synchronize()
+    x = torch.matmul(q.double(), k.double().transpose(2, 3).contiguous()) * 2.3e38
+    if is_causal:
+        x.masked_fill_(torch.ones(700, 700, dtype=torch.bool, device=dev).triu_(1), -float("inf"))
+    assert_close(to_np(out), to_np(torch.softmax(x, -1) @ v.double()), **TOL_16BIT, name="largest scale")
+
+
 @pytest.mark.parametrize("heads", [2, 64])
 def test_custom_scale_and_large_logits(dev, heads):
     """Scaled-up queries drive the lazy-rescale path (row max jumps by > 8 in
