@@ -329,7 +329,7 @@ def _growing(hkv, group, d, tokens, profile, dev):
     (140, 4, 4, 16),    # one wave walks 16 pages
     (66, 4, 1, 40),     # four waves, ten pages each
     (6, 2, 16, 64),     # eight waves, eight pages each
-    (64, 8, 4, 512),    # the balanced walk
+    (72, 8, 4, 512),    # the balanced walk
 ])
 def test_paged_running_max_growth(dev, n, hkv, group, width, head_dim, fp8, profile):
     """Maxima that grow after a wave's first step, by head: the rescale of the
@@ -385,7 +385,7 @@ def test_flash_decode_running_max_growth(dev, b, hkv, group, kv_len, head_dim, p
     (66, 4, 40),    # four waves
     (2, 2, 60),     # eight
     (2, 2, 250),    # splits
-    (64, 8, 512),   # the balanced walk
+    (72, 8, 512),   # the balanced walk
 ])
 def test_not_a_number_stays(dev, n, hkv, width, cache, dtype, value):
     """A NaN or an infinity in a query head makes all of that head's output NaN,
@@ -397,6 +397,7 @@ def test_not_a_number_stays(dev, n, hkv, width, cache, dtype, value):
         run = lambda: cuda_llm.flash_decode(q, k, v)
     else:
         case = build_paged(lens, 2 * hkv, hkv, 64, dtype, dev, fp8=cache == "fp8")
+        assert balanced_walk_taken(n, 2 * hkv, hkv, 64, width, cache == "fp8") == (width == 512)
         q = case["query"]
         run = lambda: _run_paged(case)
     clean = run()
@@ -536,7 +537,7 @@ def test_balanced_walk_wide_groups_and_head_dim_64(dev):
     lens = torch.randint(0, 8193, (80,), generator=g).tolist()
     case = build_paged(lens, 64, 2, 128, torch.bfloat16, dev, pool=30000, seed=13)
     _check_balanced(case, TOL_16BIT, False, "balanced Gq=32")
-    lens = torch.randint(0, 8193, (64,), generator=g).tolist()
+    lens = torch.randint(0, 8193, (72,), generator=g).tolist()
     for fp8 in (False, True):
         case = build_paged(lens, 32, 8, 64, torch.bfloat16, dev, fp8=fp8, pool=20000, seed=14)
         _check_balanced(case, TOL_FP8 if fp8 else TOL_16BIT, fp8, f"balanced D=64 fp8={fp8}")
