@@ -903,13 +903,30 @@ struct SplitGrid {
 // `segs` walks of `pages` pages in splits of `coarse`, or finer where those
 // leave most CUs idle and the workspace holds the partials: up to four
 // workgroups per CU, 16 pages or more per split (a step of two for each of 8
-// waves) and 16 splits, which the merge loads at once. Measured against the
-// coarse splits: 3 bf16 sequences of 90-3000 tokens with their append 20.4 ->
-// 15.6 us, 1 of 1100 14.7 -> 9.7, contiguous 1 x 8 x 4001 16.1 -> 11.2, 24 FP8
-// sequences (head dim 64) 26.9 -> 23.5. Where the coarse 16-bit splits already
-// fill half the CUs (64 walks of 256 pages 21.6 -> 22.4 us) or the FP8 ones one
-// and a half (800 workgroups 47 -> 51) they stay, as with more than 16 splits
-// (8 walks of 1024 pages 20.9 -> 33).
+// waves) and 16 splits, which the merge loads at once (more: 8 walks of 1024
+// pages 20.9 -> 33 us). Measured against the coarse splits: 3 bf16 sequences of
+// 90-3000 tokens with their append 20.4 -> 15.6 us, 1 of 1100 14.7 -> 9.7,
+// contiguous 1 x 8 x 4001 16.1 -> 11.2, 24 FP8 sequences (head dim 64) 26.9 ->
+// 23.5.
+// The lines lie by the table's width (the lengths are on the device), so what
+// they give depends on how full the tables are. Coarse -> fine in us by coarse
+// workgroups (8 kv heads, 256-page tables; lengths spread from 1/13 of the
+// longest, which is 1/2 of the table | 3/4 | all; then every one full):
+//   16-bit, D = 64    96: 12.3 -> 10.5 | 12.7 -> 11.0 | 12.7 -> 15.0; 13.0 -> 15.7
+//                    128: 12.3 -> 10.8 | 12.8 -> 14.7 | 13.0 -> 15.3; 13.3 -> 16.2
+//                    160: 12.4 -> 12.0 | 12.8 -> 12.7 | 13.1 -> 13.2; 13.8 -> 14.2
+//   16-bit, D = 128   96: 17.2 -> 11.7 | 17.7 -> 12.4 | 18.0 -> 18.5; 18.7 -> 19.7
+//                    128: 17.5 -> 12.1 | 17.9 -> 17.9 | 18.5 -> 19.0; 19.4 -> 21.2
+//                    160: 17.5 -> 14.6 | 18.3 -> 15.8 | 18.9 -> 17.8; 20.3 -> 20.6
+//   FP8, D = 64      320: 16.4 -> 12.7 | 18.0 -> 14.7 | 20.1 -> 15.7; 21.7 -> 21.3
+//                    384: 16.4 -> 15.2 | 20.7 -> 15.7 | 21.0 -> 17.4; 22.9 -> 23.9
+//                    448: 16.8 -> 15.1 | 21.0 -> 19.5 | 20.9 -> 22.6; 25.1 -> 27.1
+//   FP8, D = 128     320: 20.6 -> 20.4 | 26.2 -> 22.6 | 29.5 -> 24.7; 37.6 -> 35.7
+//                    384: 20.8 -> 22.4 | 30.0 -> 24.9 | 31.4 -> 27.6; 39.3 -> 40.5
+//                    448: 21.1 -> 24.8 | 30.9 -> 27.3 | 32.4 -> 29.8; 42.7 -> 44.7
+// Half a workgroup per CU (16-bit) and one and a half (FP8) are where the gain
+// at ordinary fills still outweighs what full tables lose (16-bit: 512 fine
+// workgroups of 8 waves go in two rounds).
 static SplitGrid split_grid(long long segs, int N, int Hq, int D, int pages, int coarse, bool fp8, size_t ws_bytes) {
   SplitGrid g;
   g.pages = coarse;
@@ -1022,7 +1039,14 @@ static hipError_t launch_paged_decode_t(const void* q, const void* kc, const voi
 
 // The contiguous cache's split grid: as a paged one's, in equal splits; one
 // split when the heads alone are about one workgroup per CU, which saves the
-// merge (256 heads of 4096 tokens, head dim 64: 47 us against 52 with two).
+// merge. One split against two, in us, head dims 64 / 128:
+//   heads  2000 tokens             4096                      16384
+//   192    19.1, 21.9 / 33.0, 38.0  35.1, 39.5 / 61.0, 71.1   116, 134 / 233, 262
+//   224    20.7, 23.6 / 37.3, 40.6  39.5, 40.9 / 77.6, 74.3   137, 144 / 272, 277
+//   256    22.6, 25.2 / 41.7, 44.3  44.3, 49.2 / 83.7, 86.3   159, 164 / 315, 318
+//   264    29.7, 29.9 / 58.4, 52.7  58.5, 58.2 / 117, 102     218, 205 / 452, 384
+// Past one per CU the second round rules; below 7/8 one split is still the
+// faster (the line could lie lower).
 static SplitGrid contig_grid(int N, int Hq, int Hkv, int D, int S, size_t ws_bytes) {
   const int cus = device_cus();
   const int pages = S / kDecodePage + (S % kDecodePage != 0);

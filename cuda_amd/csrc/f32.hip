@@ -538,10 +538,11 @@ __global__ __launch_bounds__(64 * SplitStage<D>::NW, 1) void prefill_f32_split_k
 //   causal: 27 us against 91; at 192 tiles, not causal, D = 64, 55 against 48);
 // - not causal, D = 128: up to two tiles per CU (32 heads x 1500: 453 -> 354 us);
 //   D = 64 runs two workgroups per CU well (179 us against 195 at 16 x 2048);
-// - causal, fewer than two pairs of tiles per CU: the walks differ in length, the split ones
-//   do not. D = 128 always (16 heads x 2048: 344 -> 169 us; 256 x 300: 151 ->
-//   112) but for heads of one full tile (256 x 128: 31 against 37), D = 64 where the longest walk is 1.2 times the mean load or more (16 x
-//   2048: 180 -> 105 us; 256 x 300, 1.1 times: 57 against 61).
+// - causal, fewer than two pairs of tiles per CU: the walks differ in length, the
+//   split ones do not. D = 128 always (16 heads x 2048: 344 -> 169 us; 256 x 300:
+//   151 -> 112) but for heads of one full tile (256 x 128: 31 against 37), D = 64
+//   where the longest walk is 1.2 times the mean load or more (16 x 2048: 180 ->
+//   105 us; 256 x 300, 1.1 times: 57 against 61).
 static bool f32_splits(long long grid, bool causal, int D, int S, long long n_qt,
                        long long n_bh) {
   const long long cus = device_cus();

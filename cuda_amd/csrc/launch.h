@@ -107,9 +107,10 @@ inline long long prefill_grid(int B, int Hq, int n_qt, bool causal, int wg_per_c
   return *order == kOrderPairs ? pairs : single;
 }
 
-// Split-K geometry of the decode kernels: pages of 16 tokens. The workspace
-// is sized for splits of kPagesPerWave pages, the finest that any kernel
-// takes (decode.hip: DmaCfg, contig_splits; the float32 kernel splits there).
+// Split-K geometry of the decode kernels: pages of 16 tokens. The least
+// workspace is sized for splits of kPagesPerWave pages (the float32 kernel's);
+// the 16-bit and FP8 ones split finer, down to 16 pages, only where the given
+// workspace holds their partials (decode.hip: split_grid, contig_grid).
 constexpr int kDecodePage = 16;
 constexpr int kPagesPerWave = 64;
 

@@ -203,12 +203,13 @@ ca_status ca_fp8_paged_attention(ca_dtype dtype, const void* query, const uint8_
  * scratch return CA_INVALID_ARGUMENT. The partials are those of the launch's
  * plan: for fp16/bf16 queries, when the longest context spans more than 128
  * blocks, num_seqs <= 1024 and the balanced walk's partials fit the
- * workspace ca_decode_workspace_bytes names, 2 * (4 * compute units) *
- * min(16, num_q_heads / num_kv_heads) * (head_dim + 1) * 4 + 4 * num_seqs
- * bytes (4.2 MB at head dim 128 and 4 query heads per kv head on a
- * 256-CU device, whatever the context lengths); otherwise num_seqs *
- * num_q_heads * splits * (head_dim + 1) * 4 bytes with splits =
- * ceil(max_blocks_per_seq / 128) for fp16/bf16 queries and
+ * workspace ca_decode_workspace_bytes names, 2 * waves * min(16, num_q_heads /
+ * num_kv_heads) * (head_dim + 1) * 4 + 4 * num_seqs bytes with 4 waves per
+ * compute unit (8 at head dim 64; 4.2-4.3 MB at either head dim and 4 query heads
+ * per kv head on a 256-CU device, whatever the context lengths); otherwise
+ * num_seqs * num_q_heads * splits * (head_dim + 1) * 4 bytes with splits =
+ * ceil(max_blocks_per_seq / 128) for fp16/bf16 queries (up to 16, of 16 blocks
+ * or more, for small launches whose partials stay within 8 MiB) and
  * ceil(max_blocks_per_seq / 64) for float32 (none when that is 1). Every
  * call on a device shares that device's scratch,
  * so the calls are serialised on the device: a call on another stream than

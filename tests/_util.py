@@ -6,7 +6,7 @@ import torch
 
 import oracle
 
-# north_star tolerances against the fp32 oracle
+# tolerances against the fp32 oracle
 TOL_16BIT = dict(max_abs=2e-2, mean_abs=2e-3)
 TOL_FP8 = dict(max_abs=5e-2, mean_abs=None)
 
