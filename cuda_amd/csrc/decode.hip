@@ -980,7 +980,7 @@ static PagedPlan paged_plan(int N, int Hq, int Hkv, int max_blocks, size_t ws_by
 // LDS (1024 of up to 13 pages: 15.4 us, four waves 19.4).
 static int mw_waves(long long grid, int pages) {
   const long long cus = device_cus();
-  if (pages <= 4) return 1;
+  if (pages <= 4 || 4 * 64 * grid > 0xffffffffLL) return 1;  // (a launch's threads are 32-bit)
   if (grid <= cus) return 8;
   if (pages <= 16) return grid <= 2 * cus ? 8 : 1;
   return 4;

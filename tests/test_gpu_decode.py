@@ -305,6 +305,22 @@ def test_flash_decode_waves_and_splits(dev, head_dim, b, hq, hkv, kv_len):
                  name=f"decode {kv_len}")
 
 
+def test_most_sequences(dev):
+    """2^21 sequences of 8 kv heads over shared pages: 2^24 splits, which only
+    workgroups of one wave fit into a launch's 2^32 - 1 threads."""
+    n, h, d = 2 ** 21, 8, 64
+    kc, vc = (torch.randn(1, h, d, 16, device=dev).bfloat16() for _ in range(2))
+    q = torch.randn(n, h, d, device=dev, dtype=torch.bfloat16)
+    tables = torch.zeros(n, 17, dtype=torch.int32, device=dev)
+    lens = torch.arange(n, dtype=torch.int32, device=dev) % 17
+    out = cuda_llm.paged_attention(q, kc, vc, tables, lens)
+    torch.cuda.synchronize()
+    assert torch.isfinite(out).all()
+    seqs = torch.arange(3, n, n // 61, device=dev)
+    case = dict(query=q[seqs], key_cache=kc, value_cache=vc, block_tables=tables[seqs], context_lens=lens[seqs])
+    assert_close(to_np(out[seqs]), paged_oracle(case), **TOL_16BIT, name="most sequences")
+
+
 def _growing(hkv, group, d, tokens, profile, dev):
     """Queries [Hkv, G, D] and keys [Hkv, tokens, D] whose logits grow along the
     tokens, each head of a group at its own: "ramp", by up to half a nat a token
