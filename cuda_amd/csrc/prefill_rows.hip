@@ -397,7 +397,11 @@ int prefill_rows_groups(int B, int Hq, int S, int D, float scale, bool causal) {
   const double four = estimate(4, 128, d64 ? 12 : 17, 28);
   const double two = estimate(2, d64 ? 256 : 128, d64 ? 10.5 : 13, 39, 1.45);
   if (std::min(four, two) > 0.9 * base) return 0;
-  return two < four ? 2 : 4;
+  const int groups = two < four ? 2 : 4;
+  // a workgroup per tile here, and a launch's threads are 32-bit (the 256-row
+  // kernels' launches of equal tiles are persistent)
+  const int rows = 32 * groups;
+  return bh * ((S + rows - 1) / rows) * (64 * kRowsWaves) > 4294967295.0 ? 0 : groups;
 }
 
 hipError_t launch_prefill_rows(int groups, bool f16, const void* q, const void* k, const void* v,

@@ -188,4 +188,5 @@ def prefill_rows_groups(b, hq, s, d, causal):
     two = estimate(2, 256 if d64 else 128, 10.5 if d64 else 13, 39, 1.45)
     if min(four, two) > 0.9 * base:
         return 0
-    return 2 if two < four else 4
+    groups = 2 if two < four else 4
+    return 0 if b * hq * -(-s // (32 * groups)) * 512 >= 2 ** 32 else groups

@@ -393,6 +393,24 @@ def test_shared_row_waves(dev, b, hq, hkv, s, dims, is_causal, d):
         assert np.abs(to_np(lse[bi:bi + 1, hi:hi + 1]) - lref).max() <= 1e-3
 
 
+def test_most_heads(dev):
+    """2^23 heads of 65 rows: a workgroup of 512 threads per tile would pass a
+    launch's 2^32 - 1 threads, the 256-row kernel's persistent launch does not."""
+    b, hq, s, d = 2 ** 18, 32, 65, 64
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 160e9:
+        pytest.skip("needs 160 GB of device memory")
+    k, v = (torch.randn(b, 1, s, d, device=dev, dtype=torch.bfloat16) for _ in range(2))
+    q = torch.randn(b, hq, s, d, device=dev, dtype=torch.bfloat16)
+    out = cuda_llm.flash_attention(q, k, v)
+    torch.cuda.synchronize()
+    for bi, hi in ((0, 0), (b // 2 + 1, 17), (b - 1, hq - 1)):
+        ref = oracle.attention(to_np(q[bi:bi + 1, hi:hi + 1]), to_np(k[bi:bi + 1]), to_np(v[bi:bi + 1]))
+        assert_close(to_np(out[bi:bi + 1, hi:hi + 1]), ref, **TOL_16BIT, name=f"head {bi},{hi}")
+    del q, k, v, out
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("is_causal", [False, True])
