@@ -348,7 +348,7 @@ __device__ __forceinline__ void dma_walk(const typename Tr::vec8 (&qv)[D / 32], 
     // their V slots are zeroed too, so stale cache bytes (NaN patterns
     // included) in a partially filled page cannot reach the PV product
     const int tok_end = min(Lctx, 16 * p_end);
-    const bool partial = (page0 + kStepPages) * 16 > tok_end;
+    const bool partial = page0 + kStepPages > tok_end / 16;  // (in pages: token 2^31 is no int)
     float x[8], vs[kStepPages];
     bool slot_ok[8];
 #pragma unroll
