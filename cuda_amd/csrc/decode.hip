@@ -1161,10 +1161,10 @@ __global__ __launch_bounds__(64) void decode_f32_kernel(
   const int hq0 = hk * Gq + hc * G;
   const int Gc = min(G, Gq - hc * G);
   const int L = PAGED ? min(max(0, context_lens[n]), max_blocks * kDecodePage) : S_contig;
-  const int n_splits = max(1, (L + kSplitTokens - 1) / kSplitTokens);
+  // (no sum past L: contexts go up to 2^31 - 16 tokens)
+  const int n_splits = max(1, L / kSplitTokens + (L % kSplitTokens != 0));
   if (split >= n_splits) return;
-  const int t_begin = split * kSplitTokens;
-  const int t_end = min(t_begin + kSplitTokens, L);
+  const int t_begin = split * kSplitTokens, n_tok = min(kSplitTokens, L - t_begin), t_end = t_begin + n_tok;
 
   for (int i = lane; i < G * D; i += 64) {
     const int g = i / D, d = i % D;
@@ -1195,10 +1195,10 @@ __global__ __launch_bounds__(64) void decode_f32_kernel(
     return per_block ? v_scale[(size_t)blk * Hkv + hk] : v_scale[hk];
   };
 
-  for (int t0 = t_begin; t0 < t_end; t0 += 64) {  // t0 is a multiple of 64: 4 whole pages
-    const int t = t0 + lane;
-    const bool valid = t < t_end;
-    const int tc = valid ? t : t_end - 1;
+  for (int i0 = 0; i0 < n_tok; i0 += 64) {  // t0 is a multiple of 64: 4 whole pages
+    const int t0 = t_begin + i0;
+    const bool valid = lane < n_tok - i0;
+    const int tc = valid ? t0 + lane : t_end - 1;
     float s[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) s[g] = 0.f;
@@ -1250,7 +1250,7 @@ __global__ __launch_bounds__(64) void decode_f32_kernel(
       ps[g][lane] = p;
     }
     __syncthreads();
-    const int nv = min(64, t_end - t0);
+    const int nv = min(64, n_tok - i0);
     if (PAGED) {
       for (int pg = 0; pg < 4 && 16 * pg < nv; ++pg) {
         const int blk = block_of(t0 / kDecodePage + pg);

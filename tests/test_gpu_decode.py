@@ -305,18 +305,20 @@ def test_flash_decode_waves_and_splits(dev, head_dim, b, hq, hkv, kv_len):
                  name=f"decode {kv_len}")
 
 
-def test_longest_context(dev):
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_longest_context(dev, dtype):
     """The longest context a table can name, 2^27 - 1 pages (all the same one):
-    the last step's second page, past the context, ends at token 2^31. Its
-    stand-in bytes are the query's, whose logit is 128 above the real ones."""
+    the 16-bit walk's last step has a second page, past the context, that ends
+    at token 2^31; its stand-in bytes are the query's, whose logit is 128 above
+    the real ones. float32: 2^21 splits, the last one's end past 2^31."""
     width = 2 ** 27 - 1
-    q = torch.ones(1, 1, 64, device=dev, dtype=torch.bfloat16)
-    kc, vc = (torch.full((1, 1, 64, 16), x, device=dev, dtype=torch.bfloat16) for x in (-1.0, 0.5))
+    q = torch.ones(1, 1, 64, device=dev, dtype=dtype)
+    kc, vc = (torch.full((1, 1, 64, 16), x, device=dev, dtype=dtype) for x in (-1.0, 0.5))
     tables = torch.zeros(1, width, dtype=torch.int32, device=dev)
     lens = torch.tensor([16 * width], dtype=torch.int32, device=dev)
     out = cuda_llm.paged_attention(q, kc, vc, tables, lens, softmax_scale=1.0)
     torch.cuda.synchronize()
-    assert torch.equal(out, torch.full_like(out, 0.5))
+    assert (out.double() - 0.5).abs().max().item() <= (1e-5 if dtype == torch.float32 else 0)
 
 
 def test_most_sequences(dev):
